@@ -137,7 +137,7 @@ inline bool skinny_before_gemv(int M, int N, int K) {
 }
 
 // MFMA path for few rows of A against a large N-contiguous B (skinny_gemm.hip):
-// FP16 (any alpha/beta, batched) and INT8 with zero points 0.  Same contract
+// FP16 (any alpha/beta, batched) and INT8 (any zero points).  Same contract
 // as the try_i4w_* functions.
 bool try_skinny_fp16(const uint16_t* A, const uint16_t* B, uint16_t* C, int batch, int M, int N, int K,
                      float alpha, float beta, int num_cus, hipStream_t stream, clove_status_t* status);

@@ -38,7 +38,7 @@ using I8M32 = Cfg<true, 32, 128, 1, 4, 5>;
 using I8M128 = Cfg<true, 128, 64, 4, 1, 4>;
 using I8T128 = Cfg<true, 128, 128, 2, 2, 3>;
 
-template <class CF, int OUT>
+template <class CF, int OUT, bool ZP = false>
 clove_status_t run(Args a, int batch, int cus, hipStream_t stream) {
     a.tiles_m = cdiv(a.M, CF::BM);
     a.tiles_n = cdiv(a.N, CF::BN);
@@ -63,7 +63,7 @@ clove_status_t run(Args a, int batch, int cus, hipStream_t stream) {
         a.part = s.partials;
         a.counters = s.counters;
     }
-    auto k = skinny_gemm<CF, OUT>;
+    auto k = skinny_gemm<CF, OUT, ZP>;
     if (ensure_lds(reinterpret_cast<const void*>(k), CF::LDS) != CLOVE_OK)
         return CLOVE_ERR_LAUNCH;
     CLOVE_LAUNCH(k, dim3((unsigned)(tiles * a.nsplit)), dim3(CF::NT), CF::LDS, stream, a);
@@ -187,7 +187,7 @@ bool try_skinny_int8(const Int8Args& q, int cus, hipStream_t stream, clove_statu
     // and 4096 x 11008, M = 3 / 4: 13.9 / 17.1 us here against 21.7 / 20.5 us
     // on the GEMV; at 4096 x 4096 the GEMV is ahead, 9.2 against 11.5 us)
     if (q.M <= 4 && (int64_t)q.N * q.K <= ((int64_t)32 << 20)) return false;
-    if (q.za != 0 || q.zb != 0 || !aligned16(q.A) || !aligned16(q.B) || !aligned16(q.C)) return false;
+    if (!aligned16(q.A) || !aligned16(q.B) || !aligned16(q.C)) return false;
     if (!fits31((int64_t)(q.M + 128) * q.K) || !fits31((int64_t)q.K * q.N) || !fits31((int64_t)q.M * q.N * 4))
         return false;
     Args a{};
@@ -197,11 +197,19 @@ bool try_skinny_int8(const Int8Args& q, int cus, hipStream_t stream, clove_statu
     a.sa = q.sa;
     a.sb = q.sb;
     a.scale = q.scale;
+    a.za = q.za;
+    a.zb = q.zb;
+    a.acc_add = q.acc_add;
     a.M = q.M;
     a.N = q.N;
     a.K = q.K;
+    const bool zp = q.za != 0 || q.zb != 0;
     auto pick = [&](auto out_tag) -> clove_status_t {
         constexpr int OUT = decltype(out_tag)::value;
+        auto go = [&](auto cfg) {
+            using CF = decltype(cfg);
+            return zp ? run<CF, OUT, true>(a, 1, cus, stream) : run<CF, OUT>(a, 1, cus, stream);
+        };
         // 32-row tiles up to M = 64, and up to 128 unless the weight is large
         // (cold: 4096 x 4096 at M = 64 / 128 10.8 / 13.8 us against 15.0 / 15.3
         // with 64- and 128-row tiles, 8192 x 2048 at M = 128 12.0 against 14.7;
@@ -213,11 +221,11 @@ bool try_skinny_int8(const Int8Args& q, int cus, hipStream_t stream, clove_statu
         const bool short_k = q.K <= 16 * I8M128::BK &&
                              (int64_t)cdiv(q.M, I8M128::BM) * cdiv(q.N, I8M128::BN) < cus / 2;
         const bool large_w = (int64_t)q.N * q.K > ((int64_t)32 << 20);
-        if (q.M <= 64 || (q.M <= 128 && !large_w) || short_k) return run<I8M32, OUT>(a, 1, cus, stream);
+        if (q.M <= 64 || (q.M <= 128 && !large_w) || short_k) return go(I8M32{});
         // 128x128 tiles for M <= 128 on wide weights, as for FP16 (cold, 128 x
         // 11008 x 4096 23.7 -> 20.5 us; 128 x 4096 x 11008 stays on 128x64)
-        if (q.M <= 128 && q.N >= 10240 && q.K >= 4096) return run<I8T128, OUT>(a, 1, cus, stream);
-        return run<I8M128, OUT>(a, 1, cus, stream);
+        if (q.M <= 128 && q.N >= 10240 && q.K >= 4096) return go(I8T128{});
+        return go(I8M128{});
     };
     switch (q.out) {
         case Int8Out::kHalfPerTensor: *status = pick(std::integral_constant<int, kI8Tensor>{}); break;

@@ -155,14 +155,41 @@ def test_skinny_bit_exact(M, N, K):
     assert np.array_equal(f16bits(to_host(C2)), f16bits(Cref2))
 
 
+# zero points inside the skinny kernel (row and column sums from the MFMA
+# operands): each tile shape, one and several K splits, either zero point 0,
+# sums far from 0 (constant operands), both extremes
+@pytest.mark.parametrize("M,N,K,za,zb", [
+    (5, 272, 384, 3, -5), (33, 512, 4096, -9, 0), (64, 1024, 4096, 0, 7), (100, 48, 128, -128, 127),
+    (130, 4096, 1024, 17, 0), (300, 512, 4096, -3, 5), (128, 10240, 4096, 127, -128), (512, 4096, 2048, -9, 0),
+])
+def test_skinny_zero_points_bit_exact(M, N, K, za, zb):
+    g = rng("skinny8zp", M, N, K, za, zb)
+    A = g.integers(-128, 128, (M, K)).astype(np.int8)
+    B = g.integers(-128, 128, (K, N)).astype(np.int8)
+    A[M // 2] = -128
+    B[:, N // 2] = 127
+    sa = g.uniform(0.001, 0.02, M).astype(np.float16)
+    sb = g.uniform(0.001, 0.02, N).astype(np.float16)
+    s1, s2 = np.float32(g.uniform(0.001, 0.05)), np.float32(g.uniform(0.001, 0.05))
+    C1, C2 = empty_f16(M, N), empty_f16(M, N)
+    _cg().gemm_int8(to_dev(A), to_dev(B), C1, M, N, K, float(s1), za, float(s2), zb)
+    _cg().gemm_int8_rowcol(to_dev(A), to_dev(B), to_dev(sa), to_dev(sb), C2, M, N, K, za, zb)
+    _sync()
+    rows = np.unique(np.concatenate([[0, M // 2, M - 1], g.integers(0, M, 12)]))
+    Cref1, accref = oracle.gemm_int8(A[rows], B, s1, za, s2, zb)
+    Cref2, _ = oracle.gemm_int8_rowcol(A[rows], B, sa[rows], sb, za, zb)
+    assert np.array_equal(run_acc32(A, B, za, zb)[rows], accref)
+    assert np.array_equal(f16bits(to_host(C1)[rows]), f16bits(Cref1))
+    assert np.array_equal(f16bits(to_host(C2)[rows]), f16bits(Cref2))
+
+
 # M = 2..4 on the GEMV with several K splits, non-zero zero points: per-tensor,
 # row/column scales and the raw accumulators, each bit for bit
 @pytest.mark.parametrize("M,N,K,za,zb", [(2, 4096, 4096, 3, -5), (3, 512, 2048, -7, 11), (4, 512, 2048, 9, -2),
                                          (4, 4096, 4096, 0, 0), (3, 11008, 4096, 0, 0), (4, 4096, 11008, 0, 0),
                                          (4, 11008, 4096, 3, -5)])
 def test_gemv_multirow_split_k(M, N, K, za, zb):
-    # (3 and 4 rows on 11008-wide weights take the skinny kernel when the zero
-    # points are 0, the GEMV otherwise)
+    # (3 and 4 rows on 11008-wide weights take the skinny kernel)
     g = rng("gemv8-mm", M, N, K, za, zb)
     A = g.integers(-128, 128, (M, K)).astype(np.int8)
     B = g.integers(-128, 128, (K, N)).astype(np.int8)
