@@ -6,10 +6,11 @@
 //  * dma::gemm_f16_big (f16_dma_gemm.hpp) -- large aligned shapes: 256x256x64
 //    tiles of v_mfma_f32_16x16x32_f16, A and B staged by LDS DMA, B fragments
 //    from transposing LDS reads, one tile per CU.
+//  * sk::skinny_gemm (skinny_gemm.hpp) -- the rest, any alignment and any K.
 //  * mg::mfma_gemm with the fp16 row loader for A and the transposing fp16
 //    column loader for B (mfma_gemm.hpp): LDS-tiled v_mfma_f32_32x32x16_f16,
 //    tile shape chosen per (M, N), split-K when the tile grid is too small to
-//    fill the CUs; every other shape.
+//    fill the CUs; operands past 2^31 bytes, N < 8, K = 0.
 //  * gemv_f16 -- M <= 4 decode shapes: B streamed once from HBM with 16 B
 //    loads (a 256 x 256 tile per workgroup, all in flight), fp32 FMAs on the
 //    VALU, split-K over workgroups.
@@ -97,6 +98,11 @@ __global__ void __launch_bounds__(1024) gemv_f16(GemvParams p) {
         bv[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(B + (int64_t)k * N + nc));
     }
     __builtin_amdgcn_sched_barrier(0);  // every B row requested before the first FMA
+    if (kbeg + GV_ROWS > K) {  // rows past K (the last split's): zero, not the clamped row's NaN or infinity
+#pragma unroll
+        for (int j = 0; j < GV_RPT; ++j)
+            if (kbeg + kl + GV_KL * j >= K) bv[j] = u32x4{0u, 0u, 0u, 0u};
+    }
 
     float acc[MM][8];
 #pragma unroll
@@ -357,7 +363,8 @@ clove_status_t launch_gemm_fp16(const uint16_t* A, const uint16_t* B, uint16_t* 
         clove_status_t st2;
         if (try_skinny_fp16(A, B, C, batch, M, N, K, alpha, beta, dev.num_cus, stream, &st2)) return st2;
     }
-    if (aligned && M <= 4 && K > 0) {
+    // (the GEMV reads A element by element: any K and any alignment of A and C)
+    if (aligned16(B) && N % 8 == 0 && M <= 4 && K > 0) {
         GemvParams g{A, B, C, nullptr, M, N, K, alpha, beta, sA, sB, sC, 0, 1, nullptr, nullptr};
         if (M == 1) return run_gemv<1>(g, batch, stream);
         if (M == 2) return run_gemv<2>(g, batch, stream);

@@ -6,7 +6,10 @@
 // Replaces the reference's gemm_int8 (src/kernels/gemm_int8.cu:16-137; the
 // per-element formula is :37-40, :87-96, :113-114).
 //
-//  * int8_mfma -- v_mfma_i32_32x32x32_i8 on the raw operands.  Zero points are
+//  * sk::skinny_gemm (skinny_gemm.hpp) and i8big::gemm_i8_big
+//    (i8_dma_gemm.hpp) -- nearly every product with more than four rows.
+//  * int8_mfma -- large M on few columns, operands past 2^31 bytes, N < 16,
+//    K = 0: v_mfma_i32_32x32x32_i8 on the raw operands.  Zero points are
 //    applied exactly in the epilogue with the identity
 //        sum (a-za)(b-zb) = sum ab - zb*rowsum(A) - za*colsum(B) + K*za*zb
 //    (int32 wrap-around arithmetic, exact whenever the true value fits int32),
@@ -612,7 +615,7 @@ clove_status_t run_i8big(const I8Params& q, hipStream_t stream) {
 
 template <int OUT>
 clove_status_t dispatch(I8Params p, bool aligned, int cus, hipStream_t stream) {
-    if (aligned && p.M <= 4 && p.K > 0 && p.N >= 16) return run_gemv<OUT>(p, stream);
+    if (aligned && p.M <= 4 && p.K > 0) return run_gemv<OUT>(p, stream);
     if (!aligned) return run_mfma<64, 64, 64, 2, 2, OUT, false>(p, cus, stream);
     if (p.M <= 64) return run_mfma<64, 128, 128, 2, 2, OUT, true>(p, cus, stream);
     if ((int64_t)cdiv(p.M, 256) * cdiv(p.N, 256) >= cus / 2)
@@ -644,7 +647,21 @@ clove_status_t launch_gemm_int8(const Int8Args& a, hipStream_t stream) {
             case Int8Out::kAcc32: return run_i8big<(int)Int8Out::kAcc32>(p, stream);
         }
     }
-    if (a.M > 2) {  // (three or four rows only for large weights; try_skinny_int8 decides)
+    // The GEMV takes up to four rows (A at any alignment); three or four rows on
+    // a large weight go to the skinny kernel (cold 11008 x 4096 and 4096 x
+    // 11008, M = 3 / 4: 13.9 / 17.1 us there against 21.7 / 20.5 us on the
+    // GEMV; at 4096 x 4096 the GEMV is ahead, 9.2 against 11.5 us)
+    const bool gemv = a.M <= 4 && a.K > 0 && a.N >= 16 && a.N % 16 == 0 && aligned16(a.B);
+    if (gemv && (a.M <= 2 || (int64_t)a.N * a.K <= ((int64_t)32 << 20))) {
+        switch (a.out) {
+            case Int8Out::kHalfPerTensor: return run_gemv<(int)Int8Out::kHalfPerTensor>(p, stream);
+            case Int8Out::kHalfRowCol: return run_gemv<(int)Int8Out::kHalfRowCol>(p, stream);
+            case Int8Out::kAcc32: return run_gemv<(int)Int8Out::kAcc32>(p, stream);
+        }
+    }
+    // the skinny kernel for the rest, except (M > 2048, zero points 0, whole K
+    // tiles) where the register-staged 256x256 tiles are ahead
+    if (a.M <= 2048 || a.za != 0 || a.zb != 0 || !aligned || a.K % 128 != 0) {
         clove_status_t st2;
         if (try_skinny_int8(a, dev.num_cus, stream, &st2)) return st2;
     }

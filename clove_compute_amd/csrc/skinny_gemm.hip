@@ -38,13 +38,13 @@ using I8M32 = Cfg<true, 32, 128, 1, 4, 5>;
 using I8M128 = Cfg<true, 128, 64, 4, 1, 4>;
 using I8T128 = Cfg<true, 128, 128, 2, 2, 3>;
 
-template <class CF, int OUT, bool ZP = false>
+template <class CF, int OUT, bool ZP = false, Feed FEED = kWhole>
 clove_status_t run(Args a, int batch, int cus, hipStream_t stream) {
     a.tiles_m = cdiv(a.M, CF::BM);
     a.tiles_n = cdiv(a.N, CF::BN);
     a.batch = batch;
     const int tiles = a.tiles_m * a.tiles_n * batch;
-    const int nk = a.K / CF::BK;
+    const int nk = cdiv(a.K, CF::BK);
     // split K (whole K tiles, at least two per split) until about one
     // workgroup per CU; not for short K (<= 16 K tiles), where the split's
     // publish / count / reload tail costs more than the shorter stream saves
@@ -63,10 +63,11 @@ clove_status_t run(Args a, int batch, int cus, hipStream_t stream) {
         a.part = s.partials;
         a.counters = s.counters;
     }
-    auto k = skinny_gemm<CF, OUT, ZP>;
-    if (ensure_lds(reinterpret_cast<const void*>(k), CF::LDS) != CLOVE_OK)
+    auto k = skinny_gemm<CF, OUT, ZP, FEED>;
+    constexpr int lds = FEED == kUnaligned ? CF::LDS_UA : CF::LDS;
+    if (ensure_lds(reinterpret_cast<const void*>(k), lds) != CLOVE_OK)
         return CLOVE_ERR_LAUNCH;
-    CLOVE_LAUNCH(k, dim3((unsigned)(tiles * a.nsplit)), dim3(CF::NT), CF::LDS, stream, a);
+    CLOVE_LAUNCH(k, dim3((unsigned)(tiles * a.nsplit)), dim3(CF::NT), lds, stream, a);
     return check_launch();
 }
 
@@ -111,11 +112,19 @@ F16Tile pick_f16_tile(int batch, int M, int N, int K, int cus) {
 }
 
 bool f16_domain(const void* A, const void* B, const void* C, int M, int N, int K) {
-    if (M <= 1 || K <= 0 || K % 64 != 0 || N < 8 || N % 8 != 0) return false;
+    if (M <= 1 || K <= 0 || K % 8 != 0 || N < 8 || N % 8 != 0) return false;
     if (M <= 4 && !skinny_before_gemv(M, N, K)) return false;
     if (!aligned16(A) || !aligned16(B) || !aligned16(C)) return false;
     // (the DMA offsets of the padded rows m < M + 128 must stay 32-bit)
-    return fits31((int64_t)(M + 128) * K * 2) && fits31((int64_t)K * N * 2) && fits31((int64_t)M * N * 2);
+    return fits31((int64_t)(M + 128) * K * 2) && fits31((int64_t)(K + 64) * N * 2) && fits31((int64_t)M * N * 2);
+}
+
+// The unaligned variant (UA): any strides and element-aligned pointers.  Both
+// operands hold at least one 16-byte chunk, and a row of B does (a chunk of
+// any K tile but the last then stays inside B).
+bool ua_domain(int M, int N, int K, int es) {
+    return M >= 1 && K >= 1 && N * es >= 16 && (int64_t)M * K * es >= 16 && fits31((int64_t)(M + 128) * K * es) &&
+           fits31((int64_t)(K + 128) * N * es);
 }
 
 // two-B-operand (gate, up) counterparts of the tiles above; fewer stages
@@ -130,7 +139,8 @@ using SwK32 = Cfg<false, 32, 32, 1, 1, 3, 2, 4>;
 
 bool try_skinny_fp16(const uint16_t* A, const uint16_t* B, uint16_t* C, int batch, int M, int N, int K,
                      float alpha, float beta, int cus, hipStream_t stream, clove_status_t* status) {
-    if (!f16_domain(A, B, C, M, N, K)) return false;
+    const bool al = f16_domain(A, B, C, M, N, K);
+    if (!al && !ua_domain(M, N, K, 2)) return false;
     Args a{};
     a.A = A;
     a.B = B;
@@ -143,22 +153,27 @@ bool try_skinny_fp16(const uint16_t* A, const uint16_t* B, uint16_t* C, int batc
     a.sA = (int64_t)M * K;
     a.sB = (int64_t)K * N;
     a.sC = (int64_t)M * N;
+    auto go = [&](auto cfg) {
+        using CF = decltype(cfg);
+        if (!al) return run<CF, kF16AlphaBeta, false, kUnaligned>(a, batch, cus, stream);
+        return K % CF::BK == 0 ? run<CF, kF16AlphaBeta>(a, batch, cus, stream)
+                               : run<CF, kF16AlphaBeta, false, kRagged>(a, batch, cus, stream);
+    };
     switch (pick_f16_tile(batch, M, N, K, cus)) {
-        case F16Tile::kM32: *status = run<F16M32, kF16AlphaBeta>(a, batch, cus, stream); break;
-        case F16Tile::kM128: *status = run<F16M128, kF16AlphaBeta>(a, batch, cus, stream); break;
-        case F16Tile::kT128: *status = run<F16T128, kF16AlphaBeta>(a, batch, cus, stream); break;
+        case F16Tile::kM32: *status = go(F16M32{}); break;
+        case F16Tile::kM128: *status = go(F16M128{}); break;
+        case F16Tile::kT128: *status = go(F16T128{}); break;
         case F16Tile::kT64:
-            *status = K <= 512 ? run<F16T64S2, kF16AlphaBeta>(a, batch, cus, stream)
-                               : run<F16T64, kF16AlphaBeta>(a, batch, cus, stream);
+            *status = K <= 512 ? go(F16T64S2{}) : go(F16T64{});
             break;
-        case F16Tile::kK32: *status = run<F16K32, kF16AlphaBeta>(a, batch, cus, stream); break;
+        case F16Tile::kK32: *status = go(F16K32{}); break;
     }
     return true;
 }
 
 bool try_skinny_swiglu(const uint16_t* X, const uint16_t* W_gate, const uint16_t* W_up, uint16_t* out, int T,
                        int hidden, int inter, int cus, hipStream_t stream, clove_status_t* status) {
-    if (!f16_domain(X, W_gate, out, T, inter, hidden) || !aligned16(W_up)) return false;
+    if (!f16_domain(X, W_gate, out, T, inter, hidden) || !aligned16(W_up) || hidden % 64 != 0) return false;
     Args a{};
     a.A = X;
     a.B = W_gate;
@@ -182,14 +197,10 @@ bool try_skinny_swiglu(const uint16_t* X, const uint16_t* W_gate, const uint16_t
 }
 
 bool try_skinny_int8(const Int8Args& q, int cus, hipStream_t stream, clove_status_t* status) {
-    if (q.M <= 2 || q.M > 2048 || q.K <= 0 || q.K % 128 != 0 || q.N < 16 || q.N % 16 != 0) return false;
-    // three or four rows: the GEMV unless the weight is large (cold 11008 x 4096
-    // and 4096 x 11008, M = 3 / 4: 13.9 / 17.1 us here against 21.7 / 20.5 us
-    // on the GEMV; at 4096 x 4096 the GEMV is ahead, 9.2 against 11.5 us)
-    if (q.M <= 4 && (int64_t)q.N * q.K <= ((int64_t)32 << 20)) return false;
-    if (!aligned16(q.A) || !aligned16(q.B) || !aligned16(q.C)) return false;
-    if (!fits31((int64_t)(q.M + 128) * q.K) || !fits31((int64_t)q.K * q.N) || !fits31((int64_t)q.M * q.N * 4))
-        return false;
+    const bool al = q.K > 0 && q.K % 16 == 0 && q.N >= 16 && q.N % 16 == 0 && aligned16(q.A) && aligned16(q.B) &&
+                    aligned16(q.C) && fits31((int64_t)(q.M + 128) * q.K) && fits31((int64_t)(q.K + 128) * q.N) &&
+                    fits31((int64_t)q.M * q.N * 4);
+    if (!al && !ua_domain(q.M, q.N, q.K, 1)) return false;
     Args a{};
     a.A = q.A;
     a.B = q.B;
@@ -208,6 +219,8 @@ bool try_skinny_int8(const Int8Args& q, int cus, hipStream_t stream, clove_statu
         constexpr int OUT = decltype(out_tag)::value;
         auto go = [&](auto cfg) {
             using CF = decltype(cfg);
+            // (the unaligned variant always carries the zero points)
+            if (!al) return run<CF, OUT, true, kUnaligned>(a, 1, cus, stream);
             return zp ? run<CF, OUT, true>(a, 1, cus, stream) : run<CF, OUT>(a, 1, cus, stream);
         };
         // 32-row tiles up to M = 64, and up to 128 unless the weight is large

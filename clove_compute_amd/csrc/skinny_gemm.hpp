@@ -43,6 +43,24 @@
 // thread per column, and the register-staged kernel behind it, 512 x 4096 x
 // 4096 with an activation zero point took 1041 us; here it takes 22.6).
 //
+// Ragged K (K not a multiple of the K tile): the k-rows of B past K lie past
+// the end of the operand and read as zero; A's chunks past K would read the
+// next row, so for FP16 (whose stray bits could be NaN or infinity) their
+// lanes take an offset past the end instead.
+//
+// Unaligned operands (UA): row strides or pointers that are not multiples of
+// 16 bytes, which an LDS DMA cannot take.  The same chunks go global -> VGPR
+// by 16-byte loads at element alignment (ordinary loads, which gfx950 takes at
+// any byte address) -> the same LDS layout, P K tiles ahead in registers
+// and two LDS stages.  A chunk of the last K tile is loaded from at most 16 bytes
+// before the operand's end and shifted into place, and what lies past K is
+// zeroed, so no access leaves an operand; chunks past M or N load row or
+// column 0.  Stores and the loads of C take any alignment too.  Bound as the
+// aligned form by operand bytes per CU, plus the LDS writes; measured against
+// the generic kernel, whose loader gathers element by element (us per call):
+// FP16 333 x 5001 x 2050 142 -> 31.5, 496 x 3512 x 3275 264 -> 38; INT8 with a
+// zero point 1184 x 3392 x 6900 3538 -> 95, 1 x 1408 x 7922 1932 -> 9.
+//
 // Two B operands (NB = 2, FP16 only): B and B2 share A and the tile's
 // columns; each stage holds A, then the B tile, then the B2 tile, and every
 // wave keeps both accumulator sets.  The SwiGLU epilogue (kF16SwiGLU) then
@@ -111,7 +129,31 @@ struct Cfg {
     static constexpr int RED = KW > 1 ? NW * NB * FN * FM * 4096 : 0;
     static constexpr int LDS = S * SB + RED;
     static_assert(LDS <= 160 * 1024, "LDS");
+    // UA: K tiles held in registers (16 D bytes per thread each), two LDS stages
+    static constexpr int P = D <= 2 ? 6 : D <= 5 ? 4 : D <= 6 ? 3 : 2;
+    static constexpr int LDS_UA = 2 * SB + RED;
 };
+
+// 16 bytes at any byte address, and their shift towards byte 0 by s bytes
+// (zero fill); the first v of 16 bytes kept, the rest zeroed
+typedef unsigned u32x4u __attribute__((ext_vector_type(4), aligned(1)));
+typedef unsigned u32x2u __attribute__((ext_vector_type(2), aligned(1)));
+__device__ __forceinline__ u32x4 load_any16(const unsigned char* p) { return *reinterpret_cast<const u32x4u*>(p); }
+__device__ __forceinline__ u32x4 shift_bytes(u32x4 x, unsigned s) {
+    if (s & 4) x = u32x4{x.y, x.z, x.w, 0u};
+    if (s & 8) x = u32x4{x.z, x.w, 0u, 0u};
+    x = u32x4{__builtin_amdgcn_alignbyte(x.y, x.x, s & 3), __builtin_amdgcn_alignbyte(x.z, x.y, s & 3),
+              __builtin_amdgcn_alignbyte(x.w, x.z, s & 3), x.w >> (8 * (s & 3))};
+    return s >= 16 ? u32x4{0u, 0u, 0u, 0u} : x;
+}
+__device__ __forceinline__ u32x4 keep_bytes(u32x4 x, int v) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const int b = v - 4 * d;  // bytes of this word kept
+        x[d] = b >= 4 ? x[d] : b <= 0 ? 0u : x[d] & ((1u << (8 * b)) - 1u);
+    }
+    return x;
+}
 
 // chunk swizzle of B k-row r (see the header comment): the rows one
 // transposing read touches (4 rows x 2 chunks for fp16, 8 rows x 1 chunk for
@@ -158,9 +200,18 @@ __device__ __forceinline__ void stage_wait(int ahead) {
     }
 }
 
-template <class CF, int OUT, bool ZP = false>
+// how the operands reach LDS (see the header comment): by DMA with K a multiple
+// of the K tile (any aligned K for INT8), by DMA with ragged K, through VGPRs.
+// A kernel of its own for whole K tiles: with the ragged tail's branch beside
+// every stage's DMAs, 128 x 4096 x 11008 took 32.7 instead of 32.1 us.
+enum Feed { kWhole = 0, kRagged = 1, kUnaligned = 2 };
+
+template <class CF, int OUT, bool ZP = false, Feed FEED = kWhole>
 __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
     static_assert(!ZP || CF::I8, "zero points: INT8 only");
+    constexpr bool UA = FEED == kUnaligned;
+    static_assert(FEED == kWhole || CF::NB == 1, "ragged or unaligned: one B operand");
+    static_assert(FEED != kRagged || !CF::I8, "INT8 needs no ragged form: stray k of A meet zeros of B");
     constexpr int ES = CF::ES, NW = CF::NW, FM = CF::FM, FN = CF::FN, S = CF::S;
     constexpr int BM = CF::BM, BN = CF::BN, BK = CF::BK, BNB = CF::BNB, SB = CF::SB;
     constexpr int D = CF::D;
@@ -199,7 +250,7 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
     const int m0 = tm * BM, n0 = tn * BN;
     const int M = p.M, N = p.N, K = p.K;
     const int kbeg = split * p.kps;
-    const int nkt = (min(K, kbeg + p.kps) - kbeg) / BK;
+    const int nkt = (min(K, kbeg + p.kps) - kbeg + BK - 1) / BK;
 
     const unsigned lds0 = __builtin_amdgcn_readfirstlane(
         (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)smem));
@@ -228,8 +279,16 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
     auto issue = [&](int t, int stage) {
         const int k0 = kbeg + t * BK;
         const unsigned st = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(stage * SB));
+        if (FEED == kRagged && k0 + BK > K) {
+            // ragged K: a lane whose chunk starts at or past K reads past the end, zero
+            const bool past = k0 + 8 * ((lane & 7) ^ (lane >> 3)) >= K;
 #pragma unroll
-        for (int i = 0; i < CF::DA; ++i) dma16(ra, st + (wave * CF::DA + i) * 1024, offa[i], k0 * ES);
+            for (int i = 0; i < CF::DA; ++i)
+                dma16(ra, st + (wave * CF::DA + i) * 1024, past ? 0x7ffffff0 : offa[i], k0 * ES);
+        } else {
+#pragma unroll
+            for (int i = 0; i < CF::DA; ++i) dma16(ra, st + (wave * CF::DA + i) * 1024, offa[i], k0 * ES);
+        }
 #pragma unroll
         for (int i = 0; i < CF::DB; ++i)
             dma16(rb, st + CF::A_BYTES + (wave * CF::DB + i) * 1024, offb[i], k0 * N * ES);
@@ -299,18 +358,8 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
         return s;
     };
 
-#pragma unroll
-    for (int t = 0; t < S - 1; ++t)
-        if (t < nkt) issue(t, t);
-
-    int stage = 0, stage_next = S - 1;
-    for (int t = 0; t < nkt; ++t) {
-        stage_wait<S, D>(min(S - 2, nkt - 1 - t));
-        if (t + S - 1 < nkt) issue(t + S - 1, stage_next);
-        const unsigned st = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(stage * SB));
-        stage_next = stage;
-        stage = stage + 1 == S ? 0 : stage + 1;
-
+    // one K tile (k0 its first k) from the stage at LDS address st
+    auto compute = [&](unsigned st, [[maybe_unused]] int k0) {
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
             u32x4 af[FM];
@@ -333,7 +382,11 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
                     }
                     if (p.zb != 0) {
 #pragma unroll
-                        for (int j = 0; j < FM; ++j) rsum[j] = ones_dot(af[j], rsum[j]);
+                        for (int j = 0; j < FM; ++j) {
+                            const int r = ones_dot(af[j], rsum[j]);
+                            // (aligned ragged K: chunks past K hold the next row)
+                            rsum[j] = UA || k0 + 16 * (2 * ks + kh) < K ? r : rsum[j];
+                        }
                     }
                 }
 #pragma unroll
@@ -349,6 +402,104 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
                     }
             }
         }
+    };
+
+    if constexpr (!UA) {
+#pragma unroll
+        for (int t = 0; t < S - 1; ++t)
+            if (t < nkt) issue(t, t);
+
+        int stage = 0, stage_next = S - 1;
+        for (int t = 0; t < nkt; ++t) {
+            stage_wait<S, D>(min(S - 2, nkt - 1 - t));
+            if (t + S - 1 < nkt) issue(t + S - 1, stage_next);
+            const unsigned st = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(stage * SB));
+            stage_next = stage;
+            stage = stage + 1 == S ? 0 : stage + 1;
+            compute(st, kbeg + t * BK);
+        }
+    } else {
+        constexpr int P = CF::P;
+        const unsigned a_end = (unsigned)M * K * ES, b_end = (unsigned)K * N * ES;  // bytes of A, of B
+        unsigned ua[CF::DA], ub[CF::DB];  // this lane's chunks of K tile 0
+#pragma unroll
+        for (int i = 0; i < CF::DA; ++i) {
+            const int row = m0 + 8 * (wave * CF::DA + i) + (lane >> 3);
+            ua[i] = (unsigned)(row < M ? row : 0) * K * ES + 16 * ((lane & 7) ^ (lane >> 3));
+        }
+#pragma unroll
+        for (int i = 0; i < CF::DB; ++i) {
+            const int row = RPI * (wave * CF::DB + i) + lane / CPR;
+            const int nb = n0 * ES + 16 * ((lane % CPR) ^ swz_b<BNB, I8>(row));
+            ub[i] = (unsigned)row * N * ES + (nb < N * ES ? nb : 0);
+        }
+        u32x4 rg[P][D];
+        // a K tile that is not the operands' last: every chunk lies inside (a B
+        // chunk that passes its row's end reads into the next row)
+        auto load_fast = [&](u32x4 (&r)[D], int t) {
+            const int k0 = kbeg + t * BK;
+            const unsigned char* at = Ab + (int64_t)k0 * ES;
+            const unsigned char* bt = Bb + (int64_t)k0 * N * ES;
+#pragma unroll
+            for (int i = 0; i < CF::DA; ++i) r[i] = load_any16(at + ua[i]);
+#pragma unroll
+            for (int i = 0; i < CF::DB; ++i) r[CF::DA + i] = load_any16(bt + ub[i]);
+        };
+        auto load_careful = [&](u32x4 (&r)[D], int t) {
+            const int k0 = kbeg + t * BK;
+#pragma unroll
+            for (int i = 0; i < CF::DA; ++i) {
+                const unsigned off = ua[i] + (unsigned)k0 * ES, at = min(off, a_end - 16);
+                r[i] = keep_bytes(shift_bytes(load_any16(Ab + at), off - at),
+                                  (K - k0) * ES - 16 * ((lane & 7) ^ (lane >> 3)));
+            }
+#pragma unroll
+            for (int i = 0; i < CF::DB; ++i) {
+                const unsigned off = ub[i] + (unsigned)k0 * N * ES, at = min(off, b_end - 16);
+                r[CF::DA + i] = shift_bytes(load_any16(Bb + at), off - at);  // (zero from the end on)
+            }
+        };
+        auto put = [&](const u32x4 (&r)[D], int t) {
+            const unsigned st = lds0 + (unsigned)((t & 1) * SB) + 16 * lane;
+#pragma unroll
+            for (int i = 0; i < CF::DA; ++i)
+                *reinterpret_cast<lds_u32x4*>((size_t)(st + (wave * CF::DA + i) * 1024)) = r[i];
+#pragma unroll
+            for (int i = 0; i < CF::DB; ++i)
+                *reinterpret_cast<lds_u32x4*>((size_t)(st + CF::A_BYTES + (wave * CF::DB + i) * 1024)) = r[CF::DA + i];
+        };
+        // One barrier per K tile: a wave that writes stage t % 2 again has passed
+        // barrier t + 1, and every wave reached that one with its reads of tile t
+        // complete.  The steady loop's loads are unconditional, so that the wait
+        // before a tile's LDS writes leaves the P - 1 later tiles in flight.
+        const int whole = kbeg + nkt * BK < K ? nkt : nkt - 1;  // K tiles for load_fast
+#pragma unroll
+        for (int u = 0; u < P; ++u)
+            if (u < nkt) load_careful(rg[u], u);
+        int t = 0;
+#pragma unroll 1
+        for (; t + 2 * P <= whole; t += P) {
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                put(rg[u], t + u);
+                load_fast(rg[u], t + u + P);
+                lds_barrier();
+                compute(lds0 + (unsigned)(((t + u) & 1) * SB), kbeg + (t + u) * BK);
+            }
+        }
+#pragma unroll 1
+        for (; t < nkt; t += P) {
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                if (t + u < nkt) {
+                    put(rg[u], t + u);
+                    if (t + u + P < nkt) load_careful(rg[u], t + u + P);
+                    lds_barrier();
+                    compute(lds0 + (unsigned)(((t + u) & 1) * SB), kbeg + (t + u) * BK);
+                }
+            }
+        }
+        if (CF::KW > 1 || p.nsplit > 1) __syncthreads();  // (LDS is used again below)
     }
 
     // ---- zero points: the split's correction (both lane halves added, column
@@ -377,7 +528,7 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
     // slice order ----
     constexpr int NQ = 4 / CF::KW;  // runs of 4 columns per block owned by a wave
     if constexpr (CF::KW > 1) {
-        const unsigned red = lds0 + (unsigned)(S * SB);
+        const unsigned red = lds0 + (unsigned)((UA ? 2 : S) * SB);
         // wave tile wmn, slice s, block (b, i, j), run q: 1 KB, 16 lane-contiguous
         // bytes per lane
         auto slot = [&](int s, int b, int i, int j, int q) {
@@ -471,9 +622,17 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         if (CF::KW > 1 && q / NQ != kw) continue;
-                        const int nc = min(n0 + wn * 32 * FN + 32 * i + 8 * q + 4 * kh, N - 4);
-                        oldc[j][i][q] =
-                            *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(Cb) + (int64_t)mc * N + nc);
+                        const int n = n0 + wn * 32 * FN + 32 * i + 8 * q + 4 * kh;
+                        const int nc = min(n, N - 4);
+                        const uint16_t* src = reinterpret_cast<const uint16_t*>(Cb) + (int64_t)mc * N + nc;
+                        if constexpr (UA) {
+                            // (a run cut by N: the row's last four, shifted into place)
+                            const u32x2 c = *reinterpret_cast<const u32x2u*>(src);
+                            const uint64_t w = ((uint64_t)c.y << 32 | c.x) >> (16 * min(n - nc, 3));
+                            oldc[j][i][q] = u32x2{(unsigned)w, (unsigned)(w >> 32)};
+                        } else {
+                            oldc[j][i][q] = *reinterpret_cast<const u32x2*>(src);
+                        }
                     }
             }
         }
@@ -483,9 +642,9 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
         for (int i = 0; i < FN; ++i)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int nc = min(n0 + wn * 32 * FN + 32 * i + 8 * q + 4 * kh, N - 4);
+                const int n = n0 + wn * 32 * FN + 32 * i + 8 * q + 4 * kh;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) sbv[i][q][e] = h2f(p.sb[nc + e]);
+                for (int e = 0; e < 4; ++e) sbv[i][q][e] = h2f(p.sb[min(n + e, N - 1)]);
             }
     }
 #pragma unroll
@@ -499,11 +658,17 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
             for (int q = 0; q < 4; ++q) {
                 if (CF::KW > 1 && q / NQ != kw) continue;
                 const int n = n0 + wn * 32 * FN + 32 * i + 8 * q + 4 * kh;
-                if (n >= N) continue;  // N % 8 == 0: the run is whole
+                if (n >= N) continue;  // aligned: N % 8 == 0, the run is whole
                 if constexpr (OUT == kI8Acc32) {
                     int* dst = reinterpret_cast<int*>(Cb) + (int64_t)m * N + n;
-                    *reinterpret_cast<i32x4*>(dst) =
-                        i32x4{acc[0][i][j][4 * q], acc[0][i][j][4 * q + 1], acc[0][i][j][4 * q + 2], acc[0][i][j][4 * q + 3]};
+                    if constexpr (UA) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (n + e < N) dst[e] = acc[0][i][j][4 * q + e];
+                    } else {
+                        *reinterpret_cast<i32x4*>(dst) = i32x4{acc[0][i][j][4 * q], acc[0][i][j][4 * q + 1],
+                                                               acc[0][i][j][4 * q + 2], acc[0][i][j][4 * q + 3]};
+                    }
                 } else {
                     uint16_t* dst = reinterpret_cast<uint16_t*>(Cb) + (int64_t)m * N + n;
                     float r[4];
@@ -533,7 +698,18 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
 #pragma unroll
                         for (int e = 0; e < 4; ++e) r[e] = static_cast<float>(acc[0][i][j][4 * q + e]) * (sa * sbv[i][q][e]);
                     }
-                    *reinterpret_cast<u32x2*>(dst) = u32x2{pack2h(r[0], r[1]), pack2h(r[2], r[3])};
+                    const u32x2 w = {pack2h(r[0], r[1]), pack2h(r[2], r[3])};
+                    if constexpr (UA) {
+                        if (n + 4 <= N) {
+                            *reinterpret_cast<u32x2u*>(dst) = w;
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 3; ++e)
+                                if (n + e < N) dst[e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+                        }
+                    } else {
+                        *reinterpret_cast<u32x2*>(dst) = w;
+                    }
                 }
             }
     }

@@ -341,3 +341,62 @@ def test_mid_size_tiles_small_integers_bit_exact(M, N, K):
     C = run_fp16(A, B)
     exact = A.astype(np.float64) @ B.astype(np.float64)
     assert np.array_equal(f16bits(C), f16bits(exact.astype(np.float16)))
+
+
+# Unaligned and ragged-K products on the skinny kernel (every tile shape, one
+# and several K splits, the steady loop's K tiles and the careful ones), and the
+# GEMV at odd K: small integers, so fp32 sums are exact in any order.  The
+# element after an operand's last row, and A's next rows past K, must not leak:
+# B is followed by NaNs, and one row of A holds infinities against zeros of B
+# nowhere (its own outputs are infinite or NaN, the others finite).
+@pytest.mark.parametrize("M,N,K,beta", [
+    (1, 17, 33, 0.0), (1, 4097, 2051, 0.0), (1, 4096, 2051, 1.0), (3, 5001, 4098, 1.0), (4, 2056, 77, 0.0), (5, 9, 8, 0.0),
+    (33, 33, 4099, 1.0), (64, 4001, 1024, 0.0), (100, 203, 320, 1.0), (129, 4095, 4100, 0.0), (300, 1001, 2050, 1.0),
+    (257, 515, 4101, 0.0), (600, 640, 100, 0.0), (40, 4096, 1032, 1.0), (500, 1024, 4104, 0.0),
+])
+def test_unaligned_and_ragged_k_bit_exact(M, N, K, beta):
+    import torch
+    g = rng("unaligned", M, N, K)
+    A = g.integers(-2, 3, (M, K)).astype(np.float16)
+    B = g.integers(-2, 3, (K, N)).astype(np.float16)
+    C0 = g.integers(-8, 9, (M, N)).astype(np.float16)
+    inf_row = M // 2 if M > 1 else -1
+    if inf_row >= 0:
+        A[inf_row, : min(K, 4)] = np.inf
+    ref = A.astype(np.float32) if inf_row < 0 else np.where(np.arange(M)[:, None] == inf_row, 0, A).astype(np.float32)
+    ref = ref @ B.astype(np.float32) + beta * C0.astype(np.float32)
+    # B inside a larger buffer, NaN behind its end
+    dB = torch.full((K * N + 64,), float("nan"), dtype=torch.float16, device="cuda")
+    dB[: K * N] = to_dev(B).reshape(-1)
+    dA = torch.full((M * K + 64,), float("nan"), dtype=torch.float16, device="cuda")
+    dA[: M * K] = to_dev(A).reshape(-1)
+    dC = to_dev(C0)
+    import clove_compute_amd as cg
+    cg.gemm_fp16(dA, dB, dC, M, N, K, 1.0, beta)
+    torch.cuda.synchronize()
+    keep = np.arange(M) != inf_row
+    assert np.array_equal(f16bits(to_host(dC)[keep] + np.float16(0)), f16bits(ref[keep].astype(np.float16) + np.float16(0)))
+    if inf_row >= 0:
+        assert not np.isfinite(to_host(dC)[inf_row]).all()
+
+
+# odd element offsets of all three operands, and odd batch strides
+@pytest.mark.parametrize("batch,M,N,K,off", [(1, 40, 264, 320, 1), (3, 33, 45, 77, 0), (5, 1, 129, 64, 3), (2, 200, 96, 131, 0)])
+def test_unaligned_pointers_and_batches(batch, M, N, K, off):
+    import torch
+    import clove_compute_amd as cg
+    g = rng("unaligned-b", batch, M, N, K)
+    A = g.integers(-2, 3, (batch, M, K)).astype(np.float16)
+    B = g.integers(-2, 3, (batch, K, N)).astype(np.float16)
+    bufs = []
+    for x in (A, B, np.zeros((batch, M, N), np.float16)):
+        t = torch.full((x.size + 16,), -7.0, dtype=torch.float16, device="cuda")
+        t[off: off + x.size] = to_dev(x).reshape(-1)
+        bufs.append(t)
+    views = [t[off: off + x] for t, x in zip(bufs, (A.size, B.size, batch * M * N))]
+    cg.gemm_fp16_batched(*views, batch, M, N, K)
+    torch.cuda.synchronize()
+    ref = np.matmul(A.astype(np.float32), B.astype(np.float32)).astype(np.float16)
+    got = to_host(bufs[2])
+    assert np.array_equal(got[off: off + ref.size].reshape(ref.shape), ref)
+    assert (got[:off] == -7).all() and (got[off + ref.size:] == -7).all()

@@ -233,3 +233,30 @@ def test_big_tile(M, N, K):
     assert np.array_equal(acc.cpu().numpy()[rows], accref)
     assert np.array_equal(f16bits(to_host(C1)[rows]), f16bits(Cref1))
     assert np.array_equal(f16bits(to_host(C2)[rows]), f16bits(Cref2))
+
+
+# unaligned rows (any K, any N) on the skinny kernel and ragged K on its
+# aligned form, with and without zero points; the GEMV at odd K
+@pytest.mark.parametrize("M,N,K,za,zb", [
+    (1, 17, 17, 3, -5), (2, 1001, 2906, 17, 0), (4, 4096, 2051, -9, 5), (1, 2049, 4097, 0, 0), (3, 12304, 4098, -3, 5),
+    (33, 784, 5246, -3, 5), (64, 1709, 814, -9, 0), (100, 4099, 1158, 0, 0), (130, 333, 4098, -3, 5),
+    (128, 10241, 4097, 7, 0), (300, 2624, 2112, 0, -5), (40, 512, 4176, -3, 5), (513, 1613, 894, 17, 0),
+    (2050, 272, 160, -9, 1),
+])
+def test_unaligned_and_ragged_k_bit_exact(M, N, K, za, zb):
+    g = rng("un8", M, N, K, za, zb)
+    A = g.integers(-128, 128, (M, K)).astype(np.int8)
+    B = g.integers(-128, 128, (K, N)).astype(np.int8)
+    sa = g.uniform(0.001, 0.02, M).astype(np.float16)
+    sb = g.uniform(0.001, 0.02, N).astype(np.float16)
+    s1, s2 = np.float32(g.uniform(0.001, 0.05)), np.float32(g.uniform(0.001, 0.05))
+    C1, C2 = empty_f16(M, N), empty_f16(M, N)
+    _cg().gemm_int8(to_dev(A), to_dev(B), C1, M, N, K, float(s1), za, float(s2), zb)
+    _cg().gemm_int8_rowcol(to_dev(A), to_dev(B), to_dev(sa), to_dev(sb), C2, M, N, K, za, zb)
+    _sync()
+    rows = np.unique(np.concatenate([[0, M // 2, M - 1], g.integers(0, M, 12)]))
+    Cref1, accref = oracle.gemm_int8(A[rows], B, s1, za, s2, zb)
+    Cref2, _ = oracle.gemm_int8_rowcol(A[rows], B, sa[rows], sb, za, zb)
+    assert np.array_equal(run_acc32(A, B, za, zb)[rows], accref)
+    assert np.array_equal(f16bits(to_host(C1)[rows]), f16bits(Cref1))
+    assert np.array_equal(f16bits(to_host(C2)[rows]), f16bits(Cref2))
