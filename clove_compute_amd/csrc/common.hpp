@@ -34,6 +34,20 @@ __device__ __forceinline__ To bitcast(const From& v) {
     return __builtin_bit_cast(To, v);
 }
 
+// Loads and stores at any byte address (one wide instruction: gfx950 takes
+// unaligned global accesses), and the shift of 16 bytes towards byte 0 by s
+// bytes (zero fill)
+typedef unsigned u32x4u __attribute__((ext_vector_type(4), aligned(1)));
+typedef unsigned u32x2u __attribute__((ext_vector_type(2), aligned(1)));
+__device__ __forceinline__ u32x4 load_any16(const unsigned char* p) { return *reinterpret_cast<const u32x4u*>(p); }
+__device__ __forceinline__ u32x4 shift_bytes(u32x4 x, unsigned s) {
+    if (s & 4) x = u32x4{x.y, x.z, x.w, 0u};
+    if (s & 8) x = u32x4{x.z, x.w, 0u, 0u};
+    x = u32x4{__builtin_amdgcn_alignbyte(x.y, x.x, s & 3), __builtin_amdgcn_alignbyte(x.z, x.y, s & 3),
+              __builtin_amdgcn_alignbyte(x.w, x.z, s & 3), x.w >> (8 * (s & 3))};
+    return s >= 16 ? u32x4{0u, 0u, 0u, 0u} : x;
+}
+
 // fp16 <-> fp32 (hardware conversions; narrowing is round-to-nearest-even in
 // the default MODE register)
 __device__ __forceinline__ float h2f(uint16_t h) {

@@ -100,7 +100,8 @@ clove_status_t launch_w4a16(const W4A16Args& args, hipStream_t stream);
 bool try_i4w_w4a16(const W4A16Args& args, int num_cus, hipStream_t stream, clove_status_t* status);
 bool try_i4w_int4(const Int4Args& args, int num_cus, hipStream_t stream, clove_status_t* status);
 // group-wise INT4 x INT4 on int8 MFMA (i4i4_gemm.hip): N >= 64, K % 256 == 0,
-// 16-byte aligned A; zero points in [-112, 127] (others give NaN outputs)
+// 16-byte aligned A; zero points in [-112, 127] (others give NaN outputs); and
+// any K with K % 128 != 0, any alignment, any zero points
 bool try_i4i4(const Int4Args& args, int num_cus, hipStream_t stream, clove_status_t* status);
 // the int8-MFMA kernel's per-group int32 sums P [M, N, G] (test hook; group-wise)
 clove_status_t launch_i4i4_partials(const Int4Args& args, int32_t* P, int num_cus, hipStream_t stream);

@@ -38,7 +38,7 @@ namespace {
 // The shared body of the GEMM and the partials hook: plan, scratch, the Bt
 // pre-pass, the launch.  P != null selects the partials mode (scales unused).
 clove_status_t run(const Int4Args& q, int32_t* P, int cus, hipStream_t stream) {
-    const int G = q.K / 128;
+    const int G = cdiv(q.K, 128);
     const int Npad = cdiv(q.N, BC) * BC;
     Args a{};
     a.A = q.A;
@@ -54,7 +54,13 @@ clove_status_t run(const Int4Args& q, int32_t* P, int cus, hipStream_t stream) {
     a.G = G;
     a.Npad = Npad;
     a.tiles_n = Npad / BC;
-    const Plan pl = plan_for(q.M, a.tiles_n, G, cus);
+    a.B = q.B;
+    a.sB = q.B_scale;
+    a.zB = q.B_zero;
+    a.ldb = (q.N + 1) / 2;
+    const bool anyk = q.K % 256 != 0;
+    const int G2 = G + (G & 1);
+    const Plan pl = plan_for(q.M, a.tiles_n, G2, cus);
     a.tiles_m = pl.tiles_m;
     a.nsplit = pl.nsplit;
     a.gps = pl.gps;
@@ -62,8 +68,8 @@ clove_status_t run(const Int4Args& q, int32_t* P, int cus, hipStream_t stream) {
     const int tiles = a.tiles_m * a.tiles_n;
     const size_t slab = (size_t)BR * BC * 4;  // one fp32 partial tile
     const size_t part_bytes = !P && a.nsplit > 1 ? (size_t)tiles * a.nsplit * slab : 0;
-    const size_t bt_bytes = round256((size_t)Npad * q.K);
-    const size_t sb_bytes = round256((size_t)G * Npad * 4);
+    const size_t bt_bytes = round256((size_t)Npad * G2 * 128);
+    const size_t sb_bytes = round256((size_t)G2 * Npad * 4);
     Scratch s;
     clove_status_t st = acquire_scratch(stream, part_bytes + bt_bytes + sb_bytes, (size_t)tiles, &s);
     if (st != CLOVE_OK) return st;
@@ -74,10 +80,9 @@ clove_status_t run(const Int4Args& q, int32_t* P, int cus, hipStream_t stream) {
     float* sbf = reinterpret_cast<float*>(base + part_bytes + bt_bytes);
     a.Bt = bt;
     a.sBf = sbf;
-    const int ldb = (q.N + 1) / 2;
-    CLOVE_LAUNCH(i4_prep_bt, dim3((unsigned)G, (unsigned)(Npad / PREP_COLS)), dim3(128), 0, stream, q.B, ldb,
+    CLOVE_LAUNCH(anyk ? i4_prep_bt<true> : i4_prep_bt<false>, dim3((unsigned)G2, (unsigned)(Npad / PREP_COLS)), dim3(128), 0, stream, q.B, a.ldb,
                  P ? nullptr : q.B_scale, q.B_zero, q.N, q.K, Npad, bt, sbf);
-    auto k = P ? i4i4_gemm<true> : i4i4_gemm<false>;
+    auto k = P ? i4i4_gemm<true> : anyk ? i4i4_gemm<false, true> : i4i4_gemm<false>;
     if (ensure_lds(reinterpret_cast<const void*>(k), LDS) != CLOVE_OK)
         return CLOVE_ERR_LAUNCH;
     CLOVE_LAUNCH(k, dim3((unsigned)(tiles * a.nsplit)), dim3(NT), LDS, stream, a);
@@ -97,10 +102,22 @@ bool eligible(const Int4Args& q) {
 
 }  // namespace
 
-// Group-wise mode with N >= 64 columns (fewer go to the GEMV / streaming
-// kernels).
+// any other K, any alignment (at least one 16-byte piece of A)
+bool eligible_anyk(const Int4Args& q) {
+    if (q.K <= 0 || (int64_t)q.M * (q.K / 2) < 16) return false;
+    const int64_t G2 = 2 * cdiv(q.K, 256), Npad = cdiv(q.N, BC) * BC;
+    return fits31((int64_t)(q.M + BR) * (q.K / 2) + 256) && fits31(Npad * G2 * 128) && fits31((int64_t)q.M * G2 * 2);
+}
+
+// Group-wise mode with N >= 64 columns and K % 256 == 0 (fewer columns go to
+// the GEMV / streaming kernels, K % 256 == 128 to the INT4-weight kernel, which
+// needs no padding group: 8704 x 132 x 4224 37.8 us there, 62.7 here), and any
+// N > 8 with K % 128 != 0, whose alternative is the generic kernel's byte
+// gathers (us per call: 9856 x 233 x 10076 2058 -> 132, 5634 x 126 x 9196 629
+// -> 41, 8768 x 18 x 4240 207 -> 32, 1728 x 76 x 1534 30 -> 18.5).
 bool try_i4i4(const Int4Args& q, int cus, hipStream_t stream, clove_status_t* status) {
-    if (q.mode != CLOVE_INT4_GROUPWISE || q.N < 64 || !eligible(q)) return false;
+    if (q.mode != CLOVE_INT4_GROUPWISE) return false;
+    if (!(q.N >= 64 && eligible(q)) && !(q.K % 128 != 0 && eligible_anyk(q))) return false;
     *status = run(q, nullptr, cus, stream);
     return true;
 }

@@ -59,6 +59,16 @@
 // where the row's or the column's zero point is outside the exact range), and
 // there is no end phase.
 //
+// Any K (ANYK): K that is not a multiple of 256 leaves weight rows and zA / sA
+// pairs unaligned and a last stage without its second group.  The weight
+// pieces and scale pairs then go through the VGPRs of the same waves (16-byte
+// loads at byte alignment two stages ahead, written to the ring one stage
+// ahead); Bt is padded with zero bytes to whole stages, so whatever a weight
+// row yields past K meets zeros, and the missing group's scales are 0.  These
+// shapes were always accepted with any zero point, so an output that came out
+// NaN (a zero point outside the int8 range, or a scale that is not finite) is
+// computed again from the packed operands, exactly.
+//
 // End.  Set 1 hands its fp32 sums to set 0 through LDS (fixed order).
 // Split-K over groups when the tiles do not cover the CUs: fp32 partial tiles,
 // the last workgroup to arrive sums them in split order (deterministic).  The
@@ -94,6 +104,10 @@ struct Args {
     const int8_t* Bt;     // [G, Npad, 128] int8, qB - zB (i4_prep_bt)
     const float* sBf;     // [G, Npad] fp32, NaN where zB is out of range (i4_prep_bt)
     uint16_t* C;          // [M, N] fp16
+    const uint8_t* B;     // ANYK: packed B, its scales and zero points (recomputed outputs)
+    const uint16_t* sB;
+    const uint16_t* zB;
+    int ldb;
     int M, N, K, G, Npad;
     int tiles_m, tiles_n, nsplit, gps;  // gps: groups per split, even (G is even)
     int vec_store;        // 16-byte output stores (N % 8 == 0, C 16-byte aligned)
@@ -184,7 +198,9 @@ __device__ __forceinline__ void lds_barrier() {
 // [-112, 127]).
 // Grid (G, Npad / 64), 128 threads: the group's 128 packed rows of the
 // 64-column slab are staged in LDS with coalesced loads, then thread (p, kq)
-// writes columns 2p, 2p + 1 for k = 32 kq .. 32 kq + 31.
+// writes columns 2p, 2p + 1 for k = 32 kq .. 32 kq + 31.  ANYK: zero past K
+// and for a padding group.
+template <bool ANYK>
 __global__ void __launch_bounds__(128) i4_prep_bt(const uint8_t* B, int ldb, const uint16_t* sB,
                                                   const uint16_t* zB, int N, int K, int Npad, int8_t* Bt,
                                                   float* sBf) {
@@ -198,7 +214,7 @@ __global__ void __launch_bounds__(128) i4_prep_bt(const uint8_t* B, int ldb, con
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         const int n = 2 * (nb0 + p) + c;
-        if (n < N) {
+        if (n < N && (!ANYK || 128 * g < K)) {
             zh[c] = zB[(int64_t)g * N + n];
             sh[c] = sB ? sB[(int64_t)g * N + n] : (uint16_t)0;
         }
@@ -232,7 +248,7 @@ __global__ void __launch_bounds__(128) i4_prep_bt(const uint8_t* B, int ldb, con
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         const int n = 2 * (nb0 + p) + c;
-        in[c] = n < N;
+        in[c] = n < N && (!ANYK || 128 * g < K);  // (a padding group is zero)
         z[c] = 0;
         s[c] = 0.0f;
         if (in[c]) {
@@ -253,7 +269,7 @@ __global__ void __launch_bounds__(128) i4_prep_bt(const uint8_t* B, int ldb, con
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int q = c == 0 ? (int)(b8[e] >> 4) : (int)(b8[e] & 15u);
-                v[e] = in[c] ? (unsigned)(q - z[c]) & 0xffu : 0u;
+                v[e] = in[c] && (!ANYK || 128 * g + 32 * kq + 8 * j + e < K) ? (unsigned)(q - z[c]) & 0xffu : 0u;
             }
             o[c][2 * j] = v[0] | (v[2] << 8) | (v[4] << 16) | (v[6] << 24);
             o[c][2 * j + 1] = v[1] | (v[3] << 8) | (v[5] << 16) | (v[7] << 24);
@@ -269,8 +285,34 @@ __global__ void __launch_bounds__(128) i4_prep_bt(const uint8_t* B, int ldb, con
     }
 }
 
-template <bool PART>
+// One output from the packed operands, any zero points (see ANYK): the exact
+// integer sum of every group, folded as everywhere else
+__device__ __forceinline__ float exact_output(const Args& p, int row, int col) {
+    float acc = 0.0f;
+    for (int g = 0; g < p.G; ++g) {
+        const float za = rintf(h2f(p.zA[(int64_t)row * p.G + g])), zb = rintf(h2f(p.zB[(int64_t)g * p.N + col]));
+        int qq = 0, qa = 0, qb = 0;
+        const int k1 = min(p.K, 128 * g + 128);
+        for (int k = 128 * g; k < k1; ++k) {
+            const unsigned ab = p.A[(int64_t)row * (p.K >> 1) + (k >> 1)], bb = p.B[(int64_t)k * p.ldb + (col >> 1)];
+            const int a = (int)((k & 1) ? ab & 15u : ab >> 4), b = (int)((col & 1) ? bb & 15u : bb >> 4);
+            qq += a * b;
+            qa += a;
+            qb += b;
+        }
+        float P = __builtin_nanf("");
+        if (fabsf(za) <= 65504.0f && fabsf(zb) <= 65504.0f) {
+            const int64_t ia = (int64_t)za, ib = (int64_t)zb;
+            P = (float)(qq - ib * qa - ia * qb + (int64_t)(k1 - 128 * g) * ia * ib);
+        }
+        acc = fmaf(h2f(p.sA[(int64_t)row * p.G + g]) * h2f(p.sB[(int64_t)g * p.N + col]), P, acc);
+    }
+    return acc;
+}
+
+template <bool PART, bool ANYK = false>
 __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
+    static_assert(!(PART && ANYK), "the partials hook takes whole stages");
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -285,15 +327,16 @@ __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
     const int m0 = tm * BR, n0 = tn * BC;
     const int M = p.M, K = p.K, G = p.G, Npad = p.Npad;
     const int gbeg = split * p.gps;
-    const int gend = min(G, gbeg + p.gps);
+    const int G2 = ANYK ? G + (G & 1) : G;  // groups of Bt / sBf
+    const int gend = min(G2, gbeg + p.gps);
     const int nst = (gend - gbeg) >> 1;  // two groups per stage
 
     const unsigned lds0 = __builtin_amdgcn_readfirstlane(
         (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)smem));
     const int KB = K >> 1;  // bytes per weight row
     const u32x4 ra = make_rsrc(p.A, (unsigned)M * KB);
-    const u32x4 rb = make_rsrc(p.Bt, (unsigned)G * Npad * 128);
-    const u32x4 rs = make_rsrc(p.sBf, (unsigned)G * Npad * 4);
+    const u32x4 rb = make_rsrc(p.Bt, (unsigned)G2 * Npad * 128);
+    const u32x4 rs = make_rsrc(p.sBf, (unsigned)G2 * Npad * 4);
     const u32x4 rza = make_rsrc(p.zA, (unsigned)M * G * 2);
     const u32x4 rsa = make_rsrc(p.sA, (unsigned)M * G * 2);
 
@@ -303,13 +346,15 @@ __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
     // Bt waves: blocks j = 8 (wave - 4) + i = group j >> 4 (one wave-uniform
     //   group per wave), columns 8 (j & 15) .. 8 (j & 15) + 7; wave 4 the
     //   scales of both groups, waves 5-7 a dummy piece
-    int off[8];
+    // (ANYK: a weight wave has two offsets, and off[2..10] hold its pieces and
+    // scale pair in flight -- the registers a Bt wave's offsets take)
+    int off[11];
     int offm = 0;
     if (set == 0) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const int r = 8 * (2 * wave + i) + (lane >> 3);
-            off[i] = (m0 + r) * KB + 16 * ((lane & 7) ^ swz(r));
+            off[i] = (ANYK ? min(m0 + r, M - 1) : m0 + r) * KB + 16 * ((lane & 7) ^ swz(r));
         }
         if (wave < 2) offm = 2 * ((m0 + lane) * G);
     } else {
@@ -328,6 +373,39 @@ __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
         if (wave == 0) dma4(rza, st + ZA_OFF, offm, gs * 2);
         else if (wave == 1) dma4(rsa, st + SA_OFF, offm, gs * 2);
         else dma4(rsa, lds0 + JUNK + 256 * (wave - 2), 0, 0);
+    };
+    // ANYK: the same pieces and scale pairs through registers
+    auto load_a = [&](int t) {
+        const int gs = gbeg + 2 * t;
+        const unsigned a_end = (unsigned)M * KB;
+        if (gs + 2 < G) {  // (whole groups: every piece inside its row)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const u32x4 v = load_any16(p.A + (unsigned)(off[i] + gs * 64));
+#pragma unroll
+                for (int d = 0; d < 4; ++d) off[2 + 4 * i + d] = (int)v[d];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const unsigned o = (unsigned)(off[i] + gs * 64), at = min(o, a_end - 16);
+                const u32x4 v = shift_bytes(load_any16(p.A + at), o - at);
+#pragma unroll
+                for (int d = 0; d < 4; ++d) off[2 + 4 * i + d] = (int)v[d];
+            }
+        }
+        if (wave < 2) {
+            const uint16_t* src = (wave == 0 ? p.zA : p.sA) + (int64_t)min(m0 + lane, M - 1) * G;
+            off[10] = (int)(src[gs] | (gs + 1 < G ? (unsigned)src[gs + 1] << 16 : 0u));
+        }
+    };
+    auto put_a = [&](int t) {
+        const unsigned st = lds0 + (unsigned)((t % LA) * AST);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            *reinterpret_cast<lds_u32x4*>((size_t)(st + (2 * wave + i) * 1024 + 16 * lane)) =
+                u32x4{(unsigned)off[2 + 4 * i], (unsigned)off[3 + 4 * i], (unsigned)off[4 + 4 * i], (unsigned)off[5 + 4 * i]};
+        if (wave < 2) *reinterpret_cast<lds_u32*>((size_t)(st + (wave == 0 ? ZA_OFF : SA_OFF) + 4 * lane)) = (unsigned)off[10];
     };
     auto issue_b = [&](int t) {
         const int gs = gbeg + 2 * t;
@@ -361,11 +439,19 @@ __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
     auto step = [&](int t, i32x16 (&cur)[NB], f32x16 (&spc)[NB], const i32x16 (&prev)[NB],
                     const f32x16 (&spp)[NB]) {
         const int rem = nst - 1 - t;
-        if (set == 0) wait_stages<DA>(min(rem, LA - 2));
-        else wait_stages<DB>(min(rem, LB - 2));
+        if (set == 0) {
+            if constexpr (!ANYK) wait_stages<DA>(min(rem, LA - 2));
+        } else {
+            wait_stages<DB>(min(rem, LB - 2));
+        }
         lds_barrier();
         if (set == 0) {
-            if (t + LA - 1 < nst) issue_a(t + LA - 1);
+            if constexpr (ANYK) {
+                if (t + 1 < nst) put_a(t + 1);
+                if (t + 2 < nst) load_a(t + 2);
+            } else {
+                if (t + LA - 1 < nst) issue_a(t + LA - 1);
+            }
         } else {
             if (t + LB - 1 < nst) issue_b(t + LB - 1);
         }
@@ -502,9 +588,16 @@ __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
 
     // ---- prologue: each stream fills its ring ----
     if (set == 0) {
+        if constexpr (ANYK) {
+            static_assert(LA == 2, "one stage written ahead");
+            load_a(0);
+            put_a(0);
+            if (nst > 1) load_a(1);
+        } else {
 #pragma unroll
-        for (int t = 0; t < LA - 1; ++t)
-            if (t < nst) issue_a(t);
+            for (int t = 0; t < LA - 1; ++t)
+                if (t < nst) issue_a(t);
+        }
     } else {
 #pragma unroll
         for (int t = 0; t < LB - 1; ++t)
@@ -608,6 +701,23 @@ __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
         if (gm >= M) continue;
         const u32x4 v = ld16(lds0 + 2 * (row * PITCH + 8 * cc));
         uint16_t* dst = p.C + (int64_t)gm * p.N + gn;
+        if constexpr (ANYK) {
+            bool nan = false;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                nan |= (v[e] & 0x7fffu) > 0x7c00u || (v[e] & 0x7fff0000u) > 0x7c000000u;
+            if (nan) {
+                u32x4 w = v;
+#pragma unroll 1
+                for (int e = 0; e < 8 && gn + e < p.N; ++e) {
+                    uint16_t hv = (uint16_t)w.x;
+                    w = u32x4{(w.x >> 16) | (w.y << 16), (w.y >> 16) | (w.z << 16), (w.z >> 16) | (w.w << 16), w.w >> 16};
+                    if ((hv & 0x7fffu) > 0x7c00u) hv = f2h(exact_output(p, gm, gn + e));
+                    dst[e] = hv;
+                }
+                continue;
+            }
+        }
         if (p.vec_store && gn + 7 < p.N) {
             *reinterpret_cast<u32x4*>(dst) = v;
         } else {

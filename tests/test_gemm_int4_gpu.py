@@ -240,6 +240,42 @@ def test_int8_mfma_path_zero_point_outside_range_is_nan():
     assert ok, rep
 
 
+# any K on the int8-MFMA kernel (weight rows through registers, a last stage
+# with one group, a cut last group): zero points in and outside the int8 range
+# (an affected output is computed again), every step exact, so bit for bit;
+# N < 64 with K % 128 != 0 takes it too.  The packed operands end at the
+# buffer's end or in bytes that would change the sums.
+@pytest.mark.parametrize("M,N,K,wild", [
+    (130, 64, 382, False), (64, 9, 2, False), (1, 100, 66, False), (257, 136, 1154, True), (65, 40, 330, True),
+    (200, 18, 4240, False), (300, 129, 4222, True), (513, 77, 2942, False), (1000, 200, 130, False),
+])
+def test_int8_mfma_path_any_k_bit_exact(M, N, K, wild):
+    import torch
+    g = rng("i4i4-anyk", M, N, K)
+    G = (K + 127) // 128
+    A_q = quant.pack_rows(g.integers(0, 16, (M, K)))
+    B_q = quant.pack_cols(g.integers(0, 16, (K, N)))
+    ends = np.array([-112, 127, 0, 15, 8], np.float16)
+    zA = ends[g.integers(0, 5, (M, G))]
+    zB = ends[g.integers(0, 5, (G, N))]
+    if wild:
+        zA[M // 3, G // 2] = 300.0
+        zB[0, N // 2] = -250.0
+    # one power of two for every scale, small enough for finite fp16 results
+    sA = np.full((M, G), 2.0 ** -10, np.float16)
+    sB = np.full((G, N), 2.0 ** -8, np.float16)
+    bufs = []
+    for x in (A_q, B_q):
+        t = torch.full((x.size + 64,), 0xA5, dtype=torch.uint8, device="cuda")
+        t[: x.size] = to_dev(x).reshape(-1)
+        bufs.append(t)
+    C = empty_f16(M, N, fill=float("nan"))
+    _cg().gemm_int4(bufs[0], to_dev(sA), to_dev(zA), bufs[1], to_dev(sB), to_dev(zB), C, M, N, K)
+    torch.cuda.synchronize()
+    _, ref, _ = oracle.gemm_int4_groupwise(A_q, sA, zA, B_q, sB, zB, M, N, K)
+    assert np.array_equal(f16bits(to_host(C)), f16bits(ref.astype(np.float16)))
+
+
 @pytest.mark.parametrize("M,N,K", [(4096, 128, 11008), (600, 100, 2816), (1000, 320, 1024),
                                    (11008, 128, 4096), (8192, 512, 512)])
 def test_int8_mfma_path_split_k(M, N, K):
