@@ -61,6 +61,33 @@ __device__ __forceinline__ uint16_t f2h(float f) {
     asm("" : "+v"(f));
     return bitcast<uint16_t>(static_cast<_Float16>(f));
 }
+
+// One output of the group-wise INT4 product from the packed operands, any zero
+// points: the exact integer sum of every group, folded in group order
+__device__ __forceinline__ float int4_exact_output(const uint8_t* A, const uint16_t* sA, const uint16_t* zA,
+                                                   const uint8_t* B, const uint16_t* sB, const uint16_t* zB, int row,
+                                                   int col, int N, int K, int G, int ldb) {
+    float acc = 0.0f;
+    for (int g = 0; g < G; ++g) {
+        const float za = rintf(h2f(zA[(int64_t)row * G + g])), zb = rintf(h2f(zB[(int64_t)g * N + col]));
+        int qq = 0, qa = 0, qb = 0;
+        const int k1 = min(K, 128 * g + 128);
+        for (int k = 128 * g; k < k1; ++k) {
+            const unsigned ab = A[(int64_t)row * (K >> 1) + (k >> 1)], bb = B[(int64_t)k * ldb + (col >> 1)];
+            const int a = (int)((k & 1) ? ab & 15u : ab >> 4), b = (int)((col & 1) ? bb & 15u : bb >> 4);
+            qq += a * b;
+            qa += a;
+            qb += b;
+        }
+        float P = __builtin_nanf("");
+        if (fabsf(za) <= 65504.0f && fabsf(zb) <= 65504.0f) {
+            const int64_t ia = (int64_t)za, ib = (int64_t)zb;
+            P = (float)(qq - ib * qa - ia * qb + (int64_t)(k1 - 128 * g) * ia * ib);
+        }
+        acc = fmaf(h2f(sA[(int64_t)row * G + g]) * h2f(sB[(int64_t)g * N + col]), P, acc);
+    }
+    return acc;
+}
 __device__ __forceinline__ unsigned pack2h(float lo, float hi) {
     return static_cast<unsigned>(f2h(lo)) | (static_cast<unsigned>(f2h(hi)) << 16);
 }

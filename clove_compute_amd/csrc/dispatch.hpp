@@ -98,6 +98,7 @@ clove_status_t launch_w4a16(const W4A16Args& args, hipStream_t stream);
 // what the kernel handles (the caller then takes its general path); otherwise
 // it launches and stores the launch status in *status.
 bool try_i4w_w4a16(const W4A16Args& args, int num_cus, hipStream_t stream, clove_status_t* status);
+bool try_i4w_int4_rawb(const Int4Args& args, int num_cus, hipStream_t stream, clove_status_t* status);
 bool try_i4w_int4(const Int4Args& args, int num_cus, hipStream_t stream, clove_status_t* status);
 // group-wise INT4 x INT4 on int8 MFMA (i4i4_gemm.hip): N >= 64, K % 256 == 0,
 // 16-byte aligned A; zero points in [-112, 127] (others give NaN outputs); and

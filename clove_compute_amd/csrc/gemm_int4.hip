@@ -610,6 +610,7 @@ clove_status_t launch_gemm_int4(const Int4Args& a, hipStream_t stream) {
     const int ldb = literal ? a.N / 2 : (a.N + 1) / 2;
     const int cols_valid = literal ? 2 * (a.N / 2) : a.N;
     const int nch = cdiv(a.K, 32);
+    clove_status_t st2;
     if (a.K == 0) {
         // empty sum: +0 in both modes (the reference reads no scale group then)
         const size_t n = (size_t)a.M * a.N;
@@ -617,6 +618,16 @@ clove_status_t launch_gemm_int4(const Int4Args& a, hipStream_t stream) {
                            stream, a.C, n, (uint16_t)0);
         return check_launch();
     }
+    // five to eight columns: B read in place by the INT4-weight streaming kernel,
+    // whose MFMAs cost the same for 3 or 16 columns, where the GEMV's VALU work
+    // grows with them.  Cold, us per call, GEMV against stream: 11008 x 4096 N = 3
+    // / 4 / 5 / 8 9.7 / 9.9 / 19.4 / 15.1 against 10.1 / 10.2 / 11.0 / 10.0,
+    // 4096 x 11008 N = 4 / 5 / 8 12.2 / 29.9 / 20.8 against 12.6 / 12.1 / 10.7;
+    // small weights stay (1280 x 1664 N = 8 5.2 against 6.2; 2048 x 5504 10.7
+    // against 8.0)
+    if (a.N >= 5 && (a.N > 8 || (int64_t)a.M * a.K >= ((int64_t)4 << 20)) &&
+        try_i4w_int4_rawb(a, dev.num_cus, stream, &st2))
+        return st2;
     if (a.N <= 8 && gemv_lds_bytes(a.N <= 2 ? a.N : (a.N <= 4 ? 4 : 8), nch, G) <= kMaxGemvLds) {
         GemvParams p{a.A, a.A_scale, a.A_zero, a.B, a.B_scale, a.B_zero, a.C,
                      a.M, a.N, a.K, G, ldb, cols_valid, nch};
@@ -625,7 +636,6 @@ clove_status_t launch_gemm_int4(const Int4Args& a, hipStream_t stream) {
                        : gemv_by_n<mg::kI4Groupwise>(p, aligned, dev.num_cus, stream);
     }
     if (!literal) {
-        clove_status_t st2;
         if (try_i4i4(a, dev.num_cus, stream, &st2)) return st2;
         if (try_i4w_int4(a, dev.num_cus, stream, &st2)) return st2;
     }

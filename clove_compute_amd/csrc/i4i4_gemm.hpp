@@ -285,31 +285,6 @@ __global__ void __launch_bounds__(128) i4_prep_bt(const uint8_t* B, int ldb, con
     }
 }
 
-// One output from the packed operands, any zero points (see ANYK): the exact
-// integer sum of every group, folded as everywhere else
-__device__ __forceinline__ float exact_output(const Args& p, int row, int col) {
-    float acc = 0.0f;
-    for (int g = 0; g < p.G; ++g) {
-        const float za = rintf(h2f(p.zA[(int64_t)row * p.G + g])), zb = rintf(h2f(p.zB[(int64_t)g * p.N + col]));
-        int qq = 0, qa = 0, qb = 0;
-        const int k1 = min(p.K, 128 * g + 128);
-        for (int k = 128 * g; k < k1; ++k) {
-            const unsigned ab = p.A[(int64_t)row * (p.K >> 1) + (k >> 1)], bb = p.B[(int64_t)k * p.ldb + (col >> 1)];
-            const int a = (int)((k & 1) ? ab & 15u : ab >> 4), b = (int)((col & 1) ? bb & 15u : bb >> 4);
-            qq += a * b;
-            qa += a;
-            qb += b;
-        }
-        float P = __builtin_nanf("");
-        if (fabsf(za) <= 65504.0f && fabsf(zb) <= 65504.0f) {
-            const int64_t ia = (int64_t)za, ib = (int64_t)zb;
-            P = (float)(qq - ib * qa - ia * qb + (int64_t)(k1 - 128 * g) * ia * ib);
-        }
-        acc = fmaf(h2f(p.sA[(int64_t)row * p.G + g]) * h2f(p.sB[(int64_t)g * p.N + col]), P, acc);
-    }
-    return acc;
-}
-
 template <bool PART, bool ANYK = false>
 __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
     static_assert(!(PART && ANYK), "the partials hook takes whole stages");
@@ -712,7 +687,8 @@ __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
                 for (int e = 0; e < 8 && gn + e < p.N; ++e) {
                     uint16_t hv = (uint16_t)w.x;
                     w = u32x4{(w.x >> 16) | (w.y << 16), (w.y >> 16) | (w.z << 16), (w.z >> 16) | (w.w << 16), w.w >> 16};
-                    if ((hv & 0x7fffu) > 0x7c00u) hv = f2h(exact_output(p, gm, gn + e));
+                    if ((hv & 0x7fffu) > 0x7c00u)
+                        hv = f2h(int4_exact_output(p.A, p.sA, p.zA, p.B, p.sB, p.zB, gm, gn + e, p.N, K, G, p.ldb));
                     dst[e] = hv;
                 }
                 continue;

@@ -18,7 +18,13 @@ using CfgBig = Cfg<4, 1, 2, 4, 3>;  // 256 x 128, 4 waves of 64 x 128
 // a larger burst of the grid's prologue loads (W4A16 Llama-1B layer T = 512
 // 125.6 -> 122.9 us, fused 114.9 -> 111.1 us against three stages)
 using CfgC64 = Cfg<4, 1, 1, 2, 2>;
-using CfgC32 = Cfg<2, 1, 1, 1, 4>;  // 64 x 32, 2 waves (several workgroups per CU)
+// the same with two stages ahead (75 KB), where the grid leaves a CU one
+// workgroup: nothing else then covers a stage's round trip (W4A16, cold, T =
+// 140 on 3328 x 7424 25.3 -> 23.0 us, 187 on 1920 x 11008 27.2 -> 23.4)
+using CfgC64S3 = Cfg<4, 1, 1, 2, 3>;
+// 128 x 32, three stages ahead (70 KB LDS: two workgroups per CU): few X rows
+// or few tiles, where a workgroup's chain of stages is the time
+using CfgC32 = Cfg<4, 1, 1, 1, 4>;
 // 256 x 64 (four waves of 64 x 64), one stage ahead (70 KB LDS: two workgroups
 // per CU): the fused gate/up + SwiGLU from 512 X rows up, where each wave's two
 // weight blocks (a gate and an up block per 32 outputs) share every X
@@ -94,18 +100,31 @@ clove_status_t run(Args a, int cus, int target, int min_groups, size_t extra_byt
     return check_launch();
 }
 
-// Tile choice by the number of X rows C (measured on MI355X):
-//   C <= 32: 64 x 32, two waves, three workgroups per CU (HBM-bound)
+// Tile choice by the number of X rows C (measured on MI355X, cold graph
+// replays, 130 W4A16 and 90 INT4 shapes; us per call):
+//   128 x 32 for C <= 32, and while these tiles fit the CUs once and tiles x
+//   groups stay under 16 a CU, where a stage's latency and not its MFMAs is the
+//   time (against 128 x 64: W4A16 T = 64 on 3072 x 2048 11.2 -> 8.0, 100 on
+//   2432 x 1920 13.9 -> 9.3, 427 on 1920 x 1536 12.7 -> 10.2; past it 140 on
+//   3328 x 7424, 130 tiles x 58 groups, 33.3 against 23.0; INT4 1216 x 55 x
+//   2560 18.7 -> 12.6).  For C <= 32 it replaced 64 x 32 tiles of two waves
+//   (fused SwiGLU 22016 x 4096 T = 16 26.0 -> 19.6, 16384 x 2048 11.4 -> 9.8)
+//   128 x 64 with two stages ahead while those tiles cover less than 3/8 of
+//   the CUs, split to one workgroup per CU
 //   otherwise 128 x 64 with two workgroups per CU, whose waves interleave
 //   VALU (unpack, fold) with MFMA -- ahead of 128 x 128 by 15-25 % on the
 //   INT4 N = 128 and W4A16 T = 512 shapes -- unless 256 x 128 tiles already
 //   cover the CUs (large prefill); the fused SwiGLU from 512 X rows up: 256 x
 //   128 with eight waves where those tiles cover 3/4 of the CUs, else 256 x 64
-// Splits keep at least 10 (64 x 32) or 8 groups each.
+// Splits keep at least 4 groups each (8 where two workgroups share a CU).
 template <bool XS, int OUT, class Prep>
 clove_status_t by_shape(const Args& a, int cus, size_t extra_bytes, hipStream_t stream, Prep prep) {
     const int rows = OUT == 2 ? 2 * a.R : a.R;  // weight rows
-    if (a.C <= 32) return run<CfgC32, XS, OUT>(a, cus, 3 * cus, 10, extra_bytes, stream, prep);
+    const int64_t t32 = (int64_t)cdiv(rows, CfgC32::BR) * cdiv(a.C, CfgC32::BC);
+    if (a.C <= 32 || (t32 <= cus && t32 * a.G <= 16 * cus))
+        return run<CfgC32, XS, OUT>(a, cus, cus, a.G > 44 ? 8 : 4, extra_bytes, stream, prep);
+    if (8 * (int64_t)cdiv(rows, CfgC64::BR) * cdiv(a.C, CfgC64::BC) < 3 * cus)
+        return run<CfgC64S3, XS, OUT>(a, cus, cus, 4, extra_bytes, stream, prep);
     if (OUT == 2 && a.C >= 512) {
         if (4 * cdiv(rows, CfgS128::BR) * cdiv(a.C, CfgS128::BC) >= 3 * cus)
             return run<CfgS128, XS, OUT>(a, cus, cus, 8, extra_bytes, stream, prep);
@@ -121,7 +140,7 @@ clove_status_t by_shape(const Args& a, int cus, size_t extra_bytes, hipStream_t 
 bool fits31(int64_t bytes) { return bytes < ((int64_t)1 << 31); }
 
 // ---- the streaming kernel (i4w_stream.hpp) for C <= 32 X rows ----
-template <int WF, int XF, int NG, int KS, bool XS, int OUT, bool RAWB>
+template <int WF, int XF, int NG, int KS, bool XS, int OUT, int RAWB>
 clove_status_t launch_stream(const Args& a, hipStream_t stream) {
     using SC = SCfg<WF, XF, NG, KS>;
     const int lds = SC::lds_bytes(a.G, XS, RAWB);
@@ -132,62 +151,76 @@ clove_status_t launch_stream(const Args& a, hipStream_t stream) {
     return check_launch();
 }
 
-// K slices: the fewest waves (2, 4 or 8) that leave each at most 11 groups,
-// unrolled for 8 groups when that suffices
+// K slices: 4 or 8 waves of at most 11 groups.  Short slices: a wave's chain
+// of groups is most of a small product's time (cold, us per call, against the
+// fewest waves that hold K: W4A16 T = 13 on 8128 x 1280 6.9 -> 5.2, INT4 N =
+// 12 on 10496 x 1152 7.5 -> 5.8, N = 19 on 1984 x 1920 7.2 -> 5.4, N = 9 on
+// 3840 x 5760 9.0 -> 7.6).  For 17..32 groups INT4 takes 8 waves (N = 27 on
+// 7552 x 2304 9.2 -> 8.5 against 4), W4A16 4 (T = 19 on 3712 x 3584 the same;
+// four waves leave room for more workgroups); 33..44 groups stay on 4 (INT4 N
+// = 12 on 11840 x 4864 12.4 against 13.5).
 // (BIG_G = false: the caller never passes more than 64 groups, and the
 // 11-group, 8-slice variant is not instantiated)
-template <int WF, int XF, bool XS, int OUT, bool RAWB = false, bool BIG_G = true>
+template <int WF, int XF, bool XS, int OUT, int RAWB = 0, bool BIG_G = true>
 clove_status_t stream_by_k(const Args& a, hipStream_t stream) {
     const int G = a.G;
-    if (G <= 16) return launch_stream<WF, XF, 8, 2, XS, OUT, RAWB>(a, stream);
-    if (G <= 22) return launch_stream<WF, XF, 11, 2, XS, OUT, RAWB>(a, stream);
-    if (G <= 32) return launch_stream<WF, XF, 8, 4, XS, OUT, RAWB>(a, stream);
+    if (G <= 12) return launch_stream<WF, XF, 3, 4, XS, OUT, RAWB>(a, stream);
+    if (G <= 16) return launch_stream<WF, XF, 4, 4, XS, OUT, RAWB>(a, stream);
+    if constexpr (XS) {
+        if (G <= 24) return launch_stream<WF, XF, 3, 8, XS, OUT, RAWB>(a, stream);
+        if (G <= 32) return launch_stream<WF, XF, 4, 8, XS, OUT, RAWB>(a, stream);
+    } else {
+        if (G <= 24) return launch_stream<WF, XF, 6, 4, XS, OUT, RAWB>(a, stream);
+        if (G <= 32) return launch_stream<WF, XF, 8, 4, XS, OUT, RAWB>(a, stream);
+    }
     if (G <= 44) return launch_stream<WF, XF, 11, 4, XS, OUT, RAWB>(a, stream);
-    if (!BIG_G || G <= 64) return launch_stream<WF, XF, 8, 8, XS, OUT, RAWB>(a, stream);
-    if constexpr (BIG_G) return launch_stream<WF, XF, 11, 8, XS, OUT, RAWB>(a, stream);
+    if constexpr (!(XS && XF == 2)) {  // (kRawB2MaxGroups)
+        if (G <= 48) return launch_stream<WF, XF, 6, 8, XS, OUT, RAWB>(a, stream);
+        if (!BIG_G || G <= 64) return launch_stream<WF, XF, 8, 8, XS, OUT, RAWB>(a, stream);
+        if constexpr (BIG_G) return launch_stream<WF, XF, 11, 8, XS, OUT, RAWB>(a, stream);
+    }
     return CLOVE_ERR_INVALID_ARG;
 }
 
 constexpr int kStreamMaxGroups = 88;  // K <= 11264
 
-// Two weight fragments (32 rows) per workgroup when that still gives every
-// CU a workgroup, else one (measured on the 11008 x 4096 and 4096 x 11008
-// shapes: 32 rows and 4 slices, 16 rows and 8 slices)
-// INT4 (XS) reaches this with at most 16 columns, so only one X fragment.
+// Two weight fragments (32 rows) per workgroup once one fragment each would
+// take a second round of the CUs (X is then read half as often; W4A16 T = 10
+// on 5184 x 5248 11.5 -> 9.6 us, 14 on 13184 x 1280 8.9 -> 7.3).
 // Two X fragments with two weight fragments and 11-group slices (K > 8192)
 // need more registers than a lane has: those take one weight fragment.
-template <bool XS, int OUT>
+bool stream_two_rows(const Args& a, int cus) { return cdiv(a.R, 16) > cus && (a.C <= 16 || a.G <= 64); }
+
 clove_status_t run_stream(const Args& a, int cus, hipStream_t stream) {
-    const bool wf2 = cdiv(a.R, 32) >= cus;
-    if (XS || a.C <= 16) return wf2 ? stream_by_k<2, 1, XS, OUT>(a, stream) : stream_by_k<1, 1, XS, OUT>(a, stream);
-    if constexpr (!XS) {
-        if (wf2 && a.G <= 64) return stream_by_k<2, 2, XS, OUT, false, false>(a, stream);
-        return stream_by_k<1, 2, XS, OUT>(a, stream);
-    }
-    return CLOVE_ERR_INVALID_ARG;
+    const bool wf2 = stream_two_rows(a, cus);
+    if (a.C <= 16) return wf2 ? stream_by_k<2, 1, false, 1>(a, stream) : stream_by_k<1, 1, false, 1>(a, stream);
+    if (wf2) return stream_by_k<2, 2, false, 1, 0, false>(a, stream);
+    return stream_by_k<1, 2, false, 1>(a, stream);
 }
 
 // Every workgroup of the streaming kernel reads all of X (C rows x K fp16),
 // so its cost grows with C x K per CU, while the split-K MFMA kernel reads
-// each X tile once per 64 weight rows and is flat in C.  Measured (W4A16,
-// T = 5..32 on 8192x2048, 2048x8192, 4096x4096, 4096x11008, 11008x4096): the
-// stream is ahead below ~256 KB of X per CU, counting one copy per round of
-// workgroups on a CU, and the MFMA kernel from there (4096x11008 T = 32:
-// 26.3 against 16.4 us; 2048x8192 T = 16: 12.2 against 10.8 us).
+// each X tile once per 128 weight rows and is flat in C.  Measured (W4A16, 90
+// shapes, T = 2..32, O 1024..11008, K 1024..11008; cold, us per call, stream
+// against 128 x 32 tiles): up to 16 rows the stream is ahead below ~200 KB of
+// X per CU, counting one copy per round of workgroups on a CU (T = 13 on 2048
+// x 7424, 188 KB, 10.5 against 11.1; 2176 x 8704, 221 KB, 13.6 against 11.9);
+// with two X fragments below ~128 KB and in one round (T = 24 on 2944 x 1664
+// 5.7 against 7.4; T = 32 on 4864 x 2304, 144 KB, 10.4 against 8.1; T = 20 on
+// 9216 x 1152, 90 KB in two rounds, 9.2 against 7.3).
 bool stream_ahead(const Args& a, int cus) {
-    const bool wf2 = cdiv(a.R, 32) >= cus && (a.C <= 16 || a.G <= 64);  // run_stream's weight fragments
-    const int64_t rounds = cdiv(cdiv(a.R, wf2 ? 32 : 16), cus);
-    return (int64_t)a.C * a.K * 2 * rounds < 256 * 1024;
+    const int64_t rounds = cdiv(cdiv(a.R, stream_two_rows(a, cus) ? 32 : 16), cus);
+    const int64_t bytes = (int64_t)a.C * a.K * 2 * rounds;
+    return a.C <= 16 ? bytes < 200 * 1024 : rounds == 1 && bytes < 128 * 1024;
 }
 
 }  // namespace
 
 bool try_i4w_w4a16(const W4A16Args& w, int cus, hipStream_t stream, clove_status_t* status) {
-    // three or four tokens on large weights: the streaming kernel rather than
-    // the GEMV (cold, T = 4: 4096x11008 12.1 against 22.0 us, 4096x4096 5.8
-    // against 8.0; 2048x2048 stays on the GEMV, 4.2 against 4.6)
-    const bool small_t = w.T <= 2 || (w.T <= 4 && (int64_t)w.O * w.K <= ((int64_t)8 << 20));
-    if (small_t || w.K <= 0 || w.K % 128 != 0 || !aligned16(w.X) || !aligned16(w.W)) return false;
+    // three or four tokens: the streaming kernel rather than the GEMV (cold,
+    // T = 4: 4096x11008 12.1 against 22.0 us, 2176x2176 4.3 against 6.7, 1024 x
+    // 1664 3.7 against 4.0; at T = 2 neither is ahead throughout)
+    if (w.T <= 2 || w.K <= 0 || w.K % 128 != 0 || !aligned16(w.X) || !aligned16(w.W)) return false;
     if (!fits31((int64_t)w.T * w.K * 2) || !fits31((int64_t)w.O * (w.K / 2))) return false;
     Args a{};
     a.W = w.W;
@@ -202,7 +235,7 @@ bool try_i4w_w4a16(const W4A16Args& w, int cus, hipStream_t stream, clove_status
     a.alpha = w.alpha;
     a.beta = w.beta;
     if (w.T <= 32 && a.G <= kStreamMaxGroups && stream_ahead(a, cus)) {
-        *status = run_stream<false, 1>(a, cus, stream);
+        *status = run_stream(a, cus, stream);
         return true;
     }
     if (w.T <= 4) return false;  // (the GEMV, outside the stream's domain)
@@ -211,7 +244,7 @@ bool try_i4w_w4a16(const W4A16Args& w, int cus, hipStream_t stream, clove_status
 }
 
 bool try_i4w_w4a16_swiglu(const W4A16Args& w, int cus, hipStream_t stream, clove_status_t* status) {
-    if (w.T <= 4 || w.K <= 0 || w.K % 128 != 0 || !aligned16(w.X) || !aligned16(w.W)) return false;
+    if (w.T <= 2 || w.K <= 0 || w.K % 128 != 0 || !aligned16(w.X) || !aligned16(w.W)) return false;
     if (!fits31((int64_t)w.T * w.K * 2) || !fits31((int64_t)2 * w.O * (w.K / 2))) return false;
     Args a{};
     a.W = w.W;
@@ -229,10 +262,10 @@ bool try_i4w_w4a16_swiglu(const W4A16Args& w, int cus, hipStream_t stream, clove
     return true;
 }
 
-bool try_i4w_int4_rawb(const Int4Args& q, int cus, hipStream_t stream, clove_status_t* status);
+// (raw B with two column fragments: K <= 5632, 88 KB of B in LDS)
+constexpr int kRawB2MaxGroups = 44;
 
 bool try_i4w_int4(const Int4Args& q, int cus, hipStream_t stream, clove_status_t* status) {
-    if (try_i4w_int4_rawb(q, cus, stream, status)) return true;
     if (q.mode != CLOVE_INT4_GROUPWISE || q.N <= 8 || q.K <= 0 || q.K % 128 != 0 || !aligned16(q.A))
         return false;
     const int Npad = (q.N + 63) / 64 * 64;
@@ -262,15 +295,6 @@ bool try_i4w_int4(const Int4Args& q, int cus, hipStream_t stream, clove_status_t
         args.xs = xs;
         return check_launch();
     };
-    if (q.N <= 16 && G <= kStreamMaxGroups) {
-        // the B transpose into scratch, then the streaming kernel
-        Scratch s;
-        clove_status_t st = acquire_scratch(stream, xt_bytes + xs_bytes, 0, &s);
-        if (st == CLOVE_OK) st = prep(a, reinterpret_cast<char*>(s.partials));
-        if (st == CLOVE_OK) st = run_stream<true, 0>(a, cus, stream);
-        *status = st;
-        return true;
-    }
     *status = by_shape<true, 0>(a, cus, xt_bytes + xs_bytes, stream, prep);
     return true;
 }
@@ -297,11 +321,13 @@ int rawb_wf(int R, int G, int cus) {
 }
 
 bool try_i4w_int4_rawb(const Int4Args& q, int cus, hipStream_t stream, clove_status_t* status) {
-    // 15 or 16 columns: B rows are 8 bytes, read in place (no transpose pass)
+    // up to 32 columns: B rows of at most 16 bytes, read in place (no transpose pass)
     const int G = q.K / 128;
-    if (q.mode != CLOVE_INT4_GROUPWISE || (q.N != 15 && q.N != 16) || q.K <= 0 || q.K % 128 != 0 ||
-        G > kStreamMaxGroups || !aligned16(q.A) || !aligned16(q.B) || !fits31((int64_t)q.M * (q.K / 2)))
+    if (q.mode != CLOVE_INT4_GROUPWISE || q.N < 3 || q.N > 32 || q.K <= 0 || q.K % 128 != 0 || !aligned16(q.A) ||
+        !fits31((int64_t)q.M * (q.K / 2)))
         return false;
+    // (B and its constants stay in LDS whole)
+    if (G > (q.N <= 16 ? kStreamMaxGroups : kRawB2MaxGroups)) return false;
     Args a{};
     a.W = q.A;
     a.wscale = q.A_scale;
@@ -315,12 +341,22 @@ bool try_i4w_int4_rawb(const Int4Args& q, int cus, hipStream_t stream, clove_sta
     a.bscale = q.B_scale;
     a.bzero = q.B_zero;
     a.N = q.N;
+    a.ldb = (q.N + 1) / 2;
     a.alpha = 1.0f;
     a.beta = 0.0f;
     const int wf = rawb_wf(a.R, G, cus);
-    *status = wf == 3   ? stream_by_k<3, 1, true, 0, true>(a, stream)
-              : wf == 2 ? stream_by_k<2, 1, true, 0, true>(a, stream)
-                        : stream_by_k<1, 1, true, 0, true>(a, stream);
+    if (q.N > 16) {
+        *status = wf >= 2 ? stream_by_k<2, 2, true, 0, 2, false>(a, stream) : stream_by_k<1, 2, true, 0, 2, false>(a, stream);
+        return true;
+    }
+    if (a.ldb == 8 && aligned16(q.B))
+        *status = wf == 3   ? stream_by_k<3, 1, true, 0, 1>(a, stream)
+                  : wf == 2 ? stream_by_k<2, 1, true, 0, 1>(a, stream)
+                            : stream_by_k<1, 1, true, 0, 1>(a, stream);
+    else
+        *status = wf == 3   ? stream_by_k<3, 1, true, 0, 2>(a, stream)
+                  : wf == 2 ? stream_by_k<2, 1, true, 0, 2>(a, stream)
+                            : stream_by_k<1, 1, true, 0, 2>(a, stream);
     return true;
 }
 

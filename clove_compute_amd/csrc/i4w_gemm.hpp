@@ -1,5 +1,5 @@
 // MFMA GEMM with packed INT4 weight rows for gfx950: the prefill shapes of the
-// W4A16 linear layer (T > 4 tokens) and of group-wise INT4 (N > 8 columns).
+// W4A16 linear layer (T > 2 tokens) and of group-wise INT4 (N > 8 columns).
 //
 //   out[r, c] = sum_g  sw[r,g] * sx[g,c] * P_g[r,c]
 //   P_g[r,c]  = sum_{k in group g} (q[r,k] - zw[r,g]) * x[c,k]
@@ -70,11 +70,11 @@ struct Args {
     float* part;
     unsigned* counters;
     // raw group-wise INT4 B for the streaming kernel's fused transpose
-    // (i4w_stream.hpp): B [K, 8] bytes (N = 15 or 16), sB / zB [G, N] fp16
+    // (i4w_stream.hpp): B [K, ldb] bytes (ldb <= 16), sB / zB [G, N] fp16
     const uint8_t* B;
     const uint16_t* bscale;
     const uint16_t* bzero;
-    int N;
+    int N, ldb;
 };
 
 // KS: 16-wide k-steps per stage, 8 (a whole 128-k group) or 4 (half a group:

@@ -1,5 +1,5 @@
 // Streaming MFMA GEMM with packed INT4 weight rows for few X rows (C <= 32):
-// group-wise INT4 with N in 9..32 columns and W4A16 with 5..32 tokens.  The
+// group-wise INT4 with 5..32 columns and W4A16 with 3..32 tokens.  The
 // same arithmetic as i4w_gemm (i4w_gemm.hpp):
 //
 //   out[r, c] = sum_g  sw[r,g] * sx[g,c] * P_g[r,c]
@@ -25,19 +25,24 @@
 // dwords (v_permlane16_swap, then v_permlane32_swap) gives lane group h the
 // dwords of k = 32 q + 8 h.
 //
-// RAWB (group-wise INT4 with 15 or 16 columns): no transpose pre-pass.  B
-// [K, 8] bytes (16 nibbles per k row) is contiguous, so each wave copies the
-// 1 KB of every group it owns into LDS in k-row order at the start, and
-// gfx950's ds_read_b64_tr_b4 transposes it on the way out: within a 16-lane
-// group, result lane j gets nibble j of the 16 source lanes' 8-byte rows,
-// i.e. 16 consecutive k of one column (nibble j of a row is column j ^ 1: the
-// even column sits in the high nibble), so lane l's X row is column
+// RAWB (group-wise INT4 with 5..32 columns): no transpose pre-pass.  Each
+// wave copies the groups of B it owns into LDS at the start, as rows of 8
+// bytes (16 nibbles) in k-row order, one 1 KB block per group and 16 columns,
+// and gfx950's ds_read_b64_tr_b4 transposes them on the way out: within a
+// 16-lane group, result lane j gets nibble j of the 16 source lanes' 8-byte
+// rows, i.e. 16 consecutive k of one column (nibble j of a row is column j ^
+// 1: the even column sits in the high nibble), so lane l's X row is column
 // (l % 16) ^ 1.  Two such reads give lane group h the k = 32 h .. 32 h + 31 of
 // the group, and step q uses k = 32 h + 8 q .. + 7 -- the order in which the
 // weights' 16-byte group slices arrive, so with raw B the weights need no
 // lane-group transpose either.  B nibbles come out with the even k in the
 // low nibble (unpack8<true>), and are unpacked with the same exact
 // (q - z) 2^-9 arithmetic; the extra 2^-9 is returned in the fold.
+// RAWB 1: 15 or 16 columns, B rows of 8 bytes, 16-byte aligned: 1 KB of a
+// group is contiguous.  RAWB 2: any other row length (2..16 bytes) and any
+// alignment: one 8-byte load at byte alignment per row and fragment.  Where a
+// row has fewer bytes, the rest of its 8 are the next row's; they land in
+// columns that have no output.
 #pragma once
 
 #include "i4w_gemm.hpp"
@@ -55,9 +60,9 @@ struct SCfg {
     // partial sums of the KS waves, then the workgroup's scales and zero
     // points ([ROWS][G] fp16 each) and sx ([G][16 XF] fp32)
     static constexpr int RED_BYTES = KS * XF * WF * 4 * 64 * 4;
-    static constexpr int lds_bytes(int G, bool xs, bool rawb = false) {
+    static constexpr int lds_bytes(int G, bool xs, int rawb = 0) {
         return RED_BYTES + 2 * ((ROWS * G * 2 + 15) & ~15) + (xs ? G * 16 * XF * 4 : 0) +
-               (rawb ? ((G * 16 * 2 + 15) & ~15) + G * 1024 : 0);
+               (rawb ? G * 16 * XF * 2 + G * 1024 * XF : 0) + (rawb == 2 ? 4 * KS : 0);
     }
 };
 
@@ -80,10 +85,11 @@ __device__ __forceinline__ u32x2 lds_read_tr4(unsigned a) {
     return u32x2{(unsigned)v[0], (unsigned)v[1]};
 }
 
-template <class SC, bool XS, int OUT, bool RAWB = false>
+template <class SC, bool XS, int OUT, int RAWB = 0>
 __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
     constexpr int WF = SC::WF, XF = SC::XF, NG = SC::NG, D = SC::D, ROWS = SC::ROWS;
-    static_assert(!RAWB || (XS && XF == 1 && OUT == 0), "raw B: group-wise INT4, 16 columns");
+    static_assert(XS == (RAWB != 0) && (!XS || OUT == 0), "group-wise INT4 reads B in place");
+    static_assert(RAWB != 1 || XF == 1, "rows of 8 bytes: one fragment of 16 columns");
     extern __shared__ __attribute__((aligned(16))) float red[];
 
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 4, l16 = lane & 15;
@@ -95,8 +101,9 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
     uint16_t* lds_s = reinterpret_cast<uint16_t*>(reinterpret_cast<unsigned char*>(red) + SC::RED_BYTES);
     uint16_t* lds_z = lds_s + ((ROWS * G + 7) & ~7);
     float* lds_xs = reinterpret_cast<float*>(lds_z + ((ROWS * G + 7) & ~7));
-    uint16_t* lds_zb = reinterpret_cast<uint16_t*>(lds_xs + (XS ? G * 16 * XF : 0));  // RAWB: zB [G][16]
-    unsigned char* lds_b = reinterpret_cast<unsigned char*>(lds_zb) + ((G * 16 * 2 + 15) & ~15);  // RAWB: B
+    uint16_t* lds_zb = reinterpret_cast<uint16_t*>(lds_xs + (XS ? G * 16 * XF : 0));  // RAWB: zB [G][16 XF]
+    unsigned char* lds_b = reinterpret_cast<unsigned char*>(lds_zb) + G * 16 * XF * 2;  // RAWB: B [G][XF][1 KB]
+    unsigned* lds_far = reinterpret_cast<unsigned*>(lds_b + G * 1024 * XF);              // RAWB 2: [KS]
 
     const uint8_t* wrow[WF];
 #pragma unroll
@@ -113,12 +120,23 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
     // issued after them, where a read of LDS behind an LDS DMA waits for every
     // outstanding load, the weight stream included.  (A wave without groups
     // loads group G - 1, see the staging below.)
-    u32x4 braw[RAWB ? NG : 1];
+    u32x4 braw[RAWB ? NG * XF : 1];
+    const int b_last = RAWB == 2 ? K * p.ldb - 8 : 0;  // the last 8 bytes of B
     if constexpr (RAWB) {
 #pragma unroll
         for (int j = 0; j < NG; ++j) {
             const int g = max(0, min(g0 + j, g1 - 1));
-            braw[j] = *reinterpret_cast<const u32x4*>(p.B + (int64_t)g * 1024 + 16 * lane);
+            if constexpr (RAWB == 1) {
+                braw[j] = *reinterpret_cast<const u32x4*>(p.B + (int64_t)g * 1024 + 16 * lane);
+            } else {
+#pragma unroll
+                for (int x = 0; x < XF; ++x) {
+                    const int o = (128 * g + 2 * lane) * p.ldb + 8 * x;
+                    const u32x2u a = *reinterpret_cast<const u32x2u*>(p.B + min(o, b_last));
+                    const u32x2u b = *reinterpret_cast<const u32x2u*>(p.B + min(o + p.ldb, b_last));
+                    braw[j * XF + x] = u32x4{a.x, a.y, b.x, b.y};
+                }
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -156,7 +174,6 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
     constexpr int SPL = (ROWS * NG + 63) / 64;                 // weight constants per lane
     constexpr int XPL = XS ? (16 * XF * NG + 63) / 64 : 1;     // sx entries per lane
     uint16_t sv[SPL], zv[SPL], sbv[XPL] = {}, zbv[XPL] = {};
-    float xv[XPL] = {};
 #pragma unroll
     for (int i = 0; i < SPL; ++i) {
         const int e = min(lane + 64 * i, ROWS * NG - 1), row = e / NG, gj = min(e % NG, ngs - 1);
@@ -168,15 +185,11 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
 #pragma unroll
         for (int i = 0; i < XPL; ++i) {
             const int e = min(lane + 64 * i, 16 * XF * NG - 1), gj = min(e / (16 * XF), ngs - 1), c = e % (16 * XF);
-            if constexpr (RAWB) {
-                // sB and zB (converted, and zeroed past N, at the store: a use
-                // here would wait for the load before the stream goes out)
-                const int64_t si = (int64_t)(gs0 + gj) * p.N + min(c, p.N - 1);
-                sbv[i] = p.bscale[si];
-                zbv[i] = p.bzero[si];
-            } else {
-                xv[i] = p.xs[(int64_t)(gs0 + gj) * p.ldxs + c];
-            }
+            // sB and zB (converted, and zeroed past N, at the store: a use
+            // here would wait for the load before the stream goes out)
+            const int64_t si = (int64_t)(gs0 + gj) * p.N + min(c, p.N - 1);
+            sbv[i] = p.bscale[si];
+            zbv[i] = p.bzero[si];
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // (keep the order: staging loads, then the stream)
@@ -192,9 +205,30 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
         // alternate 128-byte halves of the banks (two passes, the minimum for
         // 512 bytes)
 #pragma unroll
-        for (int j = 0; j < NG; ++j)
-            if (j < ngs)
-                *reinterpret_cast<u32x4*>(lds_b + (gs0 + j) * 1024 + (lane ^ (((lane >> 4) & 1) << 3)) * 16) = braw[j];
+        for (int j = 0; j < NG * XF; ++j) {
+            const int gj = j / XF, x = j % XF;
+            if (gj >= ngs) continue;
+            u32x4 v = braw[j];
+            if constexpr (RAWB == 2) {
+                // (a load moved back to stay inside B has its row's bytes higher up)
+                const int o = (128 * (gs0 + gj) + 2 * lane) * p.ldb + 8 * x - b_last;
+                const uint64_t a = ((uint64_t)v.y << 32 | v.x) >> (8 * max(0, o));
+                const uint64_t b = ((uint64_t)v.w << 32 | v.z) >> (8 * max(0, o + p.ldb));
+                v = u32x4{(unsigned)a, (unsigned)(a >> 32), (unsigned)b, (unsigned)(b >> 32)};
+            }
+            *reinterpret_cast<u32x4*>(lds_b + ((gs0 + gj) * XF + x) * 1024 + (lane ^ (((lane >> 4) & 1) << 3)) * 16) =
+                v;
+        }
+    }
+    if constexpr (RAWB == 2) {
+        // (see the recomputation at the end)
+        bool far = false;
+#pragma unroll
+        for (int i = 0; i < SPL; ++i) far |= !(fabsf(h2f(zv[i])) <= 256.0f);
+#pragma unroll
+        for (int i = 0; i < XPL; ++i) far |= !(fabsf(h2f(zbv[i])) <= 256.0f);
+        const unsigned any = __any(far) ? 1u : 0u;
+        if (lane == 0) lds_far[wave] = any;
     }
 #pragma unroll
     for (int i = 0; i < SPL; ++i) {
@@ -210,13 +244,9 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
             const int e = lane + 64 * i, gj = e / (16 * XF), c = e % (16 * XF);
             if (e < 16 * XF * NG && gj < ngs) {
                 const int d = (gs0 + gj) * 16 * XF + c;
-                if constexpr (RAWB) {
-                    const bool in = c < p.N;
-                    lds_xs[d] = in ? h2f(sbv[i]) : 0.0f;
-                    lds_zb[d] = in ? zbv[i] : (uint16_t)0;
-                } else {
-                    lds_xs[d] = xv[i];
-                }
+                const bool in = c < p.N;
+                lds_xs[d] = in ? h2f(sbv[i]) : 0.0f;
+                lds_zb[d] = in ? zbv[i] : (uint16_t)0;
             }
         }
     }
@@ -243,8 +273,8 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
         struct Cst {
             uint16_t z[WF], s[WF];
             f32x4 sx[XS ? XF : 1];
-            uint16_t zb;
-            u32x4 bq;
+            uint16_t zb[XF];
+            u32x4 bq[XF];
         };
         auto load_cst = [&](int j) {
             Cst c{};
@@ -258,20 +288,23 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
 #pragma unroll
                 for (int x = 0; x < XF; ++x) {
                     const f32x4 v = *reinterpret_cast<const f32x4*>(lds_xs + g * 16 * XF + 16 * x + 4 * h);
-                    // raw B: accumulator row 4 h + e is column 4 h + (e ^ 1)
-                    c.sx[x] = RAWB ? f32x4{v[1], v[0], v[3], v[2]} : v;
+                    // accumulator row 4 h + e is column 4 h + (e ^ 1)
+                    c.sx[x] = f32x4{v[1], v[0], v[3], v[2]};
                 }
             }
             if constexpr (RAWB) {
-                c.zb = lds_zb[g * 16 + (l16 ^ 1)];
                 // column l16 ^ 1, rows k = 128 g + 32 h + 8 q .. + 7 in word q
                 // (two transposing reads of 16 rows; odd blocks h have their
                 // halves swapped, see the copy above)
-                const unsigned gb = lds_b_addr + g * 1024;
                 const int sw = (h & 1) << 4;
-                const u32x2 lo = lds_read_tr4(gb + 8 * ((32 * h + l16) ^ sw));
-                const u32x2 hi = lds_read_tr4(gb + 8 * ((32 * h + 16 + l16) ^ sw));
-                c.bq = u32x4{lo.x, lo.y, hi.x, hi.y};
+#pragma unroll
+                for (int x = 0; x < XF; ++x) {
+                    c.zb[x] = lds_zb[(g * XF + x) * 16 + (l16 ^ 1)];
+                    const unsigned gb = lds_b_addr + (g * XF + x) * 1024;
+                    const u32x2 lo = lds_read_tr4(gb + 8 * ((32 * h + l16) ^ sw));
+                    const u32x2 hi = lds_read_tr4(gb + 8 * ((32 * h + 16 + l16) ^ sw));
+                    c.bq[x] = u32x4{lo.x, lo.y, hi.x, hi.y};
+                }
             }
             return c;
         };
@@ -287,16 +320,23 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
                 const _Float16 nz = (_Float16)(-rintf(h2f(c.z[f])) * (1.0f / 512.0f));
                 zz[f] = f16x2{nz, nz};
             }
-            f16x2 zzb;
+            f16x2 zzb[XF];
             if constexpr (RAWB) {
-                const _Float16 nzb = (_Float16)(-rintf(h2f(c.zb)) * (1.0f / 512.0f));
-                zzb = f16x2{nzb, nzb};
+#pragma unroll
+                for (int x = 0; x < XF; ++x) {
+                    const _Float16 nzb = (_Float16)(-rintf(h2f(c.zb[x])) * (1.0f / 512.0f));
+                    zzb[x] = f16x2{nzb, nzb};
+                }
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 f16x8 xq[XF];
                 if constexpr (RAWB) {
-                    xq[0] = unpack8<true>(q == 0 ? c.bq.x : q == 1 ? c.bq.y : q == 2 ? c.bq.z : c.bq.w, zzb);
+#pragma unroll
+                    for (int x = 0; x < XF; ++x) {
+                        const u32x4& b = c.bq[x];
+                        xq[x] = unpack8<true>(q == 0 ? b.x : q == 1 ? b.y : q == 2 ? b.z : b.w, zzb[x]);
+                    }
                 } else {
 #pragma unroll
                     for (int x = 0; x < XF; ++x) xq[x] = s.x[x][q];
@@ -365,6 +405,29 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
                 }
     }
 
+    if constexpr (RAWB == 2) {
+        // up to 8 columns: a zero point past +-256 (then a group's sum may pass
+        // 2^24, and past 2048 q - z itself is not exact in fp16) has the
+        // workgroup's outputs computed again in integers
+        unsigned far = 0;
+#pragma unroll
+        for (int w = 0; w < SC::KS; ++w) far |= lds_far[w];
+        if (p.N <= 8 && far != 0) {
+            for (int f = 0; f < WF; ++f)
+                for (int e = 0; e < 4; ++e) {
+                    const int r = r0 + 16 * f + l16, c = 4 * h + (e ^ 1);
+                    if (r >= R || c >= p.N) continue;
+                    const float v = int4_exact_output(p.W, p.wscale, p.wzero, p.B, p.bscale, p.bzero, r, c, p.N, K, G,
+                                                      p.ldb);
+#pragma unroll
+                    for (int ff = 0; ff < WF; ++ff)
+#pragma unroll
+                        for (int ee = 0; ee < 4; ++ee)
+                            if (ff == f && ee == e) acc[0][ff][ee] = v;
+                }
+        }
+    }
+
     // ---- epilogue: lane holds weight row r0 + 16 f + l16 and X rows 16 x + 4 h .. + 3 ----
     if constexpr (OUT == 1) {
         // every old value of Y first (clamped addresses), then every store: a
@@ -403,16 +466,15 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
         for (int x = 0; x < XF; ++x) {
             const int c = 16 * x + 4 * h;
             if constexpr (OUT == 0) {
-                // (raw B: accumulator entry e is column c + (e ^ 1))
-                constexpr int SW = RAWB ? 1 : 0;
+                // (accumulator entry e is column c + (e ^ 1))
                 uint16_t* dst = p.out + (int64_t)r * p.C + c;
                 if (c + 3 < p.C && (p.C & 3) == 0) {
-                    *reinterpret_cast<u32x2*>(dst) = u32x2{pack2h(acc[x][f][0 ^ SW], acc[x][f][1 ^ SW]),
-                                                           pack2h(acc[x][f][2 ^ SW], acc[x][f][3 ^ SW])};
+                    *reinterpret_cast<u32x2*>(dst) = u32x2{pack2h(acc[x][f][1], acc[x][f][0]),
+                                                           pack2h(acc[x][f][3], acc[x][f][2])};
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (c + e < p.C) dst[e] = f2h(acc[x][f][e ^ SW]);
+                        if (c + e < p.C) dst[e] = f2h(acc[x][f][e ^ 1]);
                 }
             } else {
 #pragma unroll

@@ -560,6 +560,14 @@ clove_status_t launch_w4a16_swiglu(const W4A16Args& a, hipStream_t stream) {
     const int G = cdiv(a.K, 128);
     const int nch = cdiv(a.K, 32);
     const int tv = a.T <= 1 ? 1 : (a.T <= 2 ? 2 : 4);
+    clove_status_t st2;
+    // three or four tokens on larger weights: the MFMA kernel (cold, us per
+    // call, GEMV against MFMA: 2 x 6784 x 1152 T = 3 10.5 -> 7.6, 2 x 10880 x
+    // 2560 T = 3 23.4 -> 14.0, 2 x 6528 x 2560 T = 4 16.3 -> 11.1; 2 x 2944 x
+    // 1536, 8.6 Mi weights, stays: 6.2 against 7.9)
+    if (a.T >= 3 && a.T <= 4 && (int64_t)2 * a.O * a.K >= ((int64_t)12 << 20) &&
+        try_i4w_w4a16_swiglu(a, dev.num_cus, stream, &st2))
+        return st2;
     if (a.T <= 4 && gemv_lds_bytes(tv, nch) <= kMaxGemvLds) {
         GemvParams p{a.X, a.W, a.scale, a.zero, a.Y, a.T, a.O, a.K, G, nch, 1.0f, 0.0f};
         const bool aligned = aligned16(a.W) && (a.K % 32 == 0);
@@ -567,7 +575,6 @@ clove_status_t launch_w4a16_swiglu(const W4A16Args& a, hipStream_t stream) {
         if (tv == 2) return run_gemv_swiglu<2>(p, aligned, dev.num_cus, stream);
         return run_gemv_swiglu<4>(p, aligned, dev.num_cus, stream);
     }
-    clove_status_t st2;
     if (try_i4w_w4a16_swiglu(a, dev.num_cus, stream, &st2)) return st2;
     // other shapes: gate into H, up into a library buffer, SwiGLU in place
     void* ubuf = nullptr;
@@ -594,7 +601,7 @@ clove_status_t launch_w4a16(const W4A16Args& a, hipStream_t stream) {
     const int nch = cdiv(a.K, 32);
     const int tv = a.T <= 1 ? 1 : (a.T <= 2 ? 2 : 4);
     if (a.K > 0 && a.T >= 3 && a.T <= 4) {
-        // (large weights: the streaming kernel, see try_i4w_w4a16)
+        // (the streaming kernel, see try_i4w_w4a16)
         clove_status_t st2;
         if (try_i4w_w4a16(a, dev.num_cus, stream, &st2)) return st2;
     }

@@ -183,6 +183,53 @@ def test_groupwise_stream_path_pow2_bit_exact():
     assert np.array_equal(f16bits(C), f16bits(ref.astype(np.float16)))
 
 
+# group-wise, 3..32 columns, K % 128 == 0: B read in place at any row length
+# (2..16 bytes) and alignment.  One and two column fragments, full and ragged,
+# one group, every K-slice count (G = 1, 17, 30, 44, 52, 88), one to three
+# weight fragments; the loads of the last rows are moved back inside B.
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(33, 3, 128), (70, 4, 2176), (9000, 7, 2048), (300, 8, 6656), (20, 9, 11264),
+                                   (11000, 13, 4096), (100, 16, 1024), (50, 17, 128), (8200, 18, 2176), (130, 25, 3840),
+                                   (70, 31, 5632), (40, 32, 5632)])
+def test_groupwise_raw_b_bit_exact(M, N, K, off):
+    import torch
+    A_q, sA, zA, B_q, sB, zB = make_case(M, N, K, "rawb", pow2=True, small=True)
+    buf = torch.full((off + B_q.size,), 0xFF, dtype=torch.uint8, device="cuda")
+    buf[off:] = to_dev(B_q).reshape(-1)
+    C = empty_f16(M, N, fill=float("nan"))
+    _cg().gemm_int4_ex(to_dev(A_q), to_dev(sA), to_dev(zA), buf[off:].view(B_q.shape), to_dev(sB), to_dev(zB), C, M, N, K, 0)
+    torch.cuda.synchronize()
+    rows = np.arange(M) if M <= 512 else np.unique(np.concatenate([np.arange(64), np.arange(M - 64, M)]))
+    _, ref, _ = oracle.gemm_int4_groupwise(A_q[rows], sA[rows], zA[rows], B_q, sB, zB, len(rows), N, K)
+    assert np.array_equal(f16bits(to_host(C)[rows]), f16bits(ref.astype(np.float16)))
+
+
+# up to 8 columns any zero point is exact: sums past 2^24 (|z| > 256) and
+# q - z past fp16's integers (|z| > 2048) are computed again in integers
+@pytest.mark.parametrize("z", [256.0, 257.0, -300.0, 2051.0, -7000.0])
+@pytest.mark.parametrize("N,col", [(3, 1), (8, 7)])
+def test_groupwise_raw_b_far_zero_points(N, col, z):
+    M, K = 37, 512
+    A_q, sA, zA, B_q, sB, zB = make_case(M, N, K, "far")
+    zA[5, 2] = z
+    zB[3, col] = -z
+    zA[M - 1, 0] = z
+    # every scale one power of two: the fold's products are exact, so each
+    # result is one rounding per group of an exact integer sum
+    sA[:] = np.float16(2.0 ** -8)
+    sB[:] = np.float16(2.0 ** -8)
+    if abs(z) > 1024:
+        sA[:] = np.float16(2.0 ** -12)
+        sB[:] = np.float16(2.0 ** -12)
+    C = run_int4(A_q, sA, zA, B_q, sB, zB, M, N, K)
+    P = partials_int64(A_q, zA, B_q, zB, np.arange(M), N, K)  # [M, N, G]
+    acc = np.zeros((M, N), np.float32)
+    s = np.float32(sA[0, 0]) * np.float32(sB[0, 0])
+    for g in range(K // 128):
+        acc = (np.float64(s) * np.float32(P[:, :, g]).astype(np.float64) + acc).astype(np.float32)
+    assert np.array_equal(f16bits(C), f16bits(acc.astype(np.float16)))
+
+
 # group-wise with N >= 64 and K % 256 == 0: the int8-MFMA kernel (i4i4_gemm)
 # after the Bt pre-pass.  Zero points at both ends of its exact range
 # [-112, 127] (q - z spans [-127, 127]) with power-of-two scales: every step
