@@ -9,16 +9,21 @@ namespace {
 using namespace sk;
 
 // (I8, BM, BN, WM, WN, stages)
-using F16M32 = Cfg<false, 32, 128, 1, 4, 5>;
+// (three stages: two workgroups fit a CU and the first stage waits behind a
+// smaller burst, which measured at least as fast as five on every shape with
+// M <= 32: 12 x 1344 x 2816 13.4 -> 9.3 us, 7 x 8057 x 1015 13.0 -> 11.5,
+// 25 x 8640 x 11904 36.6 -> 37.2)
+using F16M32 = Cfg<false, 32, 128, 1, 4, 3>;
 using F16M128 = Cfg<false, 128, 64, 4, 1, 4>;
 // mid-size shapes (M > 256) whose 256x256 tile grid would leave CUs idle:
-// 128x128 tiles (waves of 64x64), or 64x64 tiles when even those are too few
+// 128x128 tiles (waves of 64x64)
 // (hot launches: 2048^3 25 us with 128x128 against 45 us on the generic
-// register-staged kernel; 1024^3 8 us with 64x64 against 13 us with 128x128
-// and 21 us generic; 512x4096x4096 29 us with 128x128 in two K splits
+// register-staged kernel; 512x4096x4096 29 us with 128x128 in two K splits
 // against 33 us with 128x64)
 using F16T128 = Cfg<false, 128, 128, 2, 2, 3>;
-using F16T64 = Cfg<false, 64, 64, 2, 2, 6>;
+// few tiles: 64x64, 64 KB of LDS, so that two workgroups share a CU (505 x 2304
+// x 1088 14.6 -> 10.5 us against six stages; see pick_f16_tile)
+using F16T64 = Cfg<false, 64, 64, 2, 2, 4>;
 // the same tile one stage ahead for K <= 512: every workgroup's first stage
 // then waits behind a smaller burst of the whole grid's prologue loads (512^3:
 // 5.5 -> 4.7 us; from K = 1024 the six stages are ahead, 1024^3 8.7 against
@@ -34,30 +39,47 @@ using F16T64S2 = Cfg<false, 64, 64, 2, 2, 2>;
 // only ties or loses: 512 x 1024 x 512 5.27 -> 5.21, 1024 x 1024 x 512 5.81
 // -> 7.13)
 using F16K32 = Cfg<false, 32, 32, 1, 1, 3, 1, 4>;
-using I8M32 = Cfg<true, 32, 128, 1, 4, 5>;
+// up to 32 rows on moderate weights: 32x64 tiles, two k slices, 64 KB of LDS
+using F16N64 = Cfg<false, 32, 64, 1, 2, 4, 1, 2>;
+using I8M32 = Cfg<true, 32, 128, 1, 4, 3>;
+using I8T64 = Cfg<true, 64, 64, 2, 2, 4>;
+using I8W128 = Cfg<true, 64, 128, 2, 2, 3>;  // 72 KB LDS: two workgroups per CU
 using I8M128 = Cfg<true, 128, 64, 4, 1, 4>;
 using I8T128 = Cfg<true, 128, 128, 2, 2, 3>;
 
+// K tiles per split: split K until about one workgroup per CU, not with k
+// slices.  128-row tiles keep two K tiles per split and are not split for
+// short K (<= 16 K tiles), where the publish / count / reload tail costs more
+// than the shorter stream saves; the smaller tiles, whose tail is shorter,
+// keep four at any K (INT8 9 x 5633 x 2048 17.1 -> 12.0 us, 10 x 1228 x 1536
+// 12.1 -> 8.9; two a split measured slower on most), but FP16 32x128 tiles
+// split only past 15 (7 x 8057 x 1015 13.0 -> 11.5; 18 x 10496 x 896 7.9 ->
+// 8.9 in three splits).
+template <class CF>
+int tiles_per_split(int M, int N, int K, int batch, int cus) {
+    const int tiles = cdiv(M, CF::BM) * cdiv(N, CF::BN) * batch;
+    const int nk = cdiv(K, CF::BK);
+    int ns = tiles >= cus ? 1 : cus / tiles;
+    ns = max(1, min(ns, nk / (CF::BM == 128 ? 2 : 4)));
+    if ((CF::BM == 128 && nk <= 16) || CF::KW > 2) ns = 1;
+    if (!CF::I8 && CF::BM == 32 && nk <= 15) ns = 1;
+    return cdiv(nk, ns);
+}
+
 template <class CF, int OUT, bool ZP = false, Feed FEED = kWhole>
-clove_status_t run(Args a, int batch, int cus, hipStream_t stream) {
+clove_status_t run(Args a, int batch, int cus, hipStream_t stream, int kt_per = 0) {
     a.tiles_m = cdiv(a.M, CF::BM);
     a.tiles_n = cdiv(a.N, CF::BN);
     a.batch = batch;
     const int tiles = a.tiles_m * a.tiles_n * batch;
     const int nk = cdiv(a.K, CF::BK);
-    // split K (whole K tiles, at least two per split) until about one
-    // workgroup per CU; not for short K (<= 16 K tiles), where the split's
-    // publish / count / reload tail costs more than the shorter stream saves
-    // (512^3: 8.4 us with 4 splits, 7.2 us with none, measured)
-    int ns = tiles >= cus ? 1 : cus / tiles;
-    ns = max(1, min(ns, nk / 2));
-    if (nk <= 16 || CF::KW > 1) ns = 1;
-    const int kt_per = cdiv(nk, ns);
+    if (kt_per == 0) kt_per = tiles_per_split<CF>(a.M, a.N, a.K, batch, cus);
     a.kps = kt_per * CF::BK;
     a.nsplit = cdiv(nk, kt_per);
     if (a.nsplit > 1) {
         Scratch s;
-        const size_t bytes = (size_t)tiles * a.nsplit * CF::NT * CF::NB * CF::FM * CF::FN * 16 * sizeof(float);
+        const size_t bytes =
+            (size_t)tiles * a.nsplit * CF::NT * CF::NB * CF::FM * CF::FN * (16 / CF::KW) * sizeof(float);
         const clove_status_t st = acquire_scratch(stream, bytes, (size_t)tiles, &s);
         if (st != CLOVE_OK) return st;
         a.part = s.partials;
@@ -76,21 +98,31 @@ bool fits31(int64_t bytes) { return bytes < ((int64_t)1 << 31); }
 // The FP16 tile shapes, chosen by shape alone (so that the fused SwiGLU below
 // picks the same tiles, and with them the same split plan, as the two GEMMs
 // it replaces).
-enum class F16Tile { kM32, kM128, kT128, kT64, kK32 };
+enum class F16Tile { kM32, kN64, kM128, kT128, kT64, kK32 };
 
 F16Tile pick_f16_tile(int batch, int M, int N, int K, int cus) {
-    const bool short_k = K <= 16 * F16M128::BK;  // no split K (see run)
+    const int nk = cdiv(K, F16T64::BK);
+    const bool short_k = nk <= 16;
     const bool long_k = K >= 4096;
-    if (short_k && (int64_t)cdiv(M, F16K32::BM) * cdiv(N, F16K32::BN) * batch <= cus) return F16Tile::kK32;
+    // (up to 24 K tiles: 25 x 4160 x 1152 8.7 -> 7.2 us, 55 x 3136 x 1280 9.8 ->
+    // 8.0 against 32x128; 9 x 7680 x 1856 only ties)
+    if (nk <= 24 && (int64_t)cdiv(M, F16K32::BM) * cdiv(N, F16K32::BN) * batch <= cus) return F16Tile::kK32;
+    // 64x64 tiles while the product is small, whatever its M: their time is
+    // about tiles x K tiles (cold, 120 shapes, us per call, against the tiles
+    // below: 94 x 1536 x 2752 15.4 -> 9.5, 547 x 640 x 5056 23.6 -> 15.3, 265 x
+    // 1344 x 4224 20.3 -> 15.5, 128 x 4096 x 4096 15.6 -> 13.9, 144 x 2624 x 4352
+    // 17.1 -> 16.1; past the line 166 x 2624 x 10368 29.1 -> 30.9, 128 x 4096 x
+    // 11008 30.8 -> 35.0, 559 x 4352 x 2688 29.3 -> 39.1).  Up to 32 rows half of
+    // such a tile is padding, and 32x128 takes over above 64 tiles (8 x 4096 x
+    // 4096 11.8 -> 10.8, but 10 x 8320 x 3584 13.7 -> 16.9).
+    const int64_t t64 = (int64_t)cdiv(M, F16T64::BM) * cdiv(N, F16T64::BN) * batch;
+    if (M <= 32) return t64 <= cus / 4 ? F16Tile::kN64 : F16Tile::kM32;
+    if (M <= 64 || (t64 <= 2 * cus && t64 * nk <= 33 * cus)) return F16Tile::kT64;
     // 128x128 tiles, split K when they are few: for M > 256 once they cover
     // half the CUs or K is long, for 128 < M <= 256 on long K and N >= 4096
     // (cold weights, against 64x64 tiles for M > 256 and 128x64 up to 256:
     // 11008x4096 at M = 192 44.3 against 64.2 us, 4096x11008 at M = 384 64.1
-    // against 108.6 us, 4096x4096 at M = 384 30.6 against 43.7 us, 2048x8192
-    // at M = 512 35.2 against 47.4 us; K = 2048 and N = 2048 stay as they
-    // were: 2048x2048 at M = 384 14.0 with 64x64 against 19.0, 2048x8192 at
-    // M = 160 24.0 with 128x64 against 26.0; 64x64 for short K with few tiles:
-    // 1024^3 8 us against 13)
+    // against 108.6 us, 2048x8192 at M = 512 35.2 against 47.4 us)
     if (M > 256) {
         const int64_t t128 = (int64_t)cdiv(M, 128) * cdiv(N, 128) * batch;
         return (t128 >= cus / 2 || long_k) ? F16Tile::kT128 : F16Tile::kT64;
@@ -102,13 +134,10 @@ F16Tile pick_f16_tile(int batch, int M, int N, int K, int cus) {
     // 80 x 11008 x 4096 30.8 -> 27.7, 128 x 14336 x 4096 39.0 -> 34.1; not at
     // N = 8192, K = 2048 or N = 4096, K = 11008, where 128x64 stays ahead)
     if (M > 64 && M <= 128 && long_k && N >= 10240) return F16Tile::kT128;
-    // 32-row tiles up to M = 64 (cold 4096 x 4096 weights: M = 40 / 48 / 64 at
-    // 13.6 / 14.1 / 14.5 us against 14.9 / 15.3 / 15.5 with 64-row tiles), and
-    // for short K with few 128-row tiles, where they make 4x the workgroups
-    // without a split (512^3: 6.1 us against 7.2, measured)
+    // short K with few 128-row tiles: 32-row tiles make 4x the workgroups
+    // without a split
     const bool few = (int64_t)cdiv(M, F16M128::BM) * cdiv(N, F16M128::BN) * batch < cus / 2;
-    if (M <= 64 || (short_k && few)) return F16Tile::kM32;
-    return F16Tile::kM128;
+    return short_k && few ? F16Tile::kM32 : F16Tile::kM128;
 }
 
 bool f16_domain(const void* A, const void* B, const void* C, int M, int N, int K) {
@@ -130,9 +159,10 @@ bool ua_domain(int M, int N, int K, int es) {
 // two-B-operand (gate, up) counterparts of the tiles above; fewer stages
 // where both B tiles would not fit the LDS
 using SwM32 = Cfg<false, 32, 128, 1, 4, 4, 2>;
+using SwN64 = Cfg<false, 32, 64, 1, 2, 3, 2, 2>;
 using SwM128 = Cfg<false, 128, 64, 4, 1, 4, 2>;
 using SwT128 = Cfg<false, 128, 128, 2, 2, 3, 2>;
-using SwT64 = Cfg<false, 64, 64, 2, 2, 6, 2>;
+using SwT64 = Cfg<false, 64, 64, 2, 2, 4, 2>;
 using SwK32 = Cfg<false, 32, 32, 1, 1, 3, 2, 4>;
 
 }  // namespace
@@ -161,6 +191,7 @@ bool try_skinny_fp16(const uint16_t* A, const uint16_t* B, uint16_t* C, int batc
     };
     switch (pick_f16_tile(batch, M, N, K, cus)) {
         case F16Tile::kM32: *status = go(F16M32{}); break;
+        case F16Tile::kN64: *status = go(F16N64{}); break;
         case F16Tile::kM128: *status = go(F16M128{}); break;
         case F16Tile::kT128: *status = go(F16T128{}); break;
         case F16Tile::kT64:
@@ -188,9 +219,18 @@ bool try_skinny_swiglu(const uint16_t* X, const uint16_t* W_gate, const uint16_t
     a.sC = (int64_t)T * inter;
     switch (pick_f16_tile(1, T, inter, hidden, cus)) {
         case F16Tile::kM32: *status = run<SwM32, kF16SwiGLU>(a, 1, cus, stream); break;
+        case F16Tile::kN64: *status = run<SwN64, kF16SwiGLU>(a, 1, cus, stream); break;
         case F16Tile::kM128: *status = run<SwM128, kF16SwiGLU>(a, 1, cus, stream); break;
         case F16Tile::kT128: *status = run<SwT128, kF16SwiGLU>(a, 1, cus, stream); break;
-        case F16Tile::kT64: *status = run<SwT64, kF16SwiGLU>(a, 1, cus, stream); break;
+        case F16Tile::kT64: {
+            // (96 KB of LDS, one workgroup a CU: past one round of them 128x64 tiles
+            // under the same split, 219 x 4224 x 1280 25.5 -> 17.7 us)
+            const int kt_per = tiles_per_split<F16T64>(T, inter, hidden, 1, cus);
+            *status = T > 64 && T <= 256 && cdiv(T, 64) * cdiv(inter, 64) > cus
+                          ? run<SwM128, kF16SwiGLU>(a, 1, cus, stream, kt_per)
+                          : run<SwT64, kF16SwiGLU>(a, 1, cus, stream, kt_per);
+            break;
+        }
         case F16Tile::kK32: *status = run<SwK32, kF16SwiGLU>(a, 1, cus, stream); break;
     }
     return true;
@@ -223,21 +263,39 @@ bool try_skinny_int8(const Int8Args& q, int cus, hipStream_t stream, clove_statu
             if (!al) return run<CF, OUT, true, kUnaligned>(a, 1, cus, stream);
             return zp ? run<CF, OUT, true>(a, 1, cus, stream) : run<CF, OUT>(a, 1, cus, stream);
         };
-        // 32-row tiles up to M = 64, and up to 128 unless the weight is large
-        // (cold: 4096 x 4096 at M = 64 / 128 10.8 / 13.8 us against 15.0 / 15.3
-        // with 64- and 128-row tiles, 8192 x 2048 at M = 128 12.0 against 14.7;
-        // 11008 x 4096 at M = 128 24.2 with 128-row tiles against 30.6), from
-        // M = 160 the 128-row tiles, and for short K as for FP16.  Up to
-        // M = 2048 this kernel is ahead of the register-staged MFMA GEMM
-        // (4096 x 4096 at M = 768 / 2048 43.4 / 79.4 us against 66.8 / 156.1,
-        // 11008 x 4096 at M = 768 95.3 against 209.2); at M = 4096 it is not.
-        const bool short_k = q.K <= 16 * I8M128::BK &&
-                             (int64_t)cdiv(q.M, I8M128::BM) * cdiv(q.N, I8M128::BN) < cus / 2;
-        const bool large_w = (int64_t)q.N * q.K > ((int64_t)32 << 20);
-        if (q.M <= 64 || (q.M <= 128 && !large_w) || short_k) return go(I8M32{});
-        // 128x128 tiles for M <= 128 on wide weights, as for FP16 (cold, 128 x
-        // 11008 x 4096 23.7 -> 20.5 us; 128 x 4096 x 11008 stays on 128x64)
-        if (q.M <= 128 && q.N >= 10240 && q.K >= 4096) return go(I8T128{});
+        // (us per call, cold, 130 shapes with and without zero points, aligned and
+        // not; "was": 32x128 in five stages up to M = 64, or 128 on weights up
+        // to 32 Mi, else 128x64)
+        const int64_t t64 = (int64_t)cdiv(q.M, I8T64::BM) * cdiv(q.N, I8T64::BN);
+        const int64_t w64 = (int64_t)cdiv(q.M, I8W128::BM) * cdiv(q.N, I8W128::BN);
+        const int nk = cdiv(q.K, I8T64::BK);
+        if (q.M <= 32) return go(I8M32{});
+        // 64 rows: 64x128 tiles once 64x64 ones fill a quarter of the CUs over a
+        // longer K (39 x 13376 x 4736 28.8 -> 19.2, 62 x 4620 x 8512 28.7 -> 21.8),
+        // else 64x64 (34 x 6848 x 896 6.5 -> 5.3, 39 x 960 x 5376 12.4 -> 10.5)
+        if (q.M <= 64) return t64 > cus / 4 && nk > 16 ? go(I8W128{}) : go(I8T64{});
+        // small products, at any M: 64x64 (187 x 512 x 9728 19.8 -> 12.9, 509 x 512
+        // x 5376 16.9 -> 11.6, 128 x 4096 x 4096 11.2 -> 10.8, 613 x 2368 x 924 15.5
+        // -> 14.0; past the line 70 x 4224 x 4754 19.9 -> 23.7, 683 x 2432 x 3200
+        // 14.8 -> 18.2)
+        if (t64 <= 2 * cus && t64 * nk <= (q.M <= 128 ? 16 : 20) * cus) return go(I8T64{});
+        if (q.M <= 128) {
+            // 32-row tiles in one round on weights up to 32 Mi (past one round 82 x
+            // 10958 x 2634 36.1 -> 26.5 with 64x128), 128x128 on wide weights, as
+            // for FP16 (128 x 11008 x 4096 23.7 -> 20.5; 128 x 4096 x 11008 stays on
+            // 128x64)
+            const bool large_w = (int64_t)q.N * q.K > ((int64_t)32 << 20);
+            if (!large_w) return (int64_t)cdiv(q.M, I8M32::BM) * cdiv(q.N, I8M32::BN) <= cus ? go(I8M32{}) : go(I8W128{});
+            if (q.N >= 10240 && q.K >= 4096) return go(I8T128{});
+        }
+        // 64x128, two workgroups a CU, where that fills the chip (aligned: 134 x
+        // 9280 x 10368 98.9 -> 63.8, 577 x 4096 x 13952 120.8 -> 75.5, 986 x 2816 x
+        // 4224 43.2 -> 28.4, 1474 x 4480 x 8704 157.5 -> 103.6, 512 x 4096 x 4096
+        // 18.5 -> 17.6; with 135 tiles 1666 x 576 x 13440 39.3 -> 67.7; unaligned
+        // operands, whose K tiles go through registers, only tie).  Up to M = 2048
+        // this kernel is ahead of the register-staged MFMA GEMM; at M = 4096 it is
+        // not.
+        if (al && 4 * w64 >= 3 * cus) return go(I8W128{});
         return go(I8M128{});
     };
     switch (q.out) {

@@ -26,11 +26,12 @@
 // the CUs, with the shared publish / reduce (split order, deterministic;
 // int32 partials for INT8, so the integer accumulator stays exact).
 //
-// K slices (KW > 1, FP16 only, no split K): the small products (short K, a
-// 32x32 tile per CU or fewer) run 32x32 tiles whose four waves each take one
-// of every K tile's four k-steps; after the K loop every wave stores its sums
-// to LDS and each wave adds the four slices, in slice order, for a quarter of
-// the tile's output runs.
+// K slices (KW > 1, FP16 only): the small products (short K, a 32x32 tile per
+// CU or fewer) run 32x32 tiles whose four waves each take one of every K
+// tile's four k-steps; after the K loop every wave stores its sums to LDS and
+// each wave adds the four slices, in slice order, for a quarter of the tile's
+// output runs.  Up to 32 rows on moderate weights run 32x64 tiles with two
+// slices, which also split K over workgroups.
 //
 // Zero points (ZP, INT8): with
 //   sum (a - za)(b - zb) = sum ab - zb rowsum(A) - za colsum(B) + k za zb
@@ -103,7 +104,7 @@ struct Args {
 // KW > 1: KW waves share each wave tile and take disjoint slices of every K
 // tile's four k-steps, summed through LDS after the K loop (slice order, so
 // deterministic): KW times the workgroups of the same wave tiles for small
-// products (no split K)
+// products (split K only with KW = 2)
 template <bool I8_, int BM_, int BN_, int WM_, int WN_, int S_, int NB_ = 1, int KW_ = 1>
 struct Cfg {
     static constexpr bool I8 = I8_;
@@ -556,9 +557,9 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
                     }
     }
 
-    // ---- split-K (not with k slices: the host plans none) ----
-    if (CF::KW == 1 && p.nsplit > 1) {
-        constexpr int NC = NB * FN * FM * 4;
+    // ---- split-K (with k slices: of the runs a wave owns) ----
+    if (CF::KW < 4 && p.nsplit > 1) {
+        constexpr int NC = NB * FN * FM * NQ;
         f32x4 v[NC];
 #pragma unroll
         for (int b = 0; b < NB; ++b)
@@ -567,10 +568,12 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
 #pragma unroll
                 for (int j = 0; j < FM; ++j)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        v[((b * FN + i) * FM + j) * 4 + q] = bitcast<f32x4>(
+                    for (int q = 0; q < 4; ++q) {
+                        if (CF::KW > 1 && q / NQ != kw) continue;
+                        v[((b * FN + i) * FM + j) * NQ + q % NQ] = bitcast<f32x4>(
                             AccT4{acc[b][i][j][4 * q], acc[b][i][j][4 * q + 1], acc[b][i][j][4 * q + 2],
                                   acc[b][i][j][4 * q + 3]});
+                    }
         float* slabs = p.part + (size_t)tile * p.nsplit * NC * CF::NT * 4;
         splitk_publish<NC, CF::NT>(slabs + (size_t)split * NC * CF::NT * 4, tid, v);
         if (!splitk_arrive_is_last(p.counters + tile, (unsigned)p.nsplit, reinterpret_cast<int*>(smem)))
@@ -584,7 +587,8 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
                 for (int j = 0; j < FM; ++j)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        const AccT4 w = bitcast<AccT4>(v[((b * FN + i) * FM + j) * 4 + q]);
+                        if (CF::KW > 1 && q / NQ != kw) continue;
+                        const AccT4 w = bitcast<AccT4>(v[((b * FN + i) * FM + j) * NQ + q % NQ]);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) acc[b][i][j][4 * q + e] = w[e];
                     }

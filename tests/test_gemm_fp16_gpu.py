@@ -400,3 +400,19 @@ def test_unaligned_pointers_and_batches(batch, M, N, K, off):
     got = to_host(bufs[2])
     assert np.array_equal(got[off: off + ref.size].reshape(ref.shape), ref)
     assert (got[:off] == -7).all() and (got[off + ref.size:] == -7).all()
+
+
+# up to 32 rows on moderate weights: 32x64 tiles with two k slices, with and
+# without K splits, aligned, with ragged K and unaligned; past 32x128 tiles'
+# fifteen K tiles those split; 64x64 tiles under several K splits
+@pytest.mark.parametrize("M,N,K", [(32, 4096, 4096), (5, 1032, 2824), (9, 1001, 2050), (17, 72, 1600), (31, 3000, 1601),
+                                   (6, 6008, 1024), (20, 4168, 1000), (64, 3072, 4160), (94, 1536, 2752),
+                                   (265, 1344, 4224), (129, 190, 3535)])
+def test_small_product_tiles_bit_exact(M, N, K):
+    g = rng("small-tiles", M, N, K)
+    A = g.integers(-2, 3, (M, K)).astype(np.float16)
+    B = g.integers(-2, 3, (K, N)).astype(np.float16)
+    C0 = g.integers(-8, 9, (M, N)).astype(np.float16)
+    C = run_fp16(A, B, C0, alpha=1.0, beta=0.5)
+    exact = A.astype(np.float64) @ B.astype(np.float64) + 0.5 * C0.astype(np.float64)
+    assert np.array_equal(f16bits(C), f16bits(exact.astype(np.float16)))

@@ -260,3 +260,26 @@ def test_unaligned_and_ragged_k_bit_exact(M, N, K, za, zb):
     assert np.array_equal(run_acc32(A, B, za, zb)[rows], accref)
     assert np.array_equal(f16bits(to_host(C1)[rows]), f16bits(Cref1))
     assert np.array_equal(f16bits(to_host(C2)[rows]), f16bits(Cref2))
+
+
+# the 64x64 and 64x128 tiles: small products at any M, 33..64 rows on a longer
+# K, 65..128 rows past one round of 32-row tiles, and grids of 64x128 tiles
+# that fill the chip, each with and without zero points
+@pytest.mark.parametrize("za,zb", [(0, 0), (-9, 4)])
+@pytest.mark.parametrize("M,N,K", [(34, 688, 896), (40, 4160, 2304), (63, 4621, 2178), (100, 9216, 2048), (187, 512, 2064),
+                                   (520, 2752, 4096), (587, 400, 1152), (10, 1228, 1536)])
+def test_mid_tiles_bit_exact(M, N, K, za, zb):
+    g = rng("mid8", M, N, K, za, zb)
+    A = g.integers(-128, 128, (M, K)).astype(np.int8)
+    B = g.integers(-128, 128, (K, N)).astype(np.int8)
+    sa = g.uniform(0.001, 0.02, M).astype(np.float16)
+    sb = g.uniform(0.001, 0.02, N).astype(np.float16)
+    C = empty_f16(M, N)
+    _cg().gemm_int8_rowcol(to_dev(A), to_dev(B), to_dev(sa), to_dev(sb), C, M, N, K, za, zb)
+    _sync()
+    rows = np.unique(np.concatenate([[0, 31, min(64, M - 1), M - 1], g.integers(0, M, 12)]))
+    rows = rows[rows < M]
+    _, accref = oracle.gemm_int8(A[rows], B, np.float32(1), za, np.float32(1), zb)
+    Cref, _ = oracle.gemm_int8_rowcol(A[rows], B, sa[rows], sb, za, zb)
+    assert np.array_equal(run_acc32(A, B, za, zb)[rows], accref)
+    assert np.array_equal(f16bits(to_host(C)[rows]), f16bits(Cref))

@@ -255,6 +255,13 @@ def test_swiglu_fused_equals_gemms_then_swiglu(T, H, I):
     assert np.array_equal(f16bits(got), f16bits(to_host(ref)))
 
 
+# the same where the fused call takes other tiles than the GEMMs under their K
+# split (219 x 4224 x 1280), and k slices with a K split (20 x 1024 x 2048)
+@pytest.mark.parametrize("T,H,I", [(219, 1280, 4224), (143, 1152, 7936), (20, 2048, 1024), (35, 2688, 1536), (12, 1536, 4608)])
+def test_swiglu_fused_equals_gemms_small_tiles(T, H, I):
+    test_swiglu_fused_equals_gemms_then_swiglu(T, H, I)
+
+
 @pytest.mark.parametrize("T,H,I,offset", [(5, 60, 100, False), (3, 100, 30, False), (33, 200, 72, False),
                                           (2, 256, 128, True), (20, 128, 64, True)])
 def test_swiglu_fused_direct_fallback(T, H, I, offset):
