@@ -186,7 +186,7 @@ clove_status_t current_device_info(DeviceInfo* out) {
 }
 
 clove_status_t acquire_scratch(hipStream_t stream, size_t partial_bytes, size_t num_counters,
-                               Scratch* out) {
+                               Scratch* out, bool optional) {
     if (t_ws.mode != WsMode::kLibrary) {
         if (num_counters > kWsCounters) return CLOVE_ERR_WORKSPACE;
         char* part = nullptr;
@@ -205,6 +205,12 @@ clove_status_t acquire_scratch(hipStream_t stream, size_t partial_bytes, size_t 
     if (e.base && e.view.partial_bytes >= partial_bytes && e.view.num_counters >= num_counters) {
         *out = e.view;
         return CLOVE_OK;
+    }
+    if (optional) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        const bool known = hipStreamIsCapturing(stream, &cap) == hipSuccess;
+        if (!known) (void)hipGetLastError();
+        if (!known || cap != hipStreamCaptureStatusNone) return CLOVE_ERR_OUT_OF_MEMORY;
     }
     const size_t pb = round_up_pow2(partial_bytes, (size_t)4 << 20);
     const size_t nc = round_up_pow2(num_counters, 4096);

@@ -25,8 +25,20 @@ struct Scratch {
 // current device (implemented in capi.hip): library-owned, or carved from the
 // workspace the calling thread has bound (clove_workspace_bind), or, in a
 // workspace size query, a placeholder that only records the size.
+// `optional`: the caller can do without; during a stream capture the library's
+// scratch is then not grown (an allocation can end the capture) and the call
+// returns CLOVE_ERR_OUT_OF_MEMORY.
 clove_status_t acquire_scratch(hipStream_t stream, size_t partial_bytes, size_t num_counters,
-                               Scratch* out);
+                               Scratch* out, bool optional = false);
+
+// Whether a call whose acquire_scratch returned `st` may go on without a K
+// split: the library's own scratch could not grow (the stream is being
+// captured, or memory is short), or the bound workspace is too small and the
+// plan without a split is an ordinary one for the shape (`few`: small products,
+// which need no workspace to run).
+inline bool scratch_optional(clove_status_t st, bool few) {
+    return st == CLOVE_ERR_OUT_OF_MEMORY || (st == CLOVE_ERR_WORKSPACE && few);
+}
 
 // True while the calling thread runs a workspace size query: calls plan and
 // size their scratch but launch nothing.

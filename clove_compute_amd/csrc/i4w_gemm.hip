@@ -83,8 +83,13 @@ clove_status_t run(Args a, int cus, int target, int min_groups, size_t extra_byt
     char* extra = nullptr;
     if (part_bytes + extra_bytes > 0) {
         Scratch s;
-        const clove_status_t st = acquire_scratch(stream, part_bytes + extra_bytes, (size_t)tiles, &s);
-        if (st != CLOVE_OK) return st;
+        const clove_status_t st = acquire_scratch(stream, part_bytes + extra_bytes, (size_t)tiles, &s, extra_bytes == 0);
+        if (extra_bytes == 0 && scratch_optional(st, a.C <= 32 || a.G < 16)) {
+            a.nsplit = 1;
+            a.gps = a.G;
+        } else if (st != CLOVE_OK) {
+            return st;
+        }
         a.part = s.partials;
         a.counters = s.counters;
         extra = reinterpret_cast<char*>(s.partials) + part_bytes;
@@ -96,7 +101,7 @@ clove_status_t run(Args a, int cus, int target, int min_groups, size_t extra_byt
     static_assert(lds <= 160 * 1024, "LDS");
     if (ensure_lds(reinterpret_cast<const void*>(k), lds) != CLOVE_OK)
         return CLOVE_ERR_LAUNCH;
-    CLOVE_LAUNCH(k, dim3((unsigned)(tiles * pl.nsplit)), dim3(CF::NT), lds, stream, a);
+    CLOVE_LAUNCH(k, dim3((unsigned)(tiles * a.nsplit)), dim3(CF::NT), lds, stream, a);
     return check_launch();
 }
 

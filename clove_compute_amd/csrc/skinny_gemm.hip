@@ -11,9 +11,10 @@ using namespace sk;
 // (I8, BM, BN, WM, WN, stages)
 // (three stages: two workgroups fit a CU and the first stage waits behind a
 // smaller burst, which measured at least as fast as five on every shape with
-// M <= 32: 12 x 1344 x 2816 13.4 -> 9.3 us, 7 x 8057 x 1015 13.0 -> 11.5,
-// 25 x 8640 x 11904 36.6 -> 37.2)
+// M <= 32 and up to 128 K tiles: 12 x 1344 x 2816 13.4 -> 9.3 us, 7 x 8057 x
+// 1015 13.0 -> 11.5)
 using F16M32 = Cfg<false, 32, 128, 1, 4, 3>;
+using F16M32S5 = Cfg<false, 32, 128, 1, 4, 5>;  // past 128 K tiles (27 x 11840 x 10240 46.8 -> 44.6)
 using F16M128 = Cfg<false, 128, 64, 4, 1, 4>;
 // mid-size shapes (M > 256) whose 256x256 tile grid would leave CUs idle:
 // 128x128 tiles (waves of 64x64)
@@ -24,6 +25,8 @@ using F16T128 = Cfg<false, 128, 128, 2, 2, 3>;
 // few tiles: 64x64, 64 KB of LDS, so that two workgroups share a CU (505 x 2304
 // x 1088 14.6 -> 10.5 us against six stages; see pick_f16_tile)
 using F16T64 = Cfg<false, 64, 64, 2, 2, 4>;
+// 72 KB of LDS, two workgroups per CU (see pick_f16_tile)
+using F16W128 = Cfg<false, 64, 128, 2, 2, 3>;
 // the same tile one stage ahead for K <= 512: every workgroup's first stage
 // then waits behind a smaller burst of the whole grid's prologue loads (512^3:
 // 5.5 -> 4.7 us; from K = 1024 the six stages are ahead, 1024^3 8.7 against
@@ -80,8 +83,13 @@ clove_status_t run(Args a, int batch, int cus, hipStream_t stream, int kt_per = 
         Scratch s;
         const size_t bytes =
             (size_t)tiles * a.nsplit * CF::NT * CF::NB * CF::FM * CF::FN * (16 / CF::KW) * sizeof(float);
-        const clove_status_t st = acquire_scratch(stream, bytes, (size_t)tiles, &s);
-        if (st != CLOVE_OK) return st;
+        const clove_status_t st = acquire_scratch(stream, bytes, (size_t)tiles, &s, true);
+        if (scratch_optional(st, nk <= 16)) {
+            a.kps = nk * CF::BK;
+            a.nsplit = 1;
+        } else if (st != CLOVE_OK) {
+            return st;
+        }
         a.part = s.partials;
         a.counters = s.counters;
     }
@@ -98,7 +106,7 @@ bool fits31(int64_t bytes) { return bytes < ((int64_t)1 << 31); }
 // The FP16 tile shapes, chosen by shape alone (so that the fused SwiGLU below
 // picks the same tiles, and with them the same split plan, as the two GEMMs
 // it replaces).
-enum class F16Tile { kM32, kN64, kM128, kT128, kT64, kK32 };
+enum class F16Tile { kM32, kN64, kM128, kT128, kW128, kT64, kK32 };
 
 F16Tile pick_f16_tile(int batch, int M, int N, int K, int cus) {
     const int nk = cdiv(K, F16T64::BK);
@@ -125,6 +133,13 @@ F16Tile pick_f16_tile(int batch, int M, int N, int K, int cus) {
     // against 108.6 us, 2048x8192 at M = 512 35.2 against 47.4 us)
     if (M > 256) {
         const int64_t t128 = (int64_t)cdiv(M, 128) * cdiv(N, 128) * batch;
+        // 64x128 between them, two workgroups a CU: where the 128x128 grid is
+        // too small but this one fills 3/4 of the CUs (334 x 4288 x 1664 20.4 ->
+        // 16.7 us against 64x64, 333 x 5001 x 2050 31.9 -> 25.8), and for short
+        // K (1729 x 2752 x 704 23.4 -> 19.8 against 128x128; 559 x 4352 x 2688
+        // stays, 29.3 against 41.3)
+        const int64_t w64 = (int64_t)cdiv(M, F16W128::BM) * cdiv(N, F16W128::BN) * batch;
+        if (t128 >= cus / 2 ? short_k : !long_k && 4 * w64 >= 3 * cus) return F16Tile::kW128;
         return (t128 >= cus / 2 || long_k) ? F16Tile::kT128 : F16Tile::kT64;
     }
     if (M > 128 && long_k && N >= 4096) return F16Tile::kT128;
@@ -190,10 +205,11 @@ bool try_skinny_fp16(const uint16_t* A, const uint16_t* B, uint16_t* C, int batc
                                : run<CF, kF16AlphaBeta, false, kRagged>(a, batch, cus, stream);
     };
     switch (pick_f16_tile(batch, M, N, K, cus)) {
-        case F16Tile::kM32: *status = go(F16M32{}); break;
+        case F16Tile::kM32: *status = K > 128 * F16M32::BK ? go(F16M32S5{}) : go(F16M32{}); break;
         case F16Tile::kN64: *status = go(F16N64{}); break;
         case F16Tile::kM128: *status = go(F16M128{}); break;
         case F16Tile::kT128: *status = go(F16T128{}); break;
+        case F16Tile::kW128: *status = go(F16W128{}); break;
         case F16Tile::kT64:
             *status = K <= 512 ? go(F16T64S2{}) : go(F16T64{});
             break;
@@ -222,6 +238,15 @@ bool try_skinny_swiglu(const uint16_t* X, const uint16_t* W_gate, const uint16_t
         case F16Tile::kN64: *status = run<SwN64, kF16SwiGLU>(a, 1, cus, stream); break;
         case F16Tile::kM128: *status = run<SwM128, kF16SwiGLU>(a, 1, cus, stream); break;
         case F16Tile::kT128: *status = run<SwT128, kF16SwiGLU>(a, 1, cus, stream); break;
+        case F16Tile::kW128: {
+            // (never split there; two B tiles leave one workgroup a CU, so the
+            // larger tile where its grid is large)
+            const int nk = cdiv(hidden, F16W128::BK);
+            *status = (int64_t)cdiv(T, 128) * cdiv(inter, 128) >= cus / 2
+                          ? run<SwT128, kF16SwiGLU>(a, 1, cus, stream, nk)
+                          : run<SwT64, kF16SwiGLU>(a, 1, cus, stream, nk);
+            break;
+        }
         case F16Tile::kT64: {
             // (96 KB of LDS, one workgroup a CU: past one round of them 128x64 tiles
             // under the same split, 219 x 4224 x 1280 25.5 -> 17.7 us)

@@ -187,3 +187,50 @@ def test_bound_workspace_in_a_graph():
             _ = (dA.float() @ dA.float().T).sum().item()  # eager work between replays
     finally:
         cg.workspace_bind()
+
+
+# small products split K for speed only: where no scratch can be had (a first
+# call on a fresh stream inside a capture, or a bound workspace of the least
+# size) they run without a split
+@pytest.mark.parametrize("kind,M,N,K", [("fp16", 120, 4096, 1024), ("fp16", 100, 3072, 1000), ("w4a16", 40, 2432, 1920),
+                                        ("w4a16", 30, 4864, 2304)])
+def test_small_products_without_scratch(kind, M, N, K):
+    import torch
+    cg = _cg()
+    g = rng("noscratch", M, N, K)
+    if kind == "fp16":
+        A = to_dev(g.integers(-2, 3, (M, K)).astype(np.float16))
+        B = to_dev(g.integers(-2, 3, (K, N)).astype(np.float16))
+        run = lambda C: cg.gemm_fp16(A, B, C, M, N, K)  # noqa: E731
+    else:
+        # small integers and one power-of-two scale: exact in any split
+        A = to_dev(g.integers(-2, 3, (M, K)).astype(np.float16))
+        W = to_dev(g.integers(0, 256, (N, K // 2)).astype(np.uint8))
+        s = torch.full((N, K // 128), 2.0 ** -6, dtype=torch.float16, device="cuda")
+        z = torch.full((N, K // 128), 8.0, dtype=torch.float16, device="cuda")
+        run = lambda C: cg.gemm_w4a16(A, W, s, z, C, M, N, K)  # noqa: E731
+    ref = empty_f16(M, N)
+    run(ref)
+    torch.cuda.synchronize()
+    with cg.workspace_query() as q:
+        run(ref)
+    assert q.bytes > 0  # split when it can
+    C = empty_f16(M, N, fill=float("nan"))
+    cg.workspace_bind(_zeros_ws(65536))
+    try:
+        run(C)
+        torch.cuda.synchronize()
+    finally:
+        cg.workspace_bind()
+    assert np.array_equal(f16bits(to_host(C)), f16bits(to_host(ref)))
+    C = empty_f16(M, N, fill=float("nan"))
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        run(C)
+    for _ in range(3):
+        C.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(f16bits(to_host(C)), f16bits(to_host(ref)))
