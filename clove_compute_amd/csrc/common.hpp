@@ -48,6 +48,16 @@ __device__ __forceinline__ u32x4 shift_bytes(u32x4 x, unsigned s) {
     return s >= 16 ? u32x4{0u, 0u, 0u, 0u} : x;
 }
 
+// the first v of 16 bytes kept, the rest zeroed
+__device__ __forceinline__ u32x4 keep_bytes(u32x4 x, int v) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const int b = v - 4 * d;  // bytes of this word kept
+        x[d] = b >= 4 ? x[d] : b <= 0 ? 0u : x[d] & ((1u << (8 * b)) - 1u);
+    }
+    return x;
+}
+
 // fp16 <-> fp32 (hardware conversions; narrowing is round-to-nearest-even in
 // the default MODE register)
 __device__ __forceinline__ float h2f(uint16_t h) {

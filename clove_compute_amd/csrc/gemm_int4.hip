@@ -110,7 +110,7 @@ __global__ void __launch_bounds__((gemv_max_threads<NV, ALIGNED, 4>())) int4_gem
     // for A (loads complete in order) ----
     constexpr int BCH = 2;  // B chunks per thread in the fast path
     const bool bfast = p.ldb == 1 && NV <= 2 && nch <= BCH * NT &&
-                       (reinterpret_cast<uintptr_t>(p.B) & 15) == 0 && (K & 31) == 0;
+                       (ALIGNED ? (reinterpret_cast<uintptr_t>(p.B) & 15) == 0 && (K & 31) == 0 : K >= 16);
     // (with their groups' B scales and zero points: loaded here, not where the
     // chunk constants are formed, where they would be a second round trip)
     u32x4 braw[BCH][2];
@@ -119,8 +119,13 @@ __global__ void __launch_bounds__((gemv_max_threads<NV, ALIGNED, 4>())) int4_gem
 #pragma unroll
         for (int i = 0; i < BCH; ++i) {
             const int c = min(tid + i * NT, nch - 1);  // unconditional, see below
-            braw[i][0] = *reinterpret_cast<const u32x4*>(p.B + 32 * c);
-            braw[i][1] = *reinterpret_cast<const u32x4*>(p.B + 32 * c + 16);
+            if constexpr (ALIGNED) {
+                braw[i][0] = *reinterpret_cast<const u32x4*>(p.B + 32 * c);
+                braw[i][1] = *reinterpret_cast<const u32x4*>(p.B + 32 * c + 16);
+            } else {
+                braw[i][0] = load_any16(p.B + min(32 * c, K - 16));
+                braw[i][1] = load_any16(p.B + min(32 * c + 16, K - 16));
+            }
             if constexpr (MODE == mg::kI4Groupwise) {
 #pragma unroll
                 for (int n = 0; n < NV; ++n) {
@@ -135,6 +140,7 @@ __global__ void __launch_bounds__((gemv_max_threads<NV, ALIGNED, 4>())) int4_gem
     // A chunks and their group scale / zero.  Loads are unconditional from
     // clamped (valid) addresses and masked where used: a guarded load would
     // become a branch whose merge makes the compiler wait for it right away.
+    const uint8_t* a_last = p.A + (int64_t)p.M * (K / 2) - 16;  // !ALIGNED: M K / 2 >= 16
     u32x4 a[RPW][UPR];
     uint16_t sah[RPW][UPR], zah[RPW][UPR];
     auto load_batch = [&](int c0) {
@@ -147,18 +153,9 @@ __global__ void __launch_bounds__((gemv_max_threads<NV, ALIGNED, 4>())) int4_gem
                 if constexpr (ALIGNED) {
                     a[r][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(arow + 16 * cc));
                 } else {
-                    unsigned w[4];
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        w[d] = 0;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const int byte = 16 * cc + 4 * d + e;
-                            const unsigned b = (2 * byte < K) ? arow[min(byte, K / 2 - 1)] : 0u;
-                            w[d] |= b << (8 * e);
-                        }
-                    }
-                    a[r][u] = u32x4{w[0], w[1], w[2], w[3]};
+                    // (at most 16 bytes before A's end; shifted back where used)
+                    const uint8_t* at = arow + 16 * cc;
+                    a[r][u] = load_any16(at < a_last ? at : a_last);
                 }
                 if constexpr (MODE == mg::kI4Groupwise) {
                     const int64_t gi = (int64_t)ridx[r] * G + (cc >> 2);
@@ -198,6 +195,10 @@ __global__ void __launch_bounds__((gemv_max_threads<NV, ALIGNED, 4>())) int4_gem
         for (int i = 0; i < BCH; ++i) {
             const int c = tid + i * NT;
             if (c >= nch) continue;
+            if constexpr (!ALIGNED) {  // (zero from the end of B on)
+                braw[i][0] = shift_bytes(braw[i][0], max(0, 32 * c - (K - 16)));
+                braw[i][1] = shift_bytes(braw[i][1], max(0, 32 * c + 16 - (K - 16)));
+            }
             const unsigned v[8] = {braw[i][0].x, braw[i][0].y, braw[i][0].z, braw[i][0].w,
                                    braw[i][1].x, braw[i][1].y, braw[i][1].z, braw[i][1].w};
 #pragma unroll
@@ -221,28 +222,35 @@ __global__ void __launch_bounds__((gemv_max_threads<NV, ALIGNED, 4>())) int4_gem
             }
         }
         lds_barrier();
-    } else if (NV > 2 && p.ldb <= 4 && (reinterpret_cast<uintptr_t>(p.B) & 15) == 0) {
+    } else if (NV > 2 && p.ldb <= 4 && (!ALIGNED || (reinterpret_cast<uintptr_t>(p.B) & 15) == 0)) {
         // 3 to 8 columns (1 to 4 bytes per k row): word w of every column from
-        // rows 8w .. 8w + 7, one vector load for 1, 2 or 4 bytes per row, byte
-        // loads for 3 bytes and for the rows of the last word (rows past K
-        // read as zero)
+        // rows 8w .. 8w + 7, vector loads of the eight rows (at byte alignment),
+        // byte loads for the rows of the last word (rows past K read as zero)
         const int ldb = p.ldb;
         for (int w = tid; w < KW; w += NT) {
             const int k0 = 8 * w;
             unsigned rowb[8];  // row j's bytes, byte b of the row at bits 8b
-            if (k0 + 8 <= K && ldb != 3) {
-                if (ldb == 4) {
-                    const u32x4 v0 = *reinterpret_cast<const u32x4*>(p.B + 4 * k0);
-                    const u32x4 v1 = *reinterpret_cast<const u32x4*>(p.B + 4 * k0 + 16);
+            if (k0 + 8 <= K) {
+                if (ldb == 3) {
+                    // 24 bytes: row j is bytes 3 j .. 3 j + 2
+                    const u32x4 v0 = load_any16(p.B + 3 * k0);
+                    const u32x2u v1 = *reinterpret_cast<const u32x2u*>(p.B + 3 * k0 + 16);
+                    const unsigned d[7] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, 0u};
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        rowb[j] = __builtin_amdgcn_alignbyte(d[(3 * j >> 2) + 1], d[3 * j >> 2], (3 * j) & 3);
+                } else if (ldb == 4) {
+                    const u32x4 v0 = load_any16(p.B + 4 * k0);
+                    const u32x4 v1 = load_any16(p.B + 4 * k0 + 16);
                     rowb[0] = v0.x; rowb[1] = v0.y; rowb[2] = v0.z; rowb[3] = v0.w;
                     rowb[4] = v1.x; rowb[5] = v1.y; rowb[6] = v1.z; rowb[7] = v1.w;
                 } else if (ldb == 2) {
-                    const u32x4 v = *reinterpret_cast<const u32x4*>(p.B + 2 * k0);
+                    const u32x4 v = load_any16(p.B + 2 * k0);
                     const unsigned d[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
                     for (int j = 0; j < 8; ++j) rowb[j] = (d[j >> 1] >> (16 * (j & 1))) & 0xffffu;
                 } else {
-                    const u32x2 v = *reinterpret_cast<const u32x2*>(p.B + k0);
+                    const u32x2u v = *reinterpret_cast<const u32x2u*>(p.B + k0);
 #pragma unroll
                     for (int j = 0; j < 8; ++j) rowb[j] = ((j < 4 ? v.x : v.y) >> (8 * (j & 3))) & 0xffu;
                 }
@@ -313,7 +321,11 @@ __global__ void __launch_bounds__((gemv_max_threads<NV, ALIGNED, 4>())) int4_gem
 #pragma unroll
             for (int r = 0; r < RPW; ++r) {
                 const bool valid = row0 + r < p.M && c < nch;
-                const u32x4 av = a[r][u];
+                u32x4 av = a[r][u];
+                if (!ALIGNED && c0 + 64 * u + 64 >= nch) {  // uniform: the row's last chunk is here
+                    const uint8_t* at = p.A + (int64_t)ridx[r] * (K / 2) + 16 * cs;
+                    av = keep_bytes(shift_bytes(av, at > a_last ? (unsigned)(at - a_last) : 0u), K / 2 - 16 * cs);
+                }
                 unsigned sa = __builtin_amdgcn_udot8(av.x, kOnes, 0u, false);
                 sa = __builtin_amdgcn_udot8(av.y, kOnes, sa, false);
                 sa = __builtin_amdgcn_udot8(av.z, kOnes, sa, false);
@@ -510,27 +522,36 @@ clove_status_t run_gemv_shape(const GemvParams& p, int wpb, hipStream_t stream) 
     return check_launch();
 }
 
+template <int NV, int MODE, bool AL>
+clove_status_t run_gemv_by_shape(const GemvParams& p, const GemvShape& g, hipStream_t stream) {
+    // (rpw, upr) pairs keep rpw * upr <= 8 chunk loads per lane
+    if (g.rpw == 1 || (NV == 8 && !AL)) {
+        if (g.upr >= 8) return run_gemv_shape<NV, MODE, 1, 8, AL>(p, g.wpb, stream);
+        if (g.upr >= 6) return run_gemv_shape<NV, MODE, 1, 6, AL>(p, g.wpb, stream);
+        if (g.upr >= 4) return run_gemv_shape<NV, MODE, 1, 4, AL>(p, g.wpb, stream);
+        if (g.upr >= 2) return run_gemv_shape<NV, MODE, 1, 2, AL>(p, g.wpb, stream);
+        return run_gemv_shape<NV, MODE, 1, 1, AL>(p, g.wpb, stream);
+    }
+    if constexpr (NV == 8 && !AL) return CLOVE_ERR_INVALID_ARG;  // (not reached)
+    else if (g.rpw == 2)
+        return g.upr >= 4   ? run_gemv_shape<NV, MODE, 2, 4, AL>(p, g.wpb, stream)
+               : g.upr >= 2 ? run_gemv_shape<NV, MODE, 2, 2, AL>(p, g.wpb, stream)
+                            : run_gemv_shape<NV, MODE, 2, 1, AL>(p, g.wpb, stream);
+    else if (g.rpw == 4)
+        return g.upr >= 2 ? run_gemv_shape<NV, MODE, 4, 2, AL>(p, g.wpb, stream)
+                          : run_gemv_shape<NV, MODE, 4, 1, AL>(p, g.wpb, stream);
+    else
+        return run_gemv_shape<NV, MODE, 8, 1, AL>(p, g.wpb, stream);
+}
+
 template <int NV, int MODE>
 clove_status_t run_gemv(const GemvParams& p, bool aligned, int cus, hipStream_t stream) {
     const GemvShape g = gemv_shape(p.M, p.nch, cus, NV <= 2 ? 2 : 1);
-    // unaligned rows are assembled from byte loads (16 registers per chunk
-    // until packed): one row per wave and one chunk per lane at a time, so
-    // that the variant needs no scratch
-    if (!aligned) return run_gemv_shape<NV, MODE, 1, 1, false>(p, g.wpb, stream);
-    // (rpw, upr) pairs keep rpw * upr <= 8 chunk loads per lane
-    if (g.rpw == 1) {
-        if (g.upr >= 8) return run_gemv_shape<NV, MODE, 1, 8, true>(p, g.wpb, stream);
-        if (g.upr >= 6) return run_gemv_shape<NV, MODE, 1, 6, true>(p, g.wpb, stream);
-        if (g.upr >= 4) return run_gemv_shape<NV, MODE, 1, 4, true>(p, g.wpb, stream);
-        if (g.upr >= 2) return run_gemv_shape<NV, MODE, 1, 2, true>(p, g.wpb, stream);
-        return run_gemv_shape<NV, MODE, 1, 1, true>(p, g.wpb, stream);
-    }
-    if (g.rpw == 2) return g.upr >= 4   ? run_gemv_shape<NV, MODE, 2, 4, true>(p, g.wpb, stream)
-                           : g.upr >= 2 ? run_gemv_shape<NV, MODE, 2, 2, true>(p, g.wpb, stream)
-                                        : run_gemv_shape<NV, MODE, 2, 1, true>(p, g.wpb, stream);
-    if (g.rpw == 4) return g.upr >= 2 ? run_gemv_shape<NV, MODE, 4, 2, true>(p, g.wpb, stream)
-                                      : run_gemv_shape<NV, MODE, 4, 1, true>(p, g.wpb, stream);
-    return run_gemv_shape<NV, MODE, 8, 1, true>(p, g.wpb, stream);
+    // Unaligned rows take the same shapes, with 16-byte loads at byte alignment
+    // (cold, us per call, against byte loads of one chunk a lane: 4096 x 11006 N =
+    // 1 / 4 28.3 -> 9.2 / 31.5 -> 15.3, 1418 x 6712 N = 2 12.3 -> 4.9), but one row
+    // a wave with eight columns, whose registers would spill
+    return aligned ? run_gemv_by_shape<NV, MODE, true>(p, g, stream) : run_gemv_by_shape<NV, MODE, false>(p, g, stream);
 }
 
 // One group-wise column on rows of 65..128 aligned chunks: int4_gemv_ks, four
@@ -632,8 +653,11 @@ clove_status_t launch_gemm_int4(const Int4Args& a, hipStream_t stream) {
         GemvParams p{a.A, a.A_scale, a.A_zero, a.B, a.B_scale, a.B_zero, a.C,
                      a.M, a.N, a.K, G, ldb, cols_valid, nch};
         const bool aligned = aligned16(a.A) && (a.K % 32 == 0);
-        return literal ? gemv_by_n<mg::kI4Literal>(p, aligned, dev.num_cus, stream)
-                       : gemv_by_n<mg::kI4Groupwise>(p, aligned, dev.num_cus, stream);
+        // (the unaligned loads stay at least 16 bytes inside A: fewer bytes take
+        // the generic kernel below)
+        if (aligned || (int64_t)a.M * (a.K / 2) >= 16)
+            return literal ? gemv_by_n<mg::kI4Literal>(p, aligned, dev.num_cus, stream)
+                           : gemv_by_n<mg::kI4Groupwise>(p, aligned, dev.num_cus, stream);
     }
     if (!literal) {
         if (try_i4i4(a, dev.num_cus, stream, &st2)) return st2;

@@ -135,16 +135,6 @@ struct Cfg {
     static constexpr int LDS_UA = 2 * SB + RED;
 };
 
-// the first v of 16 bytes kept, the rest zeroed
-__device__ __forceinline__ u32x4 keep_bytes(u32x4 x, int v) {
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        const int b = v - 4 * d;  // bytes of this word kept
-        x[d] = b >= 4 ? x[d] : b <= 0 ? 0u : x[d] & ((1u << (8 * b)) - 1u);
-    }
-    return x;
-}
-
 // chunk swizzle of B k-row r (see the header comment): the rows one
 // transposing read touches (4 rows x 2 chunks for fp16, 8 rows x 1 chunk for
 // int8) land in 8 different bank groups

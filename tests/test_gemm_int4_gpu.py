@@ -405,3 +405,31 @@ def test_group_partials_zero_point_outside_range():
     assert np.all(P[bad] == np.iinfo(np.int32).min)
     ref = partials_int64(A_q, zA, B_q, zB, np.arange(M), N, K)
     assert np.array_equal(P[~bad].astype(np.int64), ref[~bad])
+
+
+# the GEMV on rows of any alignment (K not a multiple of 32, A or B at odd
+# addresses): the last chunk of a row and of A, every rows-per-wave shape, B of
+# 1 to 4 bytes per k row; group-wise and reference-literal, bit for bit
+@pytest.mark.parametrize("offA,offB", [(0, 0), (3, 1)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (1, 2, 34), (3, 1, 130), (40, 2, 2050), (700, 3, 1474), (9000, 1, 1022),
+                                   (2100, 2, 4100), (64, 5, 3000), (1500, 6, 700), (33, 7, 9210), (100, 8, 14334),
+                                   (17, 4, 2), (2, 1, 6)])
+def test_gemv_any_alignment_bit_exact(M, N, K, offA, offB):
+    import torch
+    A_q, sA, zA, B_q, sB, zB = make_case(M, N, K, "gemv-any", pow2=True, small=True)
+    a = torch.full((offA + A_q.size,), 0xFF, dtype=torch.uint8, device="cuda")
+    b = torch.full((offB + B_q.size,), 0xFF, dtype=torch.uint8, device="cuda")
+    a[offA:], b[offB:] = to_dev(A_q).reshape(-1), to_dev(B_q).reshape(-1)
+    dA, dB = a[offA:].view(A_q.shape), b[offB:].view(B_q.shape)
+    rows = np.arange(M) if M <= 256 else np.unique(np.concatenate([np.arange(64), np.arange(M - 64, M)]))
+    C = empty_f16(M, N, fill=float("nan"))
+    _cg().gemm_int4_ex(dA, to_dev(sA), to_dev(zA), dB, to_dev(sB), to_dev(zB), C, M, N, K, 0)
+    torch.cuda.synchronize()
+    _, ref, _ = oracle.gemm_int4_groupwise(A_q[rows], sA[rows], zA[rows], B_q, sB, zB, len(rows), N, K)
+    assert np.array_equal(f16bits(to_host(C)[rows]), f16bits(ref.astype(np.float16)))
+    if N % 2 == 0:  # (the literal mode's B rows are N / 2 bytes)
+        C = empty_f16(M, N, fill=float("nan"))
+        _cg().gemm_int4_ex(dA, to_dev(sA), None, dB, to_dev(sB), None, C, M, N, K, LIT)
+        torch.cuda.synchronize()
+        ref = oracle.gemm_int4_literal(A_q[rows], sA[rows], B_q, sB, len(rows), N, K)
+        assert np.array_equal(f16bits(to_host(C)[rows]), f16bits(ref))
