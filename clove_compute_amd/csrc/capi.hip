@@ -117,9 +117,9 @@ size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 // Carves `bytes` for the current call; nullptr-based in a query (nothing is
 // launched, so nothing reads it).
 clove_status_t ws_carve(size_t bytes, char** out) {
-    const size_t off = t_ws.used;
-    t_ws.used += round256(bytes);
-    if (t_ws.mode == WsMode::kBound && t_ws.used > t_ws.bytes) return CLOVE_ERR_WORKSPACE;
+    const size_t off = t_ws.used, end = off + round256(bytes);
+    if (t_ws.mode == WsMode::kBound && end > t_ws.bytes) return CLOVE_ERR_WORKSPACE;
+    t_ws.used = end;
     *out = reinterpret_cast<char*>(reinterpret_cast<uintptr_t>(t_ws.ptr) + off);
     return CLOVE_OK;
 }

@@ -139,15 +139,20 @@ clove_status_t launch_swiglu_fused_fp16(const uint16_t* X, const uint16_t* W_gat
 clove_status_t acquire_buffer(hipStream_t stream, int slot, size_t bytes, void** out);
 constexpr int kBufSwiglu = 1;  // gate / up intermediates of the unfused SwiGLU paths
 
-// FP16 with two to four rows of A: the skinny MFMA kernel rather than the
-// GEMV once the weight is large (cold, measured: 11008 x 4096 at M = 2 / 3 /
-// 4: 21.1 / 21.3 / 21.0 us against 26.5 / 32.2 / 31.8 on the GEMV; 4096 x 4096
-// at M = 3: 12.6 against 13.8; 2048 x 2048 at M = 3 and 4096 x 4096 at M = 2
-// stay on the GEMV: 9.6 against 12.6, 11.8 against 12.6).  gemm_fp16 and the
-// fused SwiGLU take the same decision per projection.
-inline bool skinny_before_gemv(int M, int N, int K) {
+// FP16 with up to four rows of A: the skinny MFMA kernel rather than the GEMV.
+// Large weights first (cold, us per call: 11008 x 4096 at M = 2 / 3 / 4 21.1 /
+// 21.3 / 21.0 against 26.5 / 32.2 / 31.8 on the GEMV).  Below that line its small
+// tiles: three or four rows always (3 x 2424 x 816 9.1 -> 5.9, 4 x 8192 x 576 9.8
+// -> 5.0, 4 x 1024 x 4096 10.1 -> 10.3, 64 heads of 4 x 320 x 64 both ways 17.1 ->
+// 7.2), one or two up to K = 640 (1 x 8192 x 576 6.7 -> 5.4, 2 x 2048 x 512 6.1 ->
+// 4.2, 64 heads of 1 x 320 x 64 11.0 -> 8.1; 1 x 2424 x 816 stays, 5.2 against 5.8).
+// One unbatched product needs K % 64 == 0 there: gemm_fp16 and the fused SwiGLU
+// take the same decision per projection, and the fused kernel takes whole K tiles.
+inline bool skinny_before_gemv(int batch, int M, int N, int K) {
     const int64_t nk = (int64_t)N * K;
-    return M >= 2 && M <= 4 && nk > (M == 2 ? ((int64_t)24 << 20) : ((int64_t)5 << 20));
+    if (M < 1 || M > 4) return false;
+    if (M >= 2 && nk > (M == 2 ? ((int64_t)24 << 20) : ((int64_t)5 << 20))) return true;
+    return (batch > 1 || K % 64 == 0) && (M >= 3 || K <= 640);
 }
 
 // MFMA path for few rows of A against a large N-contiguous B (skinny_gemm.hip):

@@ -59,7 +59,12 @@ constexpr int GV_ROWS = GV_KL * GV_RPT;   // k rows per workgroup
 // over the same k in the same order as in the one-operand kernel (the k
 // mapping does not depend on the column), so gate and up are bit-identical
 // to two gemm_fp16 calls; the epilogue rounds both to fp16 and applies SwiGLU.
-template <int MM, bool SWIGLU = false>
+//
+// UA: B rows of any alignment (N not a multiple of 8, N >= 8), by 16-byte loads
+// at element alignment; the block that passes N loads its row's last 8 columns
+// and shifts them into place.  us per call against the MFMA kernel, which
+// stages such rows through registers: see the dispatch below.
+template <int MM, bool SWIGLU = false, bool UA = false>
 __global__ void __launch_bounds__(1024) gemv_f16(GemvParams p) {
     __shared__ float red[16][MM][GV_COLS];
     __shared__ float s_up[SWIGLU ? MM : 1][SWIGLU ? GV_COLS / 2 : 1];
@@ -95,9 +100,15 @@ __global__ void __launch_bounds__(1024) gemv_f16(GemvParams p) {
 #pragma unroll
     for (int j = 0; j < GV_RPT; ++j) {
         const int k = min(kbeg + kl + GV_KL * j, K - 1);
-        bv[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(B + (int64_t)k * N + nc));
+        const uint16_t* src = B + (int64_t)k * N + nc;
+        if constexpr (UA) bv[j] = load_any16(reinterpret_cast<const unsigned char*>(src));
+        else bv[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src));
     }
     __builtin_amdgcn_sched_barrier(0);  // every B row requested before the first FMA
+    if (UA && cb * CW + CW > N) {  // uniform
+#pragma unroll
+        for (int j = 0; j < GV_RPT; ++j) bv[j] = shift_bytes(bv[j], (unsigned)min(2 * (n - nc), 16));
+    }
     if (kbeg + GV_ROWS > K) {  // rows past K (the last split's): zero, not the clamped row's NaN or infinity
 #pragma unroll
         for (int j = 0; j < GV_RPT; ++j)
@@ -306,7 +317,7 @@ clove_status_t run_dma(const uint16_t* A, const uint16_t* B, uint16_t* C, int ba
     return check_launch();
 }
 
-template <int MM, bool SWIGLU = false>
+template <int MM, bool SWIGLU = false, bool UA = false>
 clove_status_t run_gemv(GemvParams p, int batch, hipStream_t stream) {
     p.col_blocks = cdiv(p.N, SWIGLU ? GV_COLS / 2 : GV_COLS);
     p.nsplit = cdiv(p.K, GV_ROWS);
@@ -316,14 +327,14 @@ clove_status_t run_gemv(GemvParams p, int batch, hipStream_t stream) {
     if (p.nsplit > 1) {
         Scratch s;
         const size_t bytes = (size_t)tiles * p.nsplit * MM * GV_COLS * sizeof(float);
-        clove_status_t st = acquire_scratch(stream, bytes, (size_t)tiles, &s);
+        clove_status_t st = acquire_scratch(stream, bytes, (size_t)tiles, &s, UA);
         if (st != CLOVE_OK) return st;
         p.ws = s.partials;
         p.counters = s.counters;
     }
     const int64_t grid = (int64_t)tiles * p.nsplit;
     if (grid > 0x7fffffff) return CLOVE_ERR_INVALID_DIM;
-    CLOVE_LAUNCH((gemv_f16<MM, SWIGLU>), dim3((unsigned)grid), dim3(1024), 0, stream, p);
+    CLOVE_LAUNCH((gemv_f16<MM, SWIGLU, UA>), dim3((unsigned)grid), dim3(1024), 0, stream, p);
     return check_launch();
 }
 
@@ -359,7 +370,7 @@ clove_status_t launch_gemm_fp16(const uint16_t* A, const uint16_t* B, uint16_t* 
                          (N % 8 == 0);
     const int64_t sA = (int64_t)M * K, sB = (int64_t)K * N, sC = (int64_t)M * N;
 
-    if (skinny_before_gemv(M, N, K)) {
+    if (skinny_before_gemv(batch, M, N, K)) {
         clove_status_t st2;
         if (try_skinny_fp16(A, B, C, batch, M, N, K, alpha, beta, dev.num_cus, stream, &st2)) return st2;
     }
@@ -369,6 +380,17 @@ clove_status_t launch_gemm_fp16(const uint16_t* A, const uint16_t* B, uint16_t* 
         if (M == 1) return run_gemv<1>(g, batch, stream);
         if (M == 2) return run_gemv<2>(g, batch, stream);
         return run_gemv<4>(g, batch, stream);
+    }
+    // rows of B at any alignment, up to two rows of A (us per call against the
+    // MFMA kernel: 1 x 2422 x 818 9.1 -> 5.6, 1 x 9001 x 1100 13.7 -> 9.2, 2 x 2422 x
+    // 818 9.7 -> 6.8, 2 x 4097 x 4096 15.7 -> 15.6; at three rows it loses, 3 x 300 x
+    // 300 5.7 -> 8.8); without scratch for the K splits the MFMA kernel takes the
+    // call
+    if (N >= 8 && M <= 2 && K > 0) {
+        GemvParams g{A, B, C, nullptr, M, N, K, alpha, beta, sA, sB, sC, 0, 1, nullptr, nullptr};
+        const clove_status_t gst =
+            M == 1 ? run_gemv<1, false, true>(g, batch, stream) : run_gemv<2, false, true>(g, batch, stream);
+        if (gst != CLOVE_ERR_OUT_OF_MEMORY && gst != CLOVE_ERR_WORKSPACE) return gst;
     }
     Params p{};
     p.a = A; p.b = B; p.c = C;

@@ -327,7 +327,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64) int8_mfma(I8Params p) {
 // end of the kernel).
 constexpr int kIvCols = 256, kIvKl = 1024 / (kIvCols / 16), kIvRpt = 4, kIvRows = kIvKl * kIvRpt;
 
-template <int MM, int OUT>
+// UA: B rows of any alignment (N not a multiple of 16, N >= 16), by 16-byte loads
+// at byte alignment; the block that passes N loads its row's last 16 columns
+// and shifts them into place.
+template <int MM, int OUT, bool UA>
 __global__ void __launch_bounds__(1024) int8_gemv(I8Params p, int col_blocks) {
     constexpr int IV_RPT = kIvRpt, IV_ROWS = kIvRows;
     constexpr int IV_COLS = kIvCols, IV_KL = kIvKl, CL = IV_COLS / 16;  // CL: column lanes
@@ -357,9 +360,15 @@ __global__ void __launch_bounds__(1024) int8_gemv(I8Params p, int col_blocks) {
 #pragma unroll
     for (int j = 0; j < IV_RPT; ++j) {
         const int k = min(kbeg + kl + IV_KL * j, K - 1);
-        bv[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.B + (int64_t)k * N + nc));
+        const int8_t* src = p.B + (int64_t)k * N + nc;
+        if constexpr (UA) bv[j] = load_any16(reinterpret_cast<const unsigned char*>(src));
+        else bv[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src));
     }
     __builtin_amdgcn_sched_barrier(0);  // every B row requested before the first product
+    if (UA && cb * IV_COLS + IV_COLS > N) {  // uniform
+#pragma unroll
+        for (int j = 0; j < IV_RPT; ++j) bv[j] = shift_bytes(bv[j], (unsigned)min(n - nc, 16));
+    }
 
     // Each column's four k rows (k = kbeg + kl + IV_KL j, j < 4) in one dword:
     // a 4 x 4 byte transpose of the rows' 16-byte loads (v_perm), so that one
@@ -514,7 +523,7 @@ __global__ void __launch_bounds__(1024) int8_gemv(I8Params p, int col_blocks) {
 // ---------------------------------------------------------------------------
 namespace {
 
-template <int OUT>
+template <int OUT, bool UA = false>
 clove_status_t run_gemv(I8Params p, hipStream_t stream) {
     const int mm = p.M == 1 ? 1 : (p.M == 2 ? 2 : 4);
     const int rows = kIvRows;
@@ -530,11 +539,11 @@ clove_status_t run_gemv(I8Params p, hipStream_t stream) {
         // whose counter region is smaller takes the partial-tile reduction
         Scratch s;
         clove_status_t st = CLOVE_ERR_WORKSPACE;
-        if (p.nsplit < 65536) st = acquire_scratch(stream, 0, (size_t)col_blocks * mm * IV_COLS * 2, &s);
+        if (p.nsplit < 65536) st = acquire_scratch(stream, 0, (size_t)col_blocks * mm * IV_COLS * 2, &s, UA);
         if (st == CLOVE_OK) {
             p.counters = s.counters;
         } else if (st == CLOVE_ERR_WORKSPACE) {
-            st = acquire_scratch(stream, (size_t)col_blocks * p.nsplit * mm * IV_COLS * 4, (size_t)col_blocks, &s);
+            st = acquire_scratch(stream, (size_t)col_blocks * p.nsplit * mm * IV_COLS * 4, (size_t)col_blocks, &s, UA);
             if (st != CLOVE_OK) return st;
             p.ws = s.partials;
             p.counters = s.counters;
@@ -545,9 +554,9 @@ clove_status_t run_gemv(I8Params p, hipStream_t stream) {
     const int64_t g = (int64_t)col_blocks * p.nsplit;
     if (g > 0x7fffffff) return CLOVE_ERR_INVALID_DIM;
     const dim3 grid((unsigned)g);
-    if (p.M == 1) CLOVE_LAUNCH((int8_gemv<1, OUT>), grid, dim3(1024), 0, stream, p, col_blocks);
-    else if (p.M == 2) CLOVE_LAUNCH((int8_gemv<2, OUT>), grid, dim3(1024), 0, stream, p, col_blocks);
-    else CLOVE_LAUNCH((int8_gemv<4, OUT>), grid, dim3(1024), 0, stream, p, col_blocks);
+    if (p.M == 1) CLOVE_LAUNCH((int8_gemv<1, OUT, UA>), grid, dim3(1024), 0, stream, p, col_blocks);
+    else if (p.M == 2) CLOVE_LAUNCH((int8_gemv<2, OUT, UA>), grid, dim3(1024), 0, stream, p, col_blocks);
+    else CLOVE_LAUNCH((int8_gemv<4, OUT, UA>), grid, dim3(1024), 0, stream, p, col_blocks);
     return check_launch();
 }
 
@@ -658,6 +667,23 @@ clove_status_t launch_gemm_int8(const Int8Args& a, hipStream_t stream) {
             case Int8Out::kHalfRowCol: return run_gemv<(int)Int8Out::kHalfRowCol>(p, stream);
             case Int8Out::kAcc32: return run_gemv<(int)Int8Out::kAcc32>(p, stream);
         }
+    }
+    // rows of B at any alignment: one or two rows of A, three or four on mid-size
+    // weights (us per call against the skinny kernel: 1 x 1613 x 1472 11.1 -> 5.9, 1 x
+    // 10001 x 9000 32.2 -> 22.8, 2 x 4097 x 4096 with a zero point 14.1 -> 9.6, 4 x
+    // 9001 x 1100 12.4 -> 10.7; 4 x 4097 x 4096 stays, 14.1 against 17.0, and 4 x 600 x
+    // 600, 9.1 against 10.6); without scratch for the K splits the skinny kernel
+    // takes the call
+    const int64_t nk = (int64_t)a.N * a.K;
+    if (!gemv && (a.M <= 2 || (a.M <= 4 && nk >= ((int64_t)1 << 19) && nk <= ((int64_t)12 << 20))) && a.K > 0 &&
+        a.N >= 16) {
+        clove_status_t gst = CLOVE_ERR_INVALID_ARG;
+        switch (a.out) {
+            case Int8Out::kHalfPerTensor: gst = run_gemv<(int)Int8Out::kHalfPerTensor, true>(p, stream); break;
+            case Int8Out::kHalfRowCol: gst = run_gemv<(int)Int8Out::kHalfRowCol, true>(p, stream); break;
+            case Int8Out::kAcc32: gst = run_gemv<(int)Int8Out::kAcc32, true>(p, stream); break;
+        }
+        if (gst != CLOVE_ERR_OUT_OF_MEMORY && gst != CLOVE_ERR_WORKSPACE) return gst;
     }
     // the skinny kernel for the rest, except (M > 2048, zero points 0, whole K
     // tiles) where the register-staged 256x256 tiles are ahead

@@ -155,9 +155,9 @@ F16Tile pick_f16_tile(int batch, int M, int N, int K, int cus) {
     return short_k && few ? F16Tile::kM32 : F16Tile::kM128;
 }
 
-bool f16_domain(const void* A, const void* B, const void* C, int M, int N, int K) {
-    if (M <= 1 || K <= 0 || K % 8 != 0 || N < 8 || N % 8 != 0) return false;
-    if (M <= 4 && !skinny_before_gemv(M, N, K)) return false;
+bool f16_domain(int batch, const void* A, const void* B, const void* C, int M, int N, int K) {
+    if (M <= 0 || K <= 0 || K % 8 != 0 || N < 8 || N % 8 != 0) return false;
+    if (M <= 4 && !skinny_before_gemv(batch, M, N, K)) return false;
     if (!aligned16(A) || !aligned16(B) || !aligned16(C)) return false;
     // (the DMA offsets of the padded rows m < M + 128 must stay 32-bit)
     return fits31((int64_t)(M + 128) * K * 2) && fits31((int64_t)(K + 64) * N * 2) && fits31((int64_t)M * N * 2);
@@ -184,7 +184,7 @@ using SwK32 = Cfg<false, 32, 32, 1, 1, 3, 2, 4>;
 
 bool try_skinny_fp16(const uint16_t* A, const uint16_t* B, uint16_t* C, int batch, int M, int N, int K,
                      float alpha, float beta, int cus, hipStream_t stream, clove_status_t* status) {
-    const bool al = f16_domain(A, B, C, M, N, K);
+    const bool al = f16_domain(batch, A, B, C, M, N, K);
     if (!al && !ua_domain(M, N, K, 2)) return false;
     Args a{};
     a.A = A;
@@ -220,7 +220,7 @@ bool try_skinny_fp16(const uint16_t* A, const uint16_t* B, uint16_t* C, int batc
 
 bool try_skinny_swiglu(const uint16_t* X, const uint16_t* W_gate, const uint16_t* W_up, uint16_t* out, int T,
                        int hidden, int inter, int cus, hipStream_t stream, clove_status_t* status) {
-    if (!f16_domain(X, W_gate, out, T, inter, hidden) || !aligned16(W_up) || hidden % 64 != 0) return false;
+    if (!f16_domain(1, X, W_gate, out, T, inter, hidden) || !aligned16(W_up) || hidden % 64 != 0) return false;
     Args a{};
     a.A = X;
     a.B = W_gate;

@@ -122,7 +122,7 @@ clove_status_t launch_swiglu_fused_fp16(const uint16_t* X, const uint16_t* W_gat
     }
     // (the kernel family gemm_fp16 takes for each projection: the skinny
     // kernel first where it would, then the GEMV for T <= 4)
-    if (skinny_before_gemv(T, inter, hidden) &&
+    if (skinny_before_gemv(1, T, inter, hidden) &&
         try_skinny_swiglu(X, W_gate, W_up, out, T, hidden, inter, dev.num_cus, stream, &st))
         return st;
     if (try_gemv_swiglu(X, W_gate, W_up, out, T, hidden, inter, stream, &st)) return st;

@@ -416,3 +416,27 @@ def test_small_product_tiles_bit_exact(M, N, K):
     C = run_fp16(A, B, C0, alpha=1.0, beta=0.5)
     exact = A.astype(np.float64) @ B.astype(np.float64) + 0.5 * C0.astype(np.float64)
     assert np.array_equal(f16bits(C), f16bits(exact.astype(np.float16)))
+
+
+# one to four rows: the GEMV on rows of B at any alignment (the block that passes
+# N shifts its row's last columns into place) and the skinny kernel's small
+# tiles, unbatched and batched, with and without K splits
+@pytest.mark.parametrize("batch,M,N,K,off", [(1, 1, 9, 300, 0), (1, 1, 2422, 818, 1), (1, 2, 515, 1100, 0), (1, 2, 264, 512, 3),
+                                             (3, 1, 257, 33, 0), (5, 2, 8, 700, 1), (1, 1, 8192, 576, 0), (1, 2, 2048, 512, 0),
+                                             (1, 3, 2424, 816, 0), (1, 4, 304, 320, 0), (4, 3, 320, 64, 0), (4, 4, 80, 200, 0),
+                                             (2, 1, 1000, 640, 0), (1, 3, 300, 77, 1)])
+def test_few_rows_any_alignment_bit_exact(batch, M, N, K, off):
+    import torch
+    g = rng("few-rows", batch, M, N, K)
+    A = g.integers(-3, 4, (batch, M, K)).astype(np.float16)
+    B = g.integers(-3, 4, (batch, K, N)).astype(np.float16)
+    dA = torch.empty(off + A.size, dtype=torch.float16, device="cuda")
+    dB = torch.empty(off + B.size, dtype=torch.float16, device="cuda")
+    dA[off:], dB[off:] = to_dev(A).reshape(-1), to_dev(B).reshape(-1)
+    C = torch.full((off + batch * M * N + 8,), float("nan"), dtype=torch.float16, device="cuda")
+    _cg().gemm_fp16_batched(dA[off:], dB[off:], C[off:], batch, M, N, K, 1.0)
+    torch.cuda.synchronize()
+    exact = np.matmul(A.astype(np.float64), B.astype(np.float64)).astype(np.float16)
+    got = to_host(C)
+    assert np.array_equal(f16bits(got[off:off + exact.size]), f16bits(exact.reshape(-1)))
+    assert np.all(np.isnan(got[:off])) and np.all(np.isnan(got[off + exact.size:]))  # nothing past the output

@@ -241,7 +241,8 @@ def test_big_tile(M, N, K):
     (1, 17, 17, 3, -5), (2, 1001, 2906, 17, 0), (4, 4096, 2051, -9, 5), (1, 2049, 4097, 0, 0), (3, 12304, 4098, -3, 5),
     (33, 784, 5246, -3, 5), (64, 1709, 814, -9, 0), (100, 4099, 1158, 0, 0), (130, 333, 4098, -3, 5),
     (128, 10241, 4097, 7, 0), (300, 2624, 2112, 0, -5), (40, 512, 4176, -3, 5), (513, 1613, 894, 17, 0),
-    (2050, 272, 160, -9, 1),
+    (2050, 272, 160, -9, 1), (1, 515, 4100, 0, 0), (2, 1613, 1472, 17, 0), (3, 1000, 1030, -3, 5), (4, 9001, 300, 0, 7),
+    (4, 17, 40000, 3, -5),
 ])
 def test_unaligned_and_ragged_k_bit_exact(M, N, K, za, zb):
     g = rng("un8", M, N, K, za, zb)

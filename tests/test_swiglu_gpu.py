@@ -257,7 +257,8 @@ def test_swiglu_fused_equals_gemms_then_swiglu(T, H, I):
 
 # the same where the fused call takes other tiles than the GEMMs under their K
 # split (219 x 4224 x 1280), and k slices with a K split (20 x 1024 x 2048)
-@pytest.mark.parametrize("T,H,I", [(219, 1280, 4224), (143, 1152, 7936), (20, 2048, 1024), (35, 2688, 1536), (12, 1536, 4608)])
+@pytest.mark.parametrize("T,H,I", [(219, 1280, 4224), (143, 1152, 7936), (20, 2048, 1024), (35, 2688, 1536), (12, 1536, 4608),
+                                   (1, 512, 1000), (2, 640, 264), (3, 1024, 520), (4, 1000, 512), (3, 1152, 3328)])
 def test_swiglu_fused_equals_gemms_small_tiles(T, H, I):
     test_swiglu_fused_equals_gemms_then_swiglu(T, H, I)
 
