@@ -538,7 +538,9 @@ __global__ void __launch_bounds__(256) i4w_prep_b(const uint8_t* __restrict__ B,
     // workgroup makes one round trip to memory.  Every load is unconditional,
     // from a clamped address, and masked afterwards: a guarded load becomes a
     // branch whose merge waits for it, which would serialize the round trips.
-    const int c8 = tid & 15, k8 = tid >> 4;
+    // (a wave covers 4 column blocks x all 16 k blocks: each of its stores writes
+    // the 256 contiguous bytes a group takes in four columns)
+    const int k8 = tid & 15, c8 = tid >> 4;
     const int n0 = 2 * b0 + 8 * c8;
     uint16_t zh[8], sh16[8];
 #pragma unroll
