@@ -64,7 +64,6 @@ clove_status_t run(const Int4Args& q, int32_t* P, int cus, hipStream_t stream) {
     a.tiles_m = pl.tiles_m;
     a.nsplit = pl.nsplit;
     a.gps = pl.gps;
-    a.vec_store = (q.N % 8 == 0) && aligned16(q.C);
     const int tiles = a.tiles_m * a.tiles_n;
     const size_t slab = (size_t)BR * BC * 4;  // one fp32 partial tile
     const size_t part_bytes = !P && a.nsplit > 1 ? (size_t)tiles * a.nsplit * slab : 0;

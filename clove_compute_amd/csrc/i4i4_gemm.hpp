@@ -110,7 +110,6 @@ struct Args {
     int ldb;
     int M, N, K, G, Npad;
     int tiles_m, tiles_n, nsplit, gps;  // gps: groups per split, even (G is even)
-    int vec_store;        // 16-byte output stores (N % 8 == 0, C 16-byte aligned)
     float* part;
     unsigned* counters;
     int* P;               // partials mode: [M, N, G] int32
@@ -694,8 +693,8 @@ __global__ void __launch_bounds__(NT) i4i4_gemm(Args p) {
                 continue;
             }
         }
-        if (p.vec_store && gn + 7 < p.N) {
-            *reinterpret_cast<u32x4*>(dst) = v;
+        if (gn + 7 < p.N) {
+            *reinterpret_cast<u32x4u*>(dst) = v;  // (rows at any alignment)
         } else {
             const unsigned w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll

@@ -494,8 +494,10 @@ __global__ void __launch_bounds__(CF::NT) i4w_gemm(Args p) {
                 const int c = c0 + wc * 32 * FX + 32 * j + 8 * q + 4 * h;  // 4 consecutive columns
                 if constexpr (OUT == 0) {
                     uint16_t* dst = p.out + (int64_t)r * p.C + c;
-                    if (c + 3 < p.C && (p.C & 3) == 0) {
-                        *reinterpret_cast<u32x2*>(dst) =
+                    // (rows at any alignment: one store instead of four of 2 bytes, whose
+                    // partial lines cost more than the product at odd widths)
+                    if (c + 3 < p.C) {
+                        *reinterpret_cast<u32x2u*>(dst) =
                             u32x2{pack2h(acc[i][j][4 * q], acc[i][j][4 * q + 1]),
                                   pack2h(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3])};
                     } else {

@@ -468,8 +468,8 @@ __global__ void __launch_bounds__(SC::NT) i4w_stream(Args p) {
             if constexpr (OUT == 0) {
                 // (accumulator entry e is column c + (e ^ 1))
                 uint16_t* dst = p.out + (int64_t)r * p.C + c;
-                if (c + 3 < p.C && (p.C & 3) == 0) {
-                    *reinterpret_cast<u32x2*>(dst) = u32x2{pack2h(acc[x][f][1], acc[x][f][0]),
+                if (c + 3 < p.C) {
+                    *reinterpret_cast<u32x2u*>(dst) = u32x2{pack2h(acc[x][f][1], acc[x][f][0]),
                                                            pack2h(acc[x][f][3], acc[x][f][2])};
                 } else {
 #pragma unroll
