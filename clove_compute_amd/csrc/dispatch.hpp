@@ -146,11 +146,13 @@ constexpr int kBufSwiglu = 1;  // gate / up intermediates of the unfused SwiGLU 
 // -> 5.0, 4 x 1024 x 4096 10.1 -> 10.3, 64 heads of 4 x 320 x 64 both ways 17.1 ->
 // 7.2), one or two up to K = 640 (1 x 8192 x 576 6.7 -> 5.4, 2 x 2048 x 512 6.1 ->
 // 4.2, 64 heads of 1 x 320 x 64 11.0 -> 8.1; 1 x 2424 x 816 stays, 5.2 against 5.8).
-// One unbatched product needs K % 64 == 0 there: gemm_fp16 and the fused SwiGLU
-// take the same decision per projection, and the fused kernel takes whole K tiles.
+// An unbatched product of the fused SwiGLU's form (K % 8 == 0, N % 8 == 0) needs
+// K % 64 == 0 for either: the fused kernel takes whole K tiles, and with others
+// the fused call runs the GEMV, whose sums the two gemm_fp16 calls must share.
 inline bool skinny_before_gemv(int batch, int M, int N, int K) {
     const int64_t nk = (int64_t)N * K;
     if (M < 1 || M > 4) return false;
+    if (batch == 1 && K % 64 != 0 && K % 8 == 0 && N % 8 == 0) return false;
     if (M >= 2 && nk > (M == 2 ? ((int64_t)24 << 20) : ((int64_t)5 << 20))) return true;
     return (batch > 1 || K % 64 == 0) && (M >= 3 || K <= 640);
 }

@@ -263,6 +263,14 @@ def test_swiglu_fused_equals_gemms_small_tiles(T, H, I):
     test_swiglu_fused_equals_gemms_then_swiglu(T, H, I)
 
 
+# the same for two to four rows with hidden % 64 != 0, on weights above the
+# line where two to four rows with whole K tiles leave the GEMV: both calls
+# stay on it
+@pytest.mark.parametrize("T,H,I", [(2, 4104, 11008), (3, 1000, 8192), (3, 4104, 4096), (4, 2056, 4096)])
+def test_swiglu_fused_equals_gemms_ragged_hidden(T, H, I):
+    test_swiglu_fused_equals_gemms_then_swiglu(T, H, I)
+
+
 @pytest.mark.parametrize("T,H,I,offset", [(5, 60, 100, False), (3, 100, 30, False), (33, 200, 72, False),
                                           (2, 256, 128, True), (20, 128, 64, True)])
 def test_swiglu_fused_direct_fallback(T, H, I, offset):
