@@ -59,6 +59,18 @@ __global__ void zero_u32(unsigned* p, size_t n) {
     for (; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0u;
 }
 
+// Test hook (clove_test_alloc_excess): bytes added to this thread's allocations
+thread_local size_t t_alloc_excess = 0;
+
+// hipMalloc whose failure leaves nothing behind: the status is the only report
+// of it, and the error HIP keeps for the thread would come back from the next
+// check_launch, also from the launch of a call that goes on without scratch.
+bool device_malloc(void** p, size_t bytes) {
+    if (hipMalloc(p, bytes + t_alloc_excess) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 size_t round_up_pow2(size_t x, size_t floor_bytes) {
     size_t r = floor_bytes;
     while (r < x) r <<= 1;
@@ -215,7 +227,7 @@ clove_status_t acquire_scratch(hipStream_t stream, size_t partial_bytes, size_t 
     const size_t pb = round_up_pow2(partial_bytes, (size_t)4 << 20);
     const size_t nc = round_up_pow2(num_counters, 4096);
     void* base = nullptr;
-    if (hipMalloc(&base, pb + nc * sizeof(unsigned)) != hipSuccess) return CLOVE_ERR_OUT_OF_MEMORY;
+    if (!device_malloc(&base, pb + nc * sizeof(unsigned))) return CLOVE_ERR_OUT_OF_MEMORY;
     if (e.base) {
         // queued work (and calls of other host threads) may still use the old buffer
         g_retired[dev].push_back(e.base);
@@ -253,7 +265,7 @@ clove_status_t acquire_buffer(hipStream_t stream, int slot, size_t bytes, void**
     }
     const size_t nb = round_up_pow2(bytes, (size_t)1 << 20);
     void* base = nullptr;
-    if (hipMalloc(&base, nb) != hipSuccess) return CLOVE_ERR_OUT_OF_MEMORY;
+    if (!device_malloc(&base, nb)) return CLOVE_ERR_OUT_OF_MEMORY;
     if (e.base) g_retired[dev].push_back(e.base);  // as in acquire_scratch
     e.base = base;
     e.bytes = nb;
@@ -588,6 +600,10 @@ clove_status_t clove_workspace_bind(void* ptr, size_t bytes) {
     t_ws.bytes = bytes;
     return CLOVE_OK;
 }
+
+// Test hook, not part of the ABI: the calling thread's scratch allocations ask
+// for `bytes` more than they need (an amount no device holds makes them fail).
+void clove_test_alloc_excess(size_t bytes) { t_alloc_excess = bytes; }
 
 clove_status_t clove_workspace_query_begin(void) {
     if (t_ws.mode == WsMode::kQuery) return CLOVE_ERR_INVALID_ARG;

@@ -234,3 +234,41 @@ def test_small_products_without_scratch(kind, M, N, K):
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(f16bits(to_host(C)), f16bits(to_host(ref)))
+
+
+# an allocation that fails: a small product runs without its split, a GEMV over
+# several K splits reports the failure and writes nothing, and no later call
+# reports it again
+def test_failed_scratch_allocation_leaves_no_error():
+    import ctypes
+    import torch
+    from clove_compute_amd import _lib
+    cg = _cg()
+    excess = _lib.lib().clove_test_alloc_excess
+    excess.argtypes, excess.restype = [ctypes.c_size_t], None
+    g = rng("alloc-fails")
+    A = to_dev(g.integers(-2, 3, (120, 4096)).astype(np.float16))
+    B = to_dev(g.integers(-2, 3, (4096, 4096)).astype(np.float16))
+    ref, ref_long = empty_f16(120, 4096), empty_f16(2, 4096)
+    cg.gemm_fp16(A, B, ref, 120, 4096, 1024)
+    cg.gemm_fp16(A, B, ref_long, 2, 4096, 4096)
+    torch.cuda.synchronize()
+    C, C_long = empty_f16(120, 4096, fill=float("nan")), empty_f16(2, 4096, fill=float("nan"))
+    stream = torch.cuda.Stream()  # no scratch of its own yet
+    stream.wait_stream(torch.cuda.current_stream())
+    excess(1 << 50)
+    try:
+        with torch.cuda.stream(stream):
+            cg.gemm_fp16(A, B, C, 120, 4096, 1024)
+            with pytest.raises(cg.CloveError) as e:
+                cg.gemm_fp16(A, B, C_long, 2, 4096, 4096)
+    finally:
+        excess(0)
+    assert e.value.status == _lib.CLOVE_ERR_OUT_OF_MEMORY
+    torch.cuda.synchronize()
+    assert np.array_equal(f16bits(to_host(C)), f16bits(to_host(ref)))
+    assert torch.isnan(C_long).all().item()
+    with torch.cuda.stream(stream):
+        cg.gemm_fp16(A, B, C_long, 2, 4096, 4096)
+    torch.cuda.synchronize()
+    assert np.array_equal(f16bits(to_host(C_long)), f16bits(to_host(ref_long)))
