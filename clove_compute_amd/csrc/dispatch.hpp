@@ -25,20 +25,24 @@ struct Scratch {
 // current device (implemented in capi.hip): library-owned, or carved from the
 // workspace the calling thread has bound (clove_workspace_bind), or, in a
 // workspace size query, a placeholder that only records the size.
-// `optional`: the caller can do without; during a stream capture the library's
-// scratch is then not grown (an allocation can end the capture) and the call
-// returns CLOVE_ERR_OUT_OF_MEMORY.
+// `optional`: the call has an ordinary plan without scratch (another kernel, or
+// runs_unsplit); during a stream capture the library's scratch is then not
+// grown (an allocation can end the capture) and CLOVE_ERR_OUT_OF_MEMORY is
+// returned.  Every other call allocates there, which a capture in relaxed mode
+// allows: a long product recorded without its split would be slower at every
+// replay, with nothing to say so.
 clove_status_t acquire_scratch(hipStream_t stream, size_t partial_bytes, size_t num_counters,
                                Scratch* out, bool optional = false);
 
-// Whether a call whose acquire_scratch returned `st` may go on without a K
-// split: the library's own scratch could not grow (the stream is being
-// captured, or memory is short), or the bound workspace is too small and the
-// plan without a split is an ordinary one for the shape (`few`: small products,
-// which need no workspace to run).
-inline bool scratch_optional(clove_status_t st, bool few) {
-    return st == CLOVE_ERR_OUT_OF_MEMORY || (st == CLOVE_ERR_WORKSPACE && few);
+// acquire_scratch (or a launch that asked it) had too little: the library's own
+// scratch could not grow, or the bound workspace is too small
+inline bool scratch_short(clove_status_t st) {
+    return st == CLOVE_ERR_OUT_OF_MEMORY || st == CLOVE_ERR_WORKSPACE;
 }
+
+// Whether an FP16 or INT8 product runs without its K split where scratch is
+// short: up to 16 K tiles of bk, whose split saves little
+inline bool runs_unsplit(int K, int bk) { return K <= 16 * bk; }
 
 // True while the calling thread runs a workspace size query: calls plan and
 // size their scratch but launch nothing.

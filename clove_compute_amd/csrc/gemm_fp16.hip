@@ -318,7 +318,7 @@ clove_status_t run_dma(const uint16_t* A, const uint16_t* B, uint16_t* C, int ba
 }
 
 template <int MM, bool SWIGLU = false, bool UA = false>
-clove_status_t run_gemv(GemvParams p, int batch, hipStream_t stream) {
+clove_status_t run_gemv(GemvParams p, int batch, hipStream_t stream, bool optional = false) {
     p.col_blocks = cdiv(p.N, SWIGLU ? GV_COLS / 2 : GV_COLS);
     p.nsplit = cdiv(p.K, GV_ROWS);
     const int tiles = p.col_blocks * batch;
@@ -327,7 +327,7 @@ clove_status_t run_gemv(GemvParams p, int batch, hipStream_t stream) {
     if (p.nsplit > 1) {
         Scratch s;
         const size_t bytes = (size_t)tiles * p.nsplit * MM * GV_COLS * sizeof(float);
-        clove_status_t st = acquire_scratch(stream, bytes, (size_t)tiles, &s, UA);
+        clove_status_t st = acquire_scratch(stream, bytes, (size_t)tiles, &s, optional);
         if (st != CLOVE_OK) return st;
         p.ws = s.partials;
         p.counters = s.counters;
@@ -388,9 +388,10 @@ clove_status_t launch_gemm_fp16(const uint16_t* A, const uint16_t* B, uint16_t* 
     // call
     if (N >= 8 && M <= 2 && K > 0) {
         GemvParams g{A, B, C, nullptr, M, N, K, alpha, beta, sA, sB, sC, 0, 1, nullptr, nullptr};
-        const clove_status_t gst =
-            M == 1 ? run_gemv<1, false, true>(g, batch, stream) : run_gemv<2, false, true>(g, batch, stream);
-        if (gst != CLOVE_ERR_OUT_OF_MEMORY && gst != CLOVE_ERR_WORKSPACE) return gst;
+        const bool unsplit = runs_unsplit(K, 64);
+        const clove_status_t gst = M == 1 ? run_gemv<1, false, true>(g, batch, stream, unsplit)
+                                          : run_gemv<2, false, true>(g, batch, stream, unsplit);
+        if (!scratch_short(gst)) return gst;
     }
     Params p{};
     p.a = A; p.b = B; p.c = C;

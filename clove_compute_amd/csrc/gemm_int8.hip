@@ -524,7 +524,7 @@ __global__ void __launch_bounds__(1024) int8_gemv(I8Params p, int col_blocks) {
 namespace {
 
 template <int OUT, bool UA = false>
-clove_status_t run_gemv(I8Params p, hipStream_t stream) {
+clove_status_t run_gemv(I8Params p, hipStream_t stream, bool optional = false) {
     const int mm = p.M == 1 ? 1 : (p.M == 2 ? 2 : 4);
     const int rows = kIvRows;
     const int IV_COLS = kIvCols;
@@ -539,11 +539,12 @@ clove_status_t run_gemv(I8Params p, hipStream_t stream) {
         // whose counter region is smaller takes the partial-tile reduction
         Scratch s;
         clove_status_t st = CLOVE_ERR_WORKSPACE;
-        if (p.nsplit < 65536) st = acquire_scratch(stream, 0, (size_t)col_blocks * mm * IV_COLS * 2, &s, UA);
+        if (p.nsplit < 65536) st = acquire_scratch(stream, 0, (size_t)col_blocks * mm * IV_COLS * 2, &s, optional);
         if (st == CLOVE_OK) {
             p.counters = s.counters;
         } else if (st == CLOVE_ERR_WORKSPACE) {
-            st = acquire_scratch(stream, (size_t)col_blocks * p.nsplit * mm * IV_COLS * 4, (size_t)col_blocks, &s, UA);
+            st = acquire_scratch(stream, (size_t)col_blocks * p.nsplit * mm * IV_COLS * 4, (size_t)col_blocks, &s,
+                                 optional);
             if (st != CLOVE_OK) return st;
             p.ws = s.partials;
             p.counters = s.counters;
@@ -677,13 +678,14 @@ clove_status_t launch_gemm_int8(const Int8Args& a, hipStream_t stream) {
     const int64_t nk = (int64_t)a.N * a.K;
     if (!gemv && (a.M <= 2 || (a.M <= 4 && nk >= ((int64_t)1 << 19) && nk <= ((int64_t)12 << 20))) && a.K > 0 &&
         a.N >= 16) {
+        const bool unsplit = runs_unsplit(a.K, 128);
         clove_status_t gst = CLOVE_ERR_INVALID_ARG;
         switch (a.out) {
-            case Int8Out::kHalfPerTensor: gst = run_gemv<(int)Int8Out::kHalfPerTensor, true>(p, stream); break;
-            case Int8Out::kHalfRowCol: gst = run_gemv<(int)Int8Out::kHalfRowCol, true>(p, stream); break;
-            case Int8Out::kAcc32: gst = run_gemv<(int)Int8Out::kAcc32, true>(p, stream); break;
+            case Int8Out::kHalfPerTensor: gst = run_gemv<(int)Int8Out::kHalfPerTensor, true>(p, stream, unsplit); break;
+            case Int8Out::kHalfRowCol: gst = run_gemv<(int)Int8Out::kHalfRowCol, true>(p, stream, unsplit); break;
+            case Int8Out::kAcc32: gst = run_gemv<(int)Int8Out::kAcc32, true>(p, stream, unsplit); break;
         }
-        if (gst != CLOVE_ERR_OUT_OF_MEMORY && gst != CLOVE_ERR_WORKSPACE) return gst;
+        if (!scratch_short(gst)) return gst;
     }
     // the skinny kernel for the rest, except (M > 2048, zero points 0, whole K
     // tiles) where the register-staged 256x256 tiles are ahead

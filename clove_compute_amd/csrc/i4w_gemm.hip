@@ -67,7 +67,9 @@ Plan make_plan(int R, int C, int G, int cus, int target, int min_groups) {
 }
 
 // `prep(args, extra)` runs before the GEMM with `extra_bytes` of scratch
-// (after the split-K partials) and may point args.X / args.xs into it
+// (after the split-K partials) and may point args.X / args.xs into it.
+// Where scratch is short, short K, and grids that cover 3/8 of the CUs with
+// 128-row tiles of few columns, run unsplit.
 template <class CF, bool XS, int OUT, class Prep>
 clove_status_t run(Args a, int cus, int target, int min_groups, size_t extra_bytes, hipStream_t stream,
                    Prep prep) {
@@ -83,8 +85,11 @@ clove_status_t run(Args a, int cus, int target, int min_groups, size_t extra_byt
     char* extra = nullptr;
     if (part_bytes + extra_bytes > 0) {
         Scratch s;
-        const clove_status_t st = acquire_scratch(stream, part_bytes + extra_bytes, (size_t)tiles, &s, extra_bytes == 0);
-        if (extra_bytes == 0 && scratch_optional(st, a.C <= 32 || a.G < 16)) {
+        const bool unsplit = extra_bytes == 0 &&
+                             (a.C <= 32 ? a.G < 20 || 4 * cdiv(OUT == 2 ? 2 * a.R : a.R, 64) >= 3 * cus : a.G < 16);
+        const clove_status_t st =
+            acquire_scratch(stream, part_bytes + extra_bytes, (size_t)tiles, &s, unsplit);
+        if (unsplit && scratch_short(st)) {
             a.nsplit = 1;
             a.gps = a.G;
         } else if (st != CLOVE_OK) {

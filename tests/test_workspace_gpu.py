@@ -272,3 +272,81 @@ def test_failed_scratch_allocation_leaves_no_error():
         cg.gemm_fp16(A, B, C_long, 2, 4096, 4096)
     torch.cuda.synchronize()
     assert np.array_equal(f16bits(to_host(C_long)), f16bits(to_host(ref_long)))
+
+
+def _exact_call(kind, M, N, K):
+    """A call on small integers (exact in any order of the sums) and its output shape."""
+    import torch
+    cg = _cg()
+    g = rng("scratch-short", kind, M, N, K)
+    G = (K + 127) // 128
+
+    def const(r, c, v):
+        return torch.full((r, c), v, dtype=torch.float16, device="cuda")
+    if kind == "fp16":
+        A, B = (to_dev(g.integers(-2, 3, s).astype(np.float16)) for s in ((M, K), (K, N)))
+        return lambda C: cg.gemm_fp16(A, B, C, M, N, K)
+    if kind == "int8":
+        A, B = (to_dev(g.integers(-9, 10, s).astype(np.int8)) for s in ((M, K), (K, N)))
+        return lambda C: cg.gemm_int8(A, B, C, M, N, K, 0.01, 0, 0.02, 0)
+    if kind == "int4":
+        A, B = (to_dev(g.integers(0, 256, s).astype(np.uint8)) for s in ((M, K // 2), (K, (N + 1) // 2)))
+        sA, zA, sB, zB = const(M, G, 2.0 ** -6), const(M, G, 8.0), const(G, N, 2.0 ** -4), const(G, N, 7.0)
+        return lambda C: cg.gemm_int4(A, sA, zA, B, sB, zB, C, M, N, K)
+    R = 2 * N if kind == "w4a16_swiglu" else N
+    X = to_dev(g.integers(-2, 3, (M, K)).astype(np.float16))
+    W = to_dev(g.integers(0, 256, (R, K // 2)).astype(np.uint8))
+    s, z = const(R, G, 2.0 ** -8), const(R, G, 8.0)
+    if kind == "w4a16_swiglu":
+        return lambda C: cg.w4a16_swiglu(X, W, s, z, C, M, N, K)
+    return lambda C: cg.gemm_w4a16(X, W, s, z, C, M, N, K)
+
+
+# longer products keep their K split or say that scratch is missing: with a
+# bound workspace of the least size nothing runs
+@pytest.mark.parametrize("kind,M,N,K", [("fp16", 32, 4096, 4096), ("fp16", 2, 4096, 4096), ("int8", 128, 2048, 4096),
+                                        ("w4a16", 32, 1024, 11008), ("int4", 300, 40, 4226)])
+def test_long_products_report_missing_scratch(kind, M, N, K):
+    import torch
+    cg = _cg()
+    run = _exact_call(kind, M, N, K)
+    C = empty_f16(M, N, fill=float("nan"))
+    cg.workspace_bind(_zeros_ws(65536))
+    try:
+        with pytest.raises(cg.CloveError) as e:
+            run(C)
+        assert e.value.status == cg.CLOVE_ERR_WORKSPACE
+        torch.cuda.synchronize()
+    finally:
+        cg.workspace_bind()
+    assert torch.isnan(C).all().item()
+
+
+# a first call inside a capture that allows allocations records the split plan:
+# the replay has the eager call's bits (fp32 sums in another order differ)
+@pytest.mark.parametrize("kind,M,N,K", [("fp16", 32, 4096, 4096), ("w4a16", 32, 1024, 11008)])
+def test_long_products_keep_their_split_in_a_capture(kind, M, N, K):
+    import torch
+    cg = _cg()
+    g = rng("capture-split", M, N, K)
+    A = to_dev(g.standard_normal((M, K)).astype(np.float16))
+    if kind == "fp16":
+        B = to_dev((g.standard_normal((K, N)) * 0.02).astype(np.float16))
+        run = lambda C: cg.gemm_fp16(A, B, C, M, N, K)  # noqa: E731
+    else:
+        W = to_dev(g.integers(0, 256, (N, K // 2)).astype(np.uint8))
+        s = to_dev(g.uniform(0.001, 0.02, (N, K // 128)).astype(np.float16))
+        z = to_dev(g.integers(0, 16, (N, K // 128)).astype(np.float16))
+        run = lambda C: cg.gemm_w4a16(A, W, s, z, C, M, N, K)  # noqa: E731
+    ref, C = empty_f16(M, N), empty_f16(M, N, fill=float("nan"))
+    run(ref)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream(), capture_error_mode="relaxed"):
+        run(C)
+    for _ in range(3):
+        C.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(f16bits(to_host(C)), f16bits(to_host(ref)))
+        _ = (A.float() @ A.float().T).sum().item()  # eager work between replays
