@@ -8,6 +8,7 @@
 #include <cstdint>
 
 #include "clove/gemm_c.h"
+#include "common.hpp"
 
 namespace clove {
 
@@ -25,8 +26,8 @@ struct Scratch {
 // current device (implemented in capi.hip): library-owned, or carved from the
 // workspace the calling thread has bound (clove_workspace_bind), or, in a
 // workspace size query, a placeholder that only records the size.
-// `optional`: the call has an ordinary plan without scratch (another kernel, or
-// runs_unsplit); during a stream capture the library's scratch is then not
+// `optional`: the call has an ordinary plan without scratch (runs_unsplit, or
+// another kernel); during a stream capture the library's scratch is then not
 // grown (an allocation can end the capture) and CLOVE_ERR_OUT_OF_MEMORY is
 // returned.  Every other call allocates there, which a capture in relaxed mode
 // allows: a long product recorded without its split would be slower at every
@@ -41,8 +42,12 @@ inline bool scratch_short(clove_status_t st) {
 }
 
 // Whether an FP16 or INT8 product runs without its K split where scratch is
-// short: up to 16 K tiles of bk, whose split saves little
-inline bool runs_unsplit(int K, int bk) { return K <= 16 * bk; }
+// short: up to 16 K tiles of bk, whose split saves little, or (`any_k`: operands
+// that are not whole K tiles or not aligned) 64 x 64 tiles that cover the CUs --
+// the products whose plan on the generic MFMA kernel has no split either.
+inline bool runs_unsplit(bool any_k, int batch, int M, int N, int K, int bk, int cus) {
+    return hw::cdiv(K, bk) <= 16 || (any_k && (int64_t)hw::cdiv(M, 64) * hw::cdiv(N, 64) * batch >= cus);
+}
 
 // True while the calling thread runs a workspace size query: calls plan and
 // size their scratch but launch nothing.

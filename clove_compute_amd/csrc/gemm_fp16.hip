@@ -374,21 +374,24 @@ clove_status_t launch_gemm_fp16(const uint16_t* A, const uint16_t* B, uint16_t* 
         clove_status_t st2;
         if (try_skinny_fp16(A, B, C, batch, M, N, K, alpha, beta, dev.num_cus, stream, &st2)) return st2;
     }
-    // (the GEMV reads A element by element: any K and any alignment of A and C)
+    // (the GEMV reads A element by element: any K and any alignment of A and C;
+    // with those and too little scratch the MFMA kernel takes the call)
+    const bool unsplit = runs_unsplit(true, batch, M, N, K, 64, dev.num_cus);
     if (aligned16(B) && N % 8 == 0 && M <= 4 && K > 0) {
         GemvParams g{A, B, C, nullptr, M, N, K, alpha, beta, sA, sB, sC, 0, 1, nullptr, nullptr};
-        if (M == 1) return run_gemv<1>(g, batch, stream);
-        if (M == 2) return run_gemv<2>(g, batch, stream);
-        return run_gemv<4>(g, batch, stream);
+        const bool opt = !aligned && unsplit;
+        const clove_status_t gst = M == 1   ? run_gemv<1>(g, batch, stream, opt)
+                                   : M == 2 ? run_gemv<2>(g, batch, stream, opt)
+                                            : run_gemv<4>(g, batch, stream, opt);
+        if (aligned || !scratch_short(gst)) return gst;
     }
     // rows of B at any alignment, up to two rows of A (us per call against the
     // MFMA kernel: 1 x 2422 x 818 9.1 -> 5.6, 1 x 9001 x 1100 13.7 -> 9.2, 2 x 2422 x
     // 818 9.7 -> 6.8, 2 x 4097 x 4096 15.7 -> 15.6; at three rows it loses, 3 x 300 x
     // 300 5.7 -> 8.8); without scratch for the K splits the MFMA kernel takes the
     // call
-    if (N >= 8 && M <= 2 && K > 0) {
+    else if (N >= 8 && M <= 2 && K > 0) {
         GemvParams g{A, B, C, nullptr, M, N, K, alpha, beta, sA, sB, sC, 0, 1, nullptr, nullptr};
-        const bool unsplit = runs_unsplit(K, 64);
         const clove_status_t gst = M == 1 ? run_gemv<1, false, true>(g, batch, stream, unsplit)
                                           : run_gemv<2, false, true>(g, batch, stream, unsplit);
         if (!scratch_short(gst)) return gst;

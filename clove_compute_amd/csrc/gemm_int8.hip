@@ -662,12 +662,17 @@ clove_status_t launch_gemm_int8(const Int8Args& a, hipStream_t stream) {
     // 11008, M = 3 / 4: 13.9 / 17.1 us there against 21.7 / 20.5 us on the
     // GEMV; at 4096 x 4096 the GEMV is ahead, 9.2 against 11.5 us)
     const bool gemv = a.M <= 4 && a.K > 0 && a.N >= 16 && a.N % 16 == 0 && aligned16(a.B);
+    // (without scratch, with K or A unaligned, the skinny kernel takes the call)
+    const bool unsplit = runs_unsplit(true, 1, a.M, a.N, a.K, 128, dev.num_cus);
     if (gemv && (a.M <= 2 || (int64_t)a.N * a.K <= ((int64_t)32 << 20))) {
+        const bool opt = !aligned && unsplit;
+        clove_status_t gst = CLOVE_ERR_INVALID_ARG;
         switch (a.out) {
-            case Int8Out::kHalfPerTensor: return run_gemv<(int)Int8Out::kHalfPerTensor>(p, stream);
-            case Int8Out::kHalfRowCol: return run_gemv<(int)Int8Out::kHalfRowCol>(p, stream);
-            case Int8Out::kAcc32: return run_gemv<(int)Int8Out::kAcc32>(p, stream);
+            case Int8Out::kHalfPerTensor: gst = run_gemv<(int)Int8Out::kHalfPerTensor>(p, stream, opt); break;
+            case Int8Out::kHalfRowCol: gst = run_gemv<(int)Int8Out::kHalfRowCol>(p, stream, opt); break;
+            case Int8Out::kAcc32: gst = run_gemv<(int)Int8Out::kAcc32>(p, stream, opt); break;
         }
+        if (aligned || !scratch_short(gst)) return gst;
     }
     // rows of B at any alignment: one or two rows of A, three or four on mid-size
     // weights (us per call against the skinny kernel: 1 x 1613 x 1472 11.1 -> 5.9, 1 x
@@ -678,7 +683,6 @@ clove_status_t launch_gemm_int8(const Int8Args& a, hipStream_t stream) {
     const int64_t nk = (int64_t)a.N * a.K;
     if (!gemv && (a.M <= 2 || (a.M <= 4 && nk >= ((int64_t)1 << 19) && nk <= ((int64_t)12 << 20))) && a.K > 0 &&
         a.N >= 16) {
-        const bool unsplit = runs_unsplit(a.K, 128);
         clove_status_t gst = CLOVE_ERR_INVALID_ARG;
         switch (a.out) {
             case Int8Out::kHalfPerTensor: gst = run_gemv<(int)Int8Out::kHalfPerTensor, true>(p, stream, unsplit); break;

@@ -37,7 +37,7 @@ namespace {
 
 // The shared body of the GEMM and the partials hook: plan, scratch, the Bt
 // pre-pass, the launch.  P != null selects the partials mode (scales unused).
-clove_status_t run(const Int4Args& q, int32_t* P, int cus, hipStream_t stream) {
+clove_status_t run(const Int4Args& q, int32_t* P, int cus, hipStream_t stream, bool optional = false) {
     const int G = cdiv(q.K, 128);
     const int Npad = cdiv(q.N, BC) * BC;
     Args a{};
@@ -70,7 +70,7 @@ clove_status_t run(const Int4Args& q, int32_t* P, int cus, hipStream_t stream) {
     const size_t bt_bytes = round256((size_t)Npad * G2 * 128);
     const size_t sb_bytes = round256((size_t)G2 * Npad * 4);
     Scratch s;
-    clove_status_t st = acquire_scratch(stream, part_bytes + bt_bytes + sb_bytes, (size_t)tiles, &s);
+    clove_status_t st = acquire_scratch(stream, part_bytes + bt_bytes + sb_bytes, (size_t)tiles, &s, optional);
     if (st != CLOVE_OK) return st;
     char* base = reinterpret_cast<char*>(s.partials);
     a.part = s.partials;
@@ -116,9 +116,15 @@ bool eligible_anyk(const Int4Args& q) {
 // -> 41, 8768 x 18 x 4240 207 -> 32, 1728 x 76 x 1534 30 -> 18.5).
 bool try_i4i4(const Int4Args& q, int cus, hipStream_t stream, clove_status_t* status) {
     if (q.mode != CLOVE_INT4_GROUPWISE) return false;
-    if (!(q.N >= 64 && eligible(q)) && !(q.K % 128 != 0 && eligible_anyk(q))) return false;
-    *status = run(q, nullptr, cus, stream);
-    return true;
+    if (q.N >= 64 && eligible(q)) {
+        *status = run(q, nullptr, cus, stream);
+        return true;
+    }
+    if (q.K % 128 == 0 || !eligible_anyk(q)) return false;
+    // without scratch for the Bt pass, the generic kernel, whose plan needs none
+    // where its 64 x 64 tiles cover the CUs or K is short
+    *status = run(q, nullptr, cus, stream, (int64_t)cdiv(q.M, 64) * cdiv(q.N, 64) >= cus || q.K < 512);
+    return !scratch_short(*status);
 }
 
 clove_status_t launch_i4i4_partials(const Int4Args& q, int32_t* P, int cus, hipStream_t stream) {

@@ -68,11 +68,12 @@ Plan make_plan(int R, int C, int G, int cus, int target, int min_groups) {
 
 // `prep(args, extra)` runs before the GEMM with `extra_bytes` of scratch
 // (after the split-K partials) and may point args.X / args.xs into it.
-// Where scratch is short, short K, and grids that cover 3/8 of the CUs with
-// 128-row tiles of few columns, run unsplit.
+// Where scratch is short: with `other` (the caller has another kernel, which
+// needs none) the status says so; else short K, and grids that cover 3/8 of the
+// CUs with 128-row tiles of few columns, run unsplit.
 template <class CF, bool XS, int OUT, class Prep>
 clove_status_t run(Args a, int cus, int target, int min_groups, size_t extra_bytes, hipStream_t stream,
-                   Prep prep) {
+                   Prep prep, bool other) {
     // OUT 2 (SwiGLU): a tile of BR weight rows makes BR/2 outputs
     const Plan pl = make_plan<CF>(OUT == 2 ? 2 * a.R : a.R, a.C, a.G, cus, target, min_groups);
     a.tiles_r = pl.tiles_r;
@@ -85,10 +86,10 @@ clove_status_t run(Args a, int cus, int target, int min_groups, size_t extra_byt
     char* extra = nullptr;
     if (part_bytes + extra_bytes > 0) {
         Scratch s;
-        const bool unsplit = extra_bytes == 0 &&
+        const bool unsplit = extra_bytes == 0 && !other &&
                              (a.C <= 32 ? a.G < 20 || 4 * cdiv(OUT == 2 ? 2 * a.R : a.R, 64) >= 3 * cus : a.G < 16);
         const clove_status_t st =
-            acquire_scratch(stream, part_bytes + extra_bytes, (size_t)tiles, &s, unsplit);
+            acquire_scratch(stream, part_bytes + extra_bytes, (size_t)tiles, &s, unsplit || other);
         if (unsplit && scratch_short(st)) {
             a.nsplit = 1;
             a.gps = a.G;
@@ -128,23 +129,23 @@ clove_status_t run(Args a, int cus, int target, int min_groups, size_t extra_byt
 //   128 with eight waves where those tiles cover 3/4 of the CUs, else 256 x 64
 // Splits keep at least 4 groups each (8 where two workgroups share a CU).
 template <bool XS, int OUT, class Prep>
-clove_status_t by_shape(const Args& a, int cus, size_t extra_bytes, hipStream_t stream, Prep prep) {
+clove_status_t by_shape(const Args& a, int cus, size_t extra_bytes, hipStream_t stream, Prep prep, bool other = false) {
     const int rows = OUT == 2 ? 2 * a.R : a.R;  // weight rows
     const int64_t t32 = (int64_t)cdiv(rows, CfgC32::BR) * cdiv(a.C, CfgC32::BC);
     if (a.C <= 32 || (t32 <= cus && t32 * a.G <= 16 * cus))
-        return run<CfgC32, XS, OUT>(a, cus, cus, a.G > 44 ? 8 : 4, extra_bytes, stream, prep);
+        return run<CfgC32, XS, OUT>(a, cus, cus, a.G > 44 ? 8 : 4, extra_bytes, stream, prep, other);
     if (8 * (int64_t)cdiv(rows, CfgC64::BR) * cdiv(a.C, CfgC64::BC) < 3 * cus)
-        return run<CfgC64S3, XS, OUT>(a, cus, cus, 4, extra_bytes, stream, prep);
+        return run<CfgC64S3, XS, OUT>(a, cus, cus, 4, extra_bytes, stream, prep, other);
     if (OUT == 2 && a.C >= 512) {
         if (4 * cdiv(rows, CfgS128::BR) * cdiv(a.C, CfgS128::BC) >= 3 * cus)
-            return run<CfgS128, XS, OUT>(a, cus, cus, 8, extra_bytes, stream, prep);
-        return run<CfgS64, XS, OUT>(a, cus, 2 * cus, 8, extra_bytes, stream, prep);
+            return run<CfgS128, XS, OUT>(a, cus, cus, 8, extra_bytes, stream, prep, other);
+        return run<CfgS64, XS, OUT>(a, cus, 2 * cus, 8, extra_bytes, stream, prep, other);
     }
     // (SwiGLU tiles pair gate and up rows: the same outputs take twice the
     // weight rows, so the big tile waits for twice the grid)
     if (cdiv(rows, CfgBig::BR) * cdiv(a.C, CfgBig::BC) >= (OUT == 2 ? 2 : 1) * cus)
-        return run<CfgBig, XS, OUT>(a, cus, cus, 8, extra_bytes, stream, prep);
-    return run<CfgC64, XS, OUT>(a, cus, 2 * cus, 8, extra_bytes, stream, prep);
+        return run<CfgBig, XS, OUT>(a, cus, cus, 8, extra_bytes, stream, prep, other);
+    return run<CfgC64, XS, OUT>(a, cus, 2 * cus, 8, extra_bytes, stream, prep, other);
 }
 
 bool fits31(int64_t bytes) { return bytes < ((int64_t)1 << 31); }
@@ -218,10 +219,12 @@ clove_status_t run_stream(const Args& a, int cus, hipStream_t stream) {
 // with two X fragments below ~128 KB and in one round (T = 24 on 2944 x 1664
 // 5.7 against 7.4; T = 32 on 4864 x 2304, 144 KB, 10.4 against 8.1; T = 20 on
 // 9216 x 1152, 90 KB in two rounds, 9.2 against 7.3).
+int stream_rounds(const Args& a, int cus) { return cdiv(cdiv(a.R, stream_two_rows(a, cus) ? 32 : 16), cus); }
+int64_t stream_bytes(const Args& a, int cus) { return (int64_t)a.C * a.K * 2 * stream_rounds(a, cus); }
+
 bool stream_ahead(const Args& a, int cus) {
-    const int64_t rounds = cdiv(cdiv(a.R, stream_two_rows(a, cus) ? 32 : 16), cus);
-    const int64_t bytes = (int64_t)a.C * a.K * 2 * rounds;
-    return a.C <= 16 ? bytes < 200 * 1024 : rounds == 1 && bytes < 128 * 1024;
+    const int64_t bytes = stream_bytes(a, cus);
+    return a.C <= 16 ? bytes < 200 * 1024 : stream_rounds(a, cus) == 1 && bytes < 128 * 1024;
 }
 
 }  // namespace
@@ -244,12 +247,17 @@ bool try_i4w_w4a16(const W4A16Args& w, int cus, hipStream_t stream, clove_status
     a.G = w.K / 128;
     a.alpha = w.alpha;
     a.beta = w.beta;
-    if (w.T <= 32 && a.G <= kStreamMaxGroups && stream_ahead(a, cus)) {
+    const bool streams = w.T <= 32 && a.G <= kStreamMaxGroups;
+    if (streams && stream_ahead(a, cus)) {
         *status = run_stream(a, cus, stream);
         return true;
     }
     if (w.T <= 4) return false;  // (the GEMV, outside the stream's domain)
-    *status = by_shape<false, 1>(a, cus, 0, stream, [](Args&, char*) { return CLOVE_OK; });
+    // without scratch for the K split, the stream while it reads up to 256 KB of X
+    // per CU (at most 1.4 times the split tiles' time there)
+    const bool other = streams && stream_bytes(a, cus) < 256 * 1024;
+    *status = by_shape<false, 1>(a, cus, 0, stream, [](Args&, char*) { return CLOVE_OK; }, other);
+    if (other && scratch_short(*status)) *status = run_stream(a, cus, stream);
     return true;
 }
 
@@ -268,7 +276,8 @@ bool try_i4w_w4a16_swiglu(const W4A16Args& w, int cus, hipStream_t stream, clove
     a.G = w.K / 128;
     a.alpha = 1.0f;
     a.beta = 0.0f;
-    *status = by_shape<false, 2>(a, cus, 0, stream, [](Args&, char*) { return CLOVE_OK; });
+    // (up to four tokens the caller has its GEMV)
+    *status = by_shape<false, 2>(a, cus, 0, stream, [](Args&, char*) { return CLOVE_OK; }, w.T <= 4);
     return true;
 }
 

@@ -83,7 +83,7 @@ clove_status_t run(Args a, int batch, int cus, hipStream_t stream, int kt_per = 
         Scratch s;
         const size_t bytes =
             (size_t)tiles * a.nsplit * CF::NT * CF::NB * CF::FM * CF::FN * (16 / CF::KW) * sizeof(float);
-        const bool unsplit = runs_unsplit(a.K, CF::BK);
+        const bool unsplit = runs_unsplit(FEED != kWhole, batch, a.M, a.N, a.K, CF::BK, cus);
         const clove_status_t st = acquire_scratch(stream, bytes, (size_t)tiles, &s, unsplit);
         if (unsplit && scratch_short(st)) {
             a.kps = nk * CF::BK;

@@ -566,8 +566,8 @@ clove_status_t launch_w4a16_swiglu(const W4A16Args& a, hipStream_t stream) {
     // 2560 T = 3 23.4 -> 14.0, 2 x 6528 x 2560 T = 4 16.3 -> 11.1; 2 x 2944 x
     // 1536, 8.6 Mi weights, stays: 6.2 against 7.9)
     if (a.T >= 3 && a.T <= 4 && (int64_t)2 * a.O * a.K >= ((int64_t)12 << 20) &&
-        try_i4w_w4a16_swiglu(a, dev.num_cus, stream, &st2))
-        return st2;
+        try_i4w_w4a16_swiglu(a, dev.num_cus, stream, &st2) && !scratch_short(st2))
+        return st2;  // (too little scratch for its K split: the GEMV needs none)
     if (a.T <= 4 && gemv_lds_bytes(tv, nch) <= kMaxGemvLds) {
         GemvParams p{a.X, a.W, a.scale, a.zero, a.Y, a.T, a.O, a.K, G, nch, 1.0f, 0.0f};
         const bool aligned = aligned16(a.W) && (a.K % 32 == 0);

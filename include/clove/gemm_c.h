@@ -250,8 +250,20 @@ clove_status_t clove_w4a16_swiglu(const void* X, const uint8_t* W_q, const void*
  *  - library scratch (the default): the per-(device, stream) buffers above;
  *  - a bound workspace, clove_workspace_bind(ptr, bytes): calls on this thread
  *    take their split-K partials, completion counters and intermediates from
- *    [ptr, ptr + bytes) and allocate nothing; a call that needs more returns
- *    CLOVE_ERR_WORKSPACE and launches nothing.  (No kernel uses private
+ *    [ptr, ptr + bytes) and allocate nothing.  With at least the queried size
+ *    a call's results are bit for bit those with library scratch.  A call
+ *    that needs more returns CLOVE_ERR_WORKSPACE and launches nothing, unless
+ *    it has an ordinary plan that takes none, which it then runs (the same
+ *    sums, fp32 ones in another order): FP16 products up to K = 1024 and INT8
+ *    up to K = 2048 on the skinny kernel without their K split, and with any K
+ *    where operands are unaligned or K is not a whole number of K tiles and
+ *    64 x 64 tiles cover the CUs; W4A16 with fewer than 16 groups (20 with up
+ *    to 32 tokens), or with up to 32 tokens on wide layers or within the
+ *    streaming kernel's reach; w4a16_swiglu at 3 or 4 tokens; INT4 with
+ *    K % 128 != 0.  The same calls run that way when the library's scratch
+ *    cannot grow: during a stream capture, where they do not try to, or when
+ *    memory is short; every other call allocates, or returns
+ *    CLOVE_ERR_OUT_OF_MEMORY.  (No kernel uses private
  *    scratch either, which the library build checks.)  ptr must be 256-byte aligned
  *    and bytes >= CLOVE_WORKSPACE_MIN_BYTES; the first CLOVE_WORKSPACE_MIN_BYTES
  *    (the counters) must be zero before the first call, and every call leaves

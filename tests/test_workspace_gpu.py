@@ -4,7 +4,8 @@ A size query plans the calls and launches nothing; with a bound workspace of
 the queried size every entry point gives bit-for-bit the results it gives with
 library scratch (same kernels, same split plan), allocates nothing (so it can
 be captured in a HIP graph), and a call that needs more than the workspace
-holds fails with CLOVE_ERR_WORKSPACE without writing its output.
+holds fails with CLOVE_ERR_WORKSPACE without writing its output, unless it has
+an ordinary plan without scratch (short K, another kernel), which then runs.
 """
 import numpy as np
 import pytest
@@ -300,6 +301,44 @@ def _exact_call(kind, M, N, K):
     if kind == "w4a16_swiglu":
         return lambda C: cg.w4a16_swiglu(X, W, s, z, C, M, N, K)
     return lambda C: cg.gemm_w4a16(X, W, s, z, C, M, N, K)
+
+
+# calls that have a plan without scratch (the generic MFMA kernel's, the GEMV's,
+# the streaming kernel's) run where scratch is short, also on kernels that want
+# some: INT4 with ragged K, FP16 and INT8 rows with K at odd alignments, W4A16
+# tokens the streaming kernel can take, the fused SwiGLU of three tokens
+@pytest.mark.parametrize("kind,M,N,K", [("int4", 4200, 250, 130), ("int4", 300, 40, 330), ("fp16", 3, 2056, 300),
+                                        ("fp16", 2, 2050, 700), ("fp16", 160, 8192, 4104), ("int8", 3, 4112, 300),
+                                        ("int8", 40, 16384, 4098), ("w4a16", 20, 2944, 4096), ("w4a16", 17, 12300, 2560),
+                                        ("w4a16_swiglu", 3, 2000, 3200)])
+def test_calls_with_a_plan_without_scratch(kind, M, N, K):
+    import torch
+    cg = _cg()
+    run = _exact_call(kind, M, N, K)
+    ref = empty_f16(M, N)
+    run(ref)
+    torch.cuda.synchronize()
+    with cg.workspace_query() as q:
+        run(ref)
+    assert q.bytes > 0  # its own plan takes some
+    C = empty_f16(M, N, fill=float("nan"))
+    cg.workspace_bind(_zeros_ws(65536))
+    try:
+        run(C)
+        torch.cuda.synchronize()
+    finally:
+        cg.workspace_bind()
+    assert np.array_equal(f16bits(to_host(C)), f16bits(to_host(ref)))
+    C = empty_f16(M, N, fill=float("nan"))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):  # no scratch on this stream yet
+        run(C)
+    for _ in range(3):
+        C.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(f16bits(to_host(C)), f16bits(to_host(ref)))
 
 
 # longer products keep their K split or say that scratch is missing: with a
