@@ -23,15 +23,11 @@ using F16M128 = Cfg<false, 128, 64, 4, 1, 4>;
 // against 33 us with 128x64)
 using F16T128 = Cfg<false, 128, 128, 2, 2, 3>;
 // few tiles: 64x64, 64 KB of LDS, so that two workgroups share a CU (505 x 2304
-// x 1088 14.6 -> 10.5 us against six stages; see pick_f16_tile)
+// x 1088 14.6 -> 10.5 us against six stages; see pick_f16_tile).  Four stages at
+// any K: with two, for K <= 512, 109 x 5376 x 512 took 8.6 us against 5.8
 using F16T64 = Cfg<false, 64, 64, 2, 2, 4>;
 // 72 KB of LDS, two workgroups per CU (see pick_f16_tile)
 using F16W128 = Cfg<false, 64, 128, 2, 2, 3>;
-// the same tile one stage ahead for K <= 512: every workgroup's first stage
-// then waits behind a smaller burst of the whole grid's prologue loads (512^3:
-// 5.5 -> 4.7 us; from K = 1024 the six stages are ahead, 1024^3 8.7 against
-// 13.2 us)
-using F16T64S2 = Cfg<false, 64, 64, 2, 2, 2>;
 // small products (short K, at most one 32x32 tile per CU): 32x32 tiles whose
 // four waves take one k-step of every K tile each, two stages ahead -- 4x the
 // workgroups of 64x64 tiles at a quarter of the operand bytes each (hot graph
@@ -42,7 +38,7 @@ using F16T64S2 = Cfg<false, 64, 64, 2, 2, 2>;
 // only ties or loses: 512 x 1024 x 512 5.27 -> 5.21, 1024 x 1024 x 512 5.81
 // -> 7.13)
 using F16K32 = Cfg<false, 32, 32, 1, 1, 3, 1, 4>;
-// up to 32 rows on moderate weights: 32x64 tiles, two k slices, 64 KB of LDS
+// up to 32 rows, small products: 32x64 tiles, two k slices, 64 KB of LDS
 using F16N64 = Cfg<false, 32, 64, 1, 2, 4, 1, 2>;
 using I8M32 = Cfg<true, 32, 128, 1, 4, 3>;
 using I8T64 = Cfg<true, 64, 64, 2, 2, 4>;
@@ -50,22 +46,24 @@ using I8W128 = Cfg<true, 64, 128, 2, 2, 3>;  // 72 KB LDS: two workgroups per CU
 using I8M128 = Cfg<true, 128, 64, 4, 1, 4>;
 using I8T128 = Cfg<true, 128, 128, 2, 2, 3>;
 
-// K tiles per split: split K until about one workgroup per CU, not with k
-// slices.  128-row tiles keep two K tiles per split and are not split for
+// K tiles per split: split K until about one workgroup per CU, not with four
+// k slices.  128-row tiles keep two K tiles per split and are not split for
 // short K (<= 16 K tiles), where the publish / count / reload tail costs more
 // than the shorter stream saves; the smaller tiles, whose tail is shorter,
-// keep four at any K (INT8 9 x 5633 x 2048 17.1 -> 12.0 us, 10 x 1228 x 1536
-// 12.1 -> 8.9; two a split measured slower on most), but FP16 32x128 tiles
-// split only past 15 (7 x 8057 x 1015 13.0 -> 11.5; 18 x 10496 x 896 7.9 ->
-// 8.9 in three splits).
+// keep four (two a split measured slower on most) and split INT8 at any K (9 x
+// 5633 x 2048 17.1 -> 12.0 us, 10 x 1228 x 1536 12.1 -> 8.9), FP16 past 13 K tiles
+// with 64-row tiles (101 x 960 x 576 6.1 in two splits, 5.5 unsplit; 221 x 6976 x
+// 832 7.6, 6.8; at 15 and 16 K tiles they tie; not unaligned operands, 32 x 166 x
+// 64 x 484 9.9 in two splits, 12.0 unsplit) and past 15 with 32x128 ones (7 x
+// 8057 x 1015 13.0 -> 11.5; 18 x 10496 x 896 7.9 -> 8.9 in three splits).
 template <class CF>
-int tiles_per_split(int M, int N, int K, int batch, int cus) {
+int tiles_per_split(int M, int N, int K, int batch, int cus, bool ua = false) {
     const int tiles = cdiv(M, CF::BM) * cdiv(N, CF::BN) * batch;
     const int nk = cdiv(K, CF::BK);
     int ns = tiles >= cus ? 1 : cus / tiles;
     ns = max(1, min(ns, nk / (CF::BM == 128 ? 2 : 4)));
     if ((CF::BM == 128 && nk <= 16) || CF::KW > 2) ns = 1;
-    if (!CF::I8 && CF::BM == 32 && nk <= 15) ns = 1;
+    if (!CF::I8 && nk <= (CF::BM == 32 ? 15 : ua ? 0 : 13)) ns = 1;
     return cdiv(nk, ns);
 }
 
@@ -76,7 +74,7 @@ clove_status_t run(Args a, int batch, int cus, hipStream_t stream, int kt_per = 
     a.batch = batch;
     const int tiles = a.tiles_m * a.tiles_n * batch;
     const int nk = cdiv(a.K, CF::BK);
-    if (kt_per == 0) kt_per = tiles_per_split<CF>(a.M, a.N, a.K, batch, cus);
+    if (kt_per == 0) kt_per = tiles_per_split<CF>(a.M, a.N, a.K, batch, cus, FEED == kUnaligned);
     a.kps = kt_per * CF::BK;
     a.nsplit = cdiv(nk, kt_per);
     if (a.nsplit > 1) {
@@ -113,20 +111,39 @@ F16Tile pick_f16_tile(int batch, int M, int N, int K, int cus) {
     const int nk = cdiv(K, F16T64::BK);
     const bool short_k = nk <= 16;
     const bool long_k = K >= 4096;
-    // (up to 24 K tiles: 25 x 4160 x 1152 8.7 -> 7.2 us, 55 x 3136 x 1280 9.8 ->
-    // 8.0 against 32x128; 9 x 7680 x 1856 only ties)
-    if (nk <= 24 && (int64_t)cdiv(M, F16K32::BM) * cdiv(N, F16K32::BN) * batch <= cus) return F16Tile::kK32;
-    // 64x64 tiles while the product is small, whatever its M: their time is
-    // about tiles x K tiles (cold, 120 shapes, us per call, against the tiles
-    // below: 94 x 1536 x 2752 15.4 -> 9.5, 547 x 640 x 5056 23.6 -> 15.3, 265 x
-    // 1344 x 4224 20.3 -> 15.5, 128 x 4096 x 4096 15.6 -> 13.9, 144 x 2624 x 4352
-    // 17.1 -> 16.1; past the line 166 x 2624 x 10368 29.1 -> 30.9, 128 x 4096 x
-    // 11008 30.8 -> 35.0, 559 x 4352 x 2688 29.3 -> 39.1).  Up to 32 rows half of
-    // such a tile is padding, and 32x128 takes over above 64 tiles (8 x 4096 x
-    // 4096 11.8 -> 10.8, but 10 x 8320 x 3584 13.7 -> 16.9).
+    // (from 17 K tiles on, tiles that split K are ahead: 26 x 896 x 1344 9.4 us with
+    // 32x32, 6.4 with 32x64; 50 x 576 x 1472 10.0 against 6.6 with 64x64)
+    if (nk <= 16 && (int64_t)cdiv(M, F16K32::BM) * cdiv(N, F16K32::BN) * batch <= cus) return F16Tile::kK32;
+    // 64x64 tiles (up to 32 rows, where half of such a tile is padding, 32x64) while
+    // the product is small, whatever its M: their time is about tiles x K tiles (us
+    // per call over operands that rotate past the Infinity Cache, 400 shapes,
+    // against the tiles below: 153 x 1280 x 6080 16.8 -> 13.0, 190 x 3712 x 1792 13.7
+    // -> 11.8, 249 x 3200 x 2048 14.1 -> 12.7, 20 x 12096 x 1600 11.4 -> 10.1).  Not
+    //  * past 28 tiles x K tiles a CU (182 x 4096 x 3008, 35 a CU, 19.4 against 17.1
+    //    with 128x64; 128 x 4096 x 4096, 32, 18.3 against 17.3, although with three
+    //    operand sets, which that cache holds, 13.4 against 15.1), 33 where there are
+    //    splits or a second round to balance it (141 x 9024 x 1216 14.5 against 22.0;
+    //    269 x 768 x 8256, 30, 14.9 against 26.1 with 128x128; 81 x 2944 x 6528, 37, 18.8
+    //    against 16.7);
+    //  * in a second round of the CUs (182 x 5888 x 1728, 276 tiles, 19.0 against
+    //    15.0) past 6 K tiles (314 x 5120 x 320 5.3 against 6.0), unless the 128x64
+    //    tiles take one too (32 x 159 x 320 x 512 8.7 against 13.2);
+    //  * past 32 K tiles where more than half the CUs have a tile, which leaves no
+    //    room for a split (123 x 4224 x 3520 19.5 against 15.9, 7 x 9984 x 2752 14.5
+    //    against 13.8), 40 where 128-row tiles would pad another 64 rows (166 x 2944 x
+    //    2560 14.6 against 15.8); the fused SwiGLU takes the same tiles and loses
+    //    earlier (70 x 5120 x 2304 23.4 against 19.9, 151 x 3072 x 3072 27.5 against 23.6);
+    //  * up to 32 rows of unaligned operands past 28 K tiles and 64 tiles (4 x 5723 x
+    //    4904 24.2 against 19.2).
     const int64_t t64 = (int64_t)cdiv(M, F16T64::BM) * cdiv(N, F16T64::BN) * batch;
-    if (M <= 32) return t64 <= cus / 4 ? F16Tile::kN64 : F16Tile::kM32;
-    if (M <= 64 || (t64 <= 2 * cus && t64 * nk <= 33 * cus)) return F16Tile::kT64;
+    const int64_t t128x64 = (int64_t)cdiv(M, F16M128::BM) * cdiv(N, F16M128::BN) * batch;
+    const bool pads = M > 64 && cdiv(M, 64) % 2 == 1;
+    const int rounds = M > 32 && (nk <= 6 || t128x64 > cus) ? 2 : 1;
+    const bool small = t64 <= rounds * cus && t64 * nk <= (2 * t64 < cus || t64 > cus ? 33 : 28) * cus &&
+                       (2 * t64 <= cus || nk <= (pads ? 40 : 32));
+    if (M <= 32)
+        return 4 * t64 <= cus || (small && (nk <= 28 || (K % 8 == 0 && N % 8 == 0))) ? F16Tile::kN64 : F16Tile::kM32;
+    if (M <= 64 || small) return F16Tile::kT64;
     // 128x128 tiles, split K when they are few: for M > 256 once they cover
     // half the CUs or K is long, for 128 < M <= 256 on long K and N >= 4096
     // (cold weights, against 64x64 tiles for M > 256 and 128x64 up to 256:
@@ -137,10 +154,12 @@ F16Tile pick_f16_tile(int batch, int M, int N, int K, int cus) {
         // 64x128 between them, two workgroups a CU: where the 128x128 grid is
         // too small but this one fills 3/4 of the CUs (334 x 4288 x 1664 20.4 ->
         // 16.7 us against 64x64, 333 x 5001 x 2050 31.9 -> 25.8), and for short
-        // K (1729 x 2752 x 704 23.4 -> 19.8 against 128x128; 559 x 4352 x 2688
-        // stays, 29.3 against 41.3)
+        // K up to 8 K tiles (16 x 962 x 448 x 128 13.4 -> 12.0 against 128x128) or where
+        // the 128x128 tiles take a second round (1729 x 2752 x 704 23.4 -> 19.8; in one
+        // round 359 x 8384 x 960 stays, 15.5 against 20.8, and with longer K 559 x 4352 x
+        // 2688, 29.3 against 41.3)
         const int64_t w64 = (int64_t)cdiv(M, F16W128::BM) * cdiv(N, F16W128::BN) * batch;
-        if (t128 >= cus / 2 ? short_k : !long_k && 4 * w64 >= 3 * cus) return F16Tile::kW128;
+        if (t128 >= cus / 2 ? short_k && (nk <= 8 || t128 > cus) : !long_k && 4 * w64 >= 3 * cus) return F16Tile::kW128;
         return (t128 >= cus / 2 || long_k) ? F16Tile::kT128 : F16Tile::kT64;
     }
     if (M > 128 && long_k && N >= 4096) return F16Tile::kT128;
@@ -151,9 +170,11 @@ F16Tile pick_f16_tile(int batch, int M, int N, int K, int cus) {
     // N = 8192, K = 2048 or N = 4096, K = 11008, where 128x64 stays ahead)
     if (M > 64 && M <= 128 && long_k && N >= 10240) return F16Tile::kT128;
     // short K with few 128-row tiles: 32-row tiles make 4x the workgroups
-    // without a split
-    const bool few = (int64_t)cdiv(M, F16M128::BM) * cdiv(N, F16M128::BN) * batch < cus / 2;
-    return short_k && few ? F16Tile::kM32 : F16Tile::kM128;
+    // without a split; with many tiles (batches of heads), 64x128, two workgroups a
+    // CU (64 x 199 x 960 x 96 29.2 -> 21 us, 16 x 158 x 1312 x 512 19.5 -> 16.1; the
+    // same times where the stores are the bound)
+    if (short_k && t64 > 2 * cus) return F16Tile::kW128;
+    return short_k && 2 * t128x64 < cus ? F16Tile::kM32 : F16Tile::kM128;
 }
 
 bool f16_domain(int batch, const void* A, const void* B, const void* C, int M, int N, int K) {
@@ -211,9 +232,7 @@ bool try_skinny_fp16(const uint16_t* A, const uint16_t* B, uint16_t* C, int batc
         case F16Tile::kM128: *status = go(F16M128{}); break;
         case F16Tile::kT128: *status = go(F16T128{}); break;
         case F16Tile::kW128: *status = go(F16W128{}); break;
-        case F16Tile::kT64:
-            *status = K <= 512 ? go(F16T64S2{}) : go(F16T64{});
-            break;
+        case F16Tile::kT64: *status = go(F16T64{}); break;
         case F16Tile::kK32: *status = go(F16K32{}); break;
     }
     return true;
