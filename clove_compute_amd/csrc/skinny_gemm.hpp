@@ -396,7 +396,37 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
             const unsigned st = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(stage * SB));
             stage_next = stage;
             stage = stage + 1 == S ? 0 : stage + 1;
-            compute(st, kbeg + t * BK);
+            if constexpr (I8) {
+                compute(st, kbeg + t * BK);
+            } else {
+                // (the same as compute, written out: through the closure the compiler
+                // schedules the 128x64 tiles' LDS reads around other waits, 128 x 4096 x
+                // 11008 33.4 against 32.9 us, 100 x 8192 x 4096 23.1 against 22.4; INT8 is
+                // ahead with it, 512 x 4096 x 4096 with a zero point 26.4 against 27.4)
+#pragma unroll
+                for (int ks = 0; ks < NKS; ++ks) {
+                    u32x4 af[FM];
+                    const unsigned ab = st + aoff[ks];
+#pragma unroll
+                    for (int j = 0; j < FM; ++j) af[j] = lds_read16(ab + 4096 * j);
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) {
+                        u32x4 bf[FN];
+#pragma unroll
+                        for (int i = 0; i < FN; ++i) {
+                            const u32x2 lo = lds_read_tr<I8>(st + b * CF::B_BYTES + boff[ks][0][i]);
+                            const u32x2 hi = lds_read_tr<I8>(st + b * CF::B_BYTES + boff[ks][1][i]);
+                            bf[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+                        }
+#pragma unroll
+                        for (int i = 0; i < FN; ++i)
+#pragma unroll
+                            for (int j = 0; j < FM; ++j)
+                                acc[b][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                    bitcast<f16x8>(bf[i]), bitcast<f16x8>(af[j]), acc[b][i][j], 0, 0, 0);
+                    }
+                }
+            }
         }
     } else {
         constexpr int P = CF::P;
