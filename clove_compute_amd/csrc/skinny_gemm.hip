@@ -50,8 +50,10 @@ using I8T128 = Cfg<true, 128, 128, 2, 2, 3>;
 // k slices.  128-row tiles keep two K tiles per split and are not split for
 // short K (<= 16 K tiles), where the publish / count / reload tail costs more
 // than the shorter stream saves; the smaller tiles, whose tail is shorter,
-// keep four (two a split measured slower on most) and split INT8 at any K (9 x
-// 5633 x 2048 17.1 -> 12.0 us, 10 x 1228 x 1536 12.1 -> 8.9), FP16 past 13 K tiles
+// keep four (two a split measured slower on most) and split INT8 past 9 K tiles
+// (9 x 5633 x 2048 17.1 -> 12.0 us, 10 x 1228 x 1536 12.1 -> 8.9; up to 9 250 x 1792 x
+// 1024 7.3 -> 6.4 unsplit, 28 x 12160 x 1024 7.6 -> 6.8; 32-row tiles past 13 where
+// they cover a quarter of the CUs, 9 x 12544 x 1408 8.1 -> 7.7), FP16 past 13 K tiles
 // with 64-row tiles (101 x 960 x 576 6.1 in two splits, 5.5 unsplit; 221 x 6976 x
 // 832 7.6, 6.8; at 15 and 16 K tiles they tie; not unaligned operands, 32 x 166 x
 // 64 x 484 9.9 in two splits, 12.0 unsplit) and past 15 with 32x128 ones (7 x
@@ -63,7 +65,8 @@ int tiles_per_split(int M, int N, int K, int batch, int cus, bool ua = false) {
     int ns = tiles >= cus ? 1 : cus / tiles;
     ns = max(1, min(ns, nk / (CF::BM == 128 ? 2 : 4)));
     if ((CF::BM == 128 && nk <= 16) || CF::KW > 2) ns = 1;
-    if (!CF::I8 && nk <= (CF::BM == 32 ? 15 : ua ? 0 : 13)) ns = 1;
+    const int unsplit = !CF::I8 ? (CF::BM == 32 ? 15 : 13) : CF::BM == 32 && 4 * tiles > cus ? 13 : 9;
+    if (nk <= unsplit && !(ua && (CF::I8 || CF::BM != 32))) ns = 1;
     return cdiv(nk, ns);
 }
 
@@ -308,39 +311,52 @@ bool try_skinny_int8(const Int8Args& q, int cus, hipStream_t stream, clove_statu
             if (!al) return run<CF, OUT, true, kUnaligned>(a, 1, cus, stream);
             return zp ? run<CF, OUT, true>(a, 1, cus, stream) : run<CF, OUT>(a, 1, cus, stream);
         };
-        // (us per call, cold, 130 shapes with and without zero points, aligned and
-        // not; "was": 32x128 in five stages up to M = 64, or 128 on weights up
-        // to 32 Mi, else 128x64)
+        // (us per call, 350 shapes over operands that rotate past the Infinity Cache
+        // unless three sets are named, which it holds; "was": 32x128 in five stages
+        // up to M = 64, or 128 on weights up to 32 Mi, else 128x64)
         const int64_t t64 = (int64_t)cdiv(q.M, I8T64::BM) * cdiv(q.N, I8T64::BN);
         const int64_t w64 = (int64_t)cdiv(q.M, I8W128::BM) * cdiv(q.N, I8W128::BN);
+        const int64_t t128x64 = (int64_t)cdiv(q.M, I8M128::BM) * cdiv(q.N, I8M128::BN);
         const int nk = cdiv(q.K, I8T64::BK);
         if (q.M <= 32) return go(I8M32{});
         // 64 rows: 64x128 tiles once 64x64 ones fill a quarter of the CUs over a
-        // longer K (39 x 13376 x 4736 28.8 -> 19.2, 62 x 4620 x 8512 28.7 -> 21.8),
-        // else 64x64 (34 x 6848 x 896 6.5 -> 5.3, 39 x 960 x 5376 12.4 -> 10.5)
-        if (q.M <= 64) return t64 > cus / 4 && nk > 16 ? go(I8W128{}) : go(I8T64{});
-        // small products, at any M: 64x64 (187 x 512 x 9728 19.8 -> 12.9, 509 x 512
-        // x 5376 16.9 -> 11.6, 128 x 4096 x 4096 11.2 -> 10.8, 613 x 2368 x 924 15.5
-        // -> 14.0; past the line 70 x 4224 x 4754 19.9 -> 23.7, 683 x 2432 x 3200
-        // 14.8 -> 18.2)
-        if (t64 <= 2 * cus && t64 * nk <= (q.M <= 128 ? 16 : 20) * cus) return go(I8T64{});
+        // longer K, 18 tiles x K tiles a CU (39 x 13376 x 4736, 30 a CU, 28.8 -> 19.2, 62
+        // x 4620 x 8512, 19, 28.7 -> 21.8, three sets; 56 x 7616 x 9984, 36, 27.0 with 64x64,
+        // 22.7; 42 x 4480 x 4736, 10, 11.8 with 64x64, 13.5), else 64x64 (34 x 6848 x 896
+        // 6.5 -> 5.3, 39 x 960 x 5376 12.4 -> 10.5, three sets)
+        if (q.M <= 64) return 4 * t64 > cus && t64 * nk > 18 * cus ? go(I8W128{}) : go(I8T64{});
+        // small products, at any M, in one round of the CUs (two where unaligned, 276 x
+        // 5703 x 498 12.7 against 16.1): 64x64 (187 x 512 x 9728
+        // 19.8 -> 12.9, 509 x 512 x 5376 16.9 -> 11.6, three sets; from 16 tiles x K
+        // tiles a CU, 20 from 129 rows, 70 x 4224 x 4754 19.9 -> 23.7, 683 x 2432 x
+        // 3200 14.8 -> 18.2, 128 x 4096 x 4096 14.1 -> 14.4; in a second round 245 x 5696 x 1152 9.2 -> 12.0, 132 x 6336
+        // x 1664 11.5 -> 14.5)
+        if (t64 <= (al ? 1 : 2) * cus && t64 * nk < (q.M <= 128 ? 16 : 20) * cus) return go(I8T64{});
         if (q.M <= 128) {
-            // 32-row tiles in one round on weights up to 32 Mi (past one round 82 x
-            // 10958 x 2634 36.1 -> 26.5 with 64x128), 128x128 on wide weights, as
-            // for FP16 (128 x 11008 x 4096 23.7 -> 20.5; 128 x 4096 x 11008 stays on
-            // 128x64)
+            // 32-row tiles in one round on weights up to 32 Mi, 128x128 on wide
+            // weights, as for FP16 (128 x 11008 x 4096 23.7 -> 20.5; 128 x 4096 x 11008
+            // stays on 128x64); unaligned past one round 64x128 (82 x 10958 x 2634 36.1
+            // -> 26.5), aligned 128x64 (75 x 12864 x 2816 14.9, with 64x128 18.8)
             const bool large_w = (int64_t)q.N * q.K > ((int64_t)32 << 20);
-            if (!large_w) return (int64_t)cdiv(q.M, I8M32::BM) * cdiv(q.N, I8M32::BN) <= cus ? go(I8M32{}) : go(I8W128{});
-            if (q.N >= 10240 && q.K >= 4096) return go(I8T128{});
+            if (!large_w && (int64_t)cdiv(q.M, I8M32::BM) * cdiv(q.N, I8M32::BN) <= cus) return go(I8M32{});
+            if (large_w && q.N >= 10240 && q.K >= 4096) return go(I8T128{});
+            return !al && !large_w ? go(I8W128{}) : go(I8M128{});
         }
-        // 64x128, two workgroups a CU, where that fills the chip (aligned: 134 x
-        // 9280 x 10368 98.9 -> 63.8, 577 x 4096 x 13952 120.8 -> 75.5, 986 x 2816 x
-        // 4224 43.2 -> 28.4, 1474 x 4480 x 8704 157.5 -> 103.6, 512 x 4096 x 4096
-        // 18.5 -> 17.6; with 135 tiles 1666 x 576 x 13440 39.3 -> 67.7; unaligned
-        // operands, whose K tiles go through registers, only tie).  Up to M = 2048
-        // this kernel is ahead of the register-staged MFMA GEMM; at M = 4096 it is
-        // not.
-        if (al && 4 * w64 >= 3 * cus) return go(I8W128{});
+        // 64x128, two workgroups a CU, where that fills the chip (aligned: 577 x 4096 x
+        // 13952 120.8 -> 75.5, 986 x 2816 x 4224 43.2 -> 28.4, 1474 x 4480 x 8704 157.5 ->
+        // 103.6, three sets, 512 x 4096 x 4096 22.9 -> 22.0; with 135 tiles 1666 x 576 x
+        // 13440 39.3 -> 67.7; unaligned operands, whose K tiles go through registers, only
+        // tie), unless it starts a second round that 128x64 does not (339 x 5440 x 2304
+        // 15.6 -> 20.7).  Up to 256 rows each B panel is read by as many 64-row tiles from
+        // HBM, and 128x64 stays (199 x 11328 x 4480 43.1 -> 48.6) unless it takes a second
+        // round and either pads another 64 rows (134 x 9280 x 10368 98.9 -> 63.8, three
+        // sets, 141 x 11200 x 1664 20.5 -> 13.4) or K is short (194 x 11008 x 1664 25.0 ->
+        // 17.1).  Up to M = 2048, and with ragged K beyond, this kernel is ahead of the
+        // register-staged MFMA GEMM (K % 128 != 0: 4096 x 4096 x 4112 163 -> 117, 2100 x
+        // 4096 x 1040 165 -> 27); with whole K tiles at M = 4096 it is not.
+        if (al && (q.M <= 256 ? (q.M <= 192 || nk <= 16) && t128x64 > cus
+                               : 4 * w64 >= 3 * cus && (w64 <= cus || t128x64 > cus)))
+            return go(I8W128{});
         return go(I8M128{});
     };
     switch (q.out) {
