@@ -25,6 +25,9 @@ using CfgC64S3 = Cfg<4, 1, 1, 2, 3>;
 // 128 x 32, three stages ahead (70 KB LDS: two workgroups per CU): few X rows
 // or few tiles, where a workgroup's chain of stages is the time
 using CfgC32 = Cfg<4, 1, 1, 1, 4>;
+// 64 x 32, two waves, for few tiles over a long K: half the partial tile that the
+// last workgroup of a tile adds up from every split
+using CfgC32H = Cfg<2, 1, 1, 1, 4>;
 // 256 x 64 (four waves of 64 x 64), one stage ahead (70 KB LDS: two workgroups
 // per CU): the fused gate/up + SwiGLU from 512 X rows up, where each wave's two
 // weight blocks (a gate and an up block per 32 outputs) share every X
@@ -111,17 +114,22 @@ clove_status_t run(Args a, int cus, int target, int min_groups, size_t extra_byt
     return check_launch();
 }
 
-// Tile choice by the number of X rows C (measured on MI355X, cold graph
-// replays, 130 W4A16 and 90 INT4 shapes; us per call):
+// Tile choice by the number of X rows C (us per call, 500 W4A16 and INT4 shapes,
+// weights that rotate past the Infinity Cache unless three sets are named):
 //   128 x 32 for C <= 32, and while these tiles fit the CUs once and tiles x
-//   groups stay under 16 a CU, where a stage's latency and not its MFMAs is the
-//   time (against 128 x 64: W4A16 T = 64 on 3072 x 2048 11.2 -> 8.0, 100 on
-//   2432 x 1920 13.9 -> 9.3, 427 on 1920 x 1536 12.7 -> 10.2; past it 140 on
-//   3328 x 7424, 130 tiles x 58 groups, 33.3 against 23.0; INT4 1216 x 55 x
-//   2560 18.7 -> 12.6).  For C <= 32 it replaced 64 x 32 tiles of two waves
-//   (fused SwiGLU 22016 x 4096 T = 16 26.0 -> 19.6, 16384 x 2048 11.4 -> 9.8)
-//   128 x 64 with two stages ahead while those tiles cover less than 3/8 of
-//   the CUs, split to one workgroup per CU
+//   groups stay under 12 a CU (16 up to 20 groups), where a stage's latency and not
+//   its MFMAs is the time (against 128 x 64, three sets: W4A16 T = 64 on 3072 x 2048
+//   11.2 -> 8.0, 100 on 2432 x 1920 13.9 -> 9.3, 427 on 1920 x 1536 12.7 -> 10.2; INT4
+//   1216 x 55 x 2560 18.7 -> 12.6; the fused SwiGLU of 63 on 6144 x 1920, 11 a CU, 17.6
+//   -> 12.4; T = 397 on 2304 x 2176, 15, 14.7 -> 13.1; past it INT4 8320 x 43 x 3584, 14,
+//   21.4 -> 26.3, W4A16 T = 45 on 5888 x 4480, 13, 14.6 -> 16.0).  For C <= 32 it
+//   replaced 64 x 32 tiles of two waves (fused SwiGLU 22016 x 4096 T = 16 26.0 ->
+//   19.6), which stay for few tiles over 40 groups or more (W4A16 T = 26 on 1536 x
+//   10368 13.9 -> 11.8, INT4 1600 x 16 x 12416 18.5 -> 16.9; 2944 x 7808, 23 tiles x 61
+//   groups, 13.2 -> 15.4)
+//   128 x 64 with two stages ahead while those tiles cover less than 1/3 of the
+//   CUs, split to one workgroup per CU (with two splits some CUs have none: 158 on
+//   3840 x 5632, 90 tiles, 22.0 -> 23.7, INT4 11456 x 36 x 12672 50.0 -> 54.2)
 //   otherwise 128 x 64 with two workgroups per CU, whose waves interleave
 //   VALU (unpack, fold) with MFMA -- ahead of 128 x 128 by 15-25 % on the
 //   INT4 N = 128 and W4A16 T = 512 shapes -- unless 256 x 128 tiles already
@@ -132,9 +140,13 @@ template <bool XS, int OUT, class Prep>
 clove_status_t by_shape(const Args& a, int cus, size_t extra_bytes, hipStream_t stream, Prep prep, bool other = false) {
     const int rows = OUT == 2 ? 2 * a.R : a.R;  // weight rows
     const int64_t t32 = (int64_t)cdiv(rows, CfgC32::BR) * cdiv(a.C, CfgC32::BC);
-    if (a.C <= 32 || (t32 <= cus && t32 * a.G <= 16 * cus))
+    if constexpr (OUT != 2) {
+        if (a.C <= 32 && a.G >= 40 && 10 * t32 <= cus && t32 * a.G <= 5 * cus)
+            return run<CfgC32H, XS, OUT>(a, cus, 3 * cus, 10, extra_bytes, stream, prep, other);
+    }
+    if (a.C <= 32 || (t32 <= cus && t32 * a.G <= (a.G <= 20 ? 16 : 12) * cus))
         return run<CfgC32, XS, OUT>(a, cus, cus, a.G > 44 ? 8 : 4, extra_bytes, stream, prep, other);
-    if (8 * (int64_t)cdiv(rows, CfgC64::BR) * cdiv(a.C, CfgC64::BC) < 3 * cus)
+    if (3 * (int64_t)cdiv(rows, CfgC64::BR) * cdiv(a.C, CfgC64::BC) < cus)
         return run<CfgC64S3, XS, OUT>(a, cus, cus, 4, extra_bytes, stream, prep, other);
     if (OUT == 2 && a.C >= 512) {
         if (4 * cdiv(rows, CfgS128::BR) * cdiv(a.C, CfgS128::BC) >= 3 * cus)
@@ -166,10 +178,14 @@ clove_status_t launch_stream(const Args& a, hipStream_t stream) {
 // of groups is most of a small product's time (cold, us per call, against the
 // fewest waves that hold K: W4A16 T = 13 on 8128 x 1280 6.9 -> 5.2, INT4 N =
 // 12 on 10496 x 1152 7.5 -> 5.8, N = 19 on 1984 x 1920 7.2 -> 5.4, N = 9 on
-// 3840 x 5760 9.0 -> 7.6).  For 17..32 groups INT4 takes 8 waves (N = 27 on
-// 7552 x 2304 9.2 -> 8.5 against 4), W4A16 4 (T = 19 on 3712 x 3584 the same;
-// four waves leave room for more workgroups); 33..44 groups stay on 4 (INT4 N
-// = 12 on 11840 x 4864 12.4 against 13.5).
+// 3840 x 5760 9.0 -> 7.6; three operand sets).  For 17..32 groups INT4 takes 8
+// waves (N = 27 on 7552 x 2304 9.2 -> 8.5 against 4), but 4 past 24 groups with
+// three weight fragments, whose eight waves' partial sums fill the LDS of a CU
+// (N = 16 on 11008 x 4096 8.7 against 9.0 us); W4A16 4 (T = 19 on 3712 x 3584 the
+// same; four waves leave room for more workgroups), or 2 of 11 groups up to 22
+// from 8 tokens on in one round of the CUs (T = 12 on 1664 x 2560 5.15 against
+// 5.45, 20 on 3840 x 2304 6.8 against 7.3); 33..44 groups stay on 4 (INT4 N = 12 on
+// 11840 x 4864 12.4 against 13.5).
 // (BIG_G = false: the caller never passes more than 64 groups, and the
 // 11-group, 8-slice variant is not instantiated)
 template <int WF, int XF, bool XS, int OUT, int RAWB = 0, bool BIG_G = true>
@@ -179,8 +195,15 @@ clove_status_t stream_by_k(const Args& a, hipStream_t stream) {
     if (G <= 16) return launch_stream<WF, XF, 4, 4, XS, OUT, RAWB>(a, stream);
     if constexpr (XS) {
         if (G <= 24) return launch_stream<WF, XF, 3, 8, XS, OUT, RAWB>(a, stream);
-        if (G <= 32) return launch_stream<WF, XF, 4, 8, XS, OUT, RAWB>(a, stream);
+        if constexpr (WF == 3) {
+            if (G <= 32) return launch_stream<WF, XF, 8, 4, XS, OUT, RAWB>(a, stream);
+        } else {
+            if (G <= 32) return launch_stream<WF, XF, 4, 8, XS, OUT, RAWB>(a, stream);
+        }
     } else {
+        if constexpr (WF == 1) {
+            if (G > 16 && G <= 22 && a.C >= 8) return launch_stream<WF, XF, 11, 2, XS, OUT, RAWB>(a, stream);
+        }
         if (G <= 24) return launch_stream<WF, XF, 6, 4, XS, OUT, RAWB>(a, stream);
         if (G <= 32) return launch_stream<WF, XF, 8, 4, XS, OUT, RAWB>(a, stream);
     }
@@ -326,10 +349,12 @@ bool try_i4w_int4(const Int4Args& q, int cus, hipStream_t stream, clove_status_t
 // 8192 x 4096 7.58 / 7.30 / 8.66, 16384 x 4096 12.06 / 11.17 / 14.40,
 // 4096 x 4096 5.52 / 6.87 / 8.29, 14336 x 2048 7.48 / 9.15 / 11.13, 11008 x
 // 2048 7.17 / 8.98 / 7.81: the rule picks the fastest of the three in each.
-int rawb_wf(int R, int G, int cus) {
+// (most: two with two column fragments, whose accumulators take the registers;
+// WF = 1 / 2 at N = 23: 8384 x 2944 11.2 / 13.8, 10816 x 3456 N = 25 15.1 / 18.4)
+int rawb_wf(int R, int G, int cus, int most) {
     int best = 1;
     int64_t best_rows = -1;
-    for (int wf = 1; wf <= 3; ++wf) {
+    for (int wf = 1; wf <= most; ++wf) {
         const int64_t rows = (int64_t)cdiv(cdiv(R, 16 * wf), cus) * wf;
         if (best_rows < 0 || rows < best_rows || (rows == best_rows && G > 16)) {
             best = wf;
@@ -345,8 +370,12 @@ bool try_i4w_int4_rawb(const Int4Args& q, int cus, hipStream_t stream, clove_sta
     if (q.mode != CLOVE_INT4_GROUPWISE || q.N < 3 || q.N > 32 || q.K <= 0 || q.K % 128 != 0 || !aligned16(q.A) ||
         !fits31((int64_t)q.M * (q.K / 2)))
         return false;
-    // (B and its constants stay in LDS whole)
+    // (B and its constants stay in LDS whole; two column fragments past 32 groups
+    // only in one round of 32-row workgroups: 8256 x 20 x 4352 24.2 against 19.0 us on
+    // the 128 x 32 tiles, 9856 x 22 x 4224 25.7 against 19.3; 7232 x 18 x 4608 13.7 against
+    // 18.1)
     if (G > (q.N <= 16 ? kStreamMaxGroups : kRawB2MaxGroups)) return false;
+    if (q.N > 16 && G > 32 && cdiv(q.M, 32) > cus) return false;
     Args a{};
     a.W = q.A;
     a.wscale = q.A_scale;
@@ -363,9 +392,9 @@ bool try_i4w_int4_rawb(const Int4Args& q, int cus, hipStream_t stream, clove_sta
     a.ldb = (q.N + 1) / 2;
     a.alpha = 1.0f;
     a.beta = 0.0f;
-    const int wf = rawb_wf(a.R, G, cus);
+    const int wf = rawb_wf(a.R, G, cus, q.N > 16 ? 2 : 3);
     if (q.N > 16) {
-        *status = wf >= 2 ? stream_by_k<2, 2, true, 0, 2, false>(a, stream) : stream_by_k<1, 2, true, 0, 2, false>(a, stream);
+        *status = wf == 2 ? stream_by_k<2, 2, true, 0, 2, false>(a, stream) : stream_by_k<1, 2, true, 0, 2, false>(a, stream);
         return true;
     }
     if (a.ldb == 8 && aligned16(q.B))
