@@ -367,7 +367,7 @@ int rawb_wf(int R, int G, int cus, int most) {
 bool try_i4w_int4_rawb(const Int4Args& q, int cus, hipStream_t stream, clove_status_t* status) {
     // up to 32 columns: B rows of at most 16 bytes, read in place (no transpose pass)
     const int G = q.K / 128;
-    if (q.mode != CLOVE_INT4_GROUPWISE || q.N < 3 || q.N > 32 || q.K <= 0 || q.K % 128 != 0 || !aligned16(q.A) ||
+    if (q.mode != CLOVE_INT4_GROUPWISE || q.N < 5 || q.N > 32 || q.K <= 0 || q.K % 128 != 0 || !aligned16(q.A) ||
         !fits31((int64_t)q.M * (q.K / 2)))
         return false;
     // (B and its constants stay in LDS whole; two column fragments past 32 groups

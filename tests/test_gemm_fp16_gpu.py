@@ -440,3 +440,23 @@ def test_few_rows_any_alignment_bit_exact(batch, M, N, K, off):
     got = to_host(C)
     assert np.array_equal(f16bits(got[off:off + exact.size]), f16bits(exact.reshape(-1)))
     assert np.all(np.isnan(got[:off])) and np.all(np.isnan(got[off + exact.size:]))  # nothing past the output
+
+
+# every tile of the unaligned form that the cases above leave out (64x128 at 333 x
+# 5001, 128x128, 128x64, 32x64 past 64 tiles, 64x64 in a second round) and the
+# aligned and ragged ones chosen by other sizes: 64x128 for batches of heads and
+# up to 8 K tiles, 32x64 up to one per CU, 64x64 unsplit up to 13 K tiles
+@pytest.mark.parametrize("batch,M,N,K", [(1, 333, 5001, 450), (1, 300, 2003, 4101), (1, 100, 5001, 2050), (1, 24, 5943, 1137),
+                                         (1, 161, 7573, 310), (3, 159, 320, 100), (16, 199, 2000, 96), (8, 259, 1792, 128),
+                                         (1, 20, 8000, 1600), (1, 7, 12000, 1024), (1, 101, 960, 576), (1, 314, 5120, 320)])
+def test_tile_rules_bit_exact(batch, M, N, K):
+    import torch
+    g = rng("tile-rules", batch, M, N, K)
+    A = to_dev(g.integers(-2, 3, (batch, M, K)).astype(np.float16))
+    B = to_dev(g.integers(-2, 3, (batch, K, N)).astype(np.float16))
+    C0 = g.integers(-8, 9, (batch, M, N)).astype(np.float16)
+    C = to_dev(C0)
+    _cg().gemm_fp16_batched(A, B, C, batch, M, N, K, 1.0, 0.5)
+    torch.cuda.synchronize()
+    exact = np.matmul(to_host(A).astype(np.float32), to_host(B).astype(np.float32)) + 0.5 * C0.astype(np.float32)
+    assert np.array_equal(f16bits(to_host(C)), f16bits(exact.astype(np.float16)))

@@ -183,14 +183,15 @@ def test_groupwise_stream_path_pow2_bit_exact():
     assert np.array_equal(f16bits(C), f16bits(ref.astype(np.float16)))
 
 
-# group-wise, 3..32 columns, K % 128 == 0: B read in place at any row length
-# (2..16 bytes) and alignment.  One and two column fragments, full and ragged,
-# one group, every K-slice count (G = 1, 17, 30, 44, 52, 88), one to three
-# weight fragments; the loads of the last rows are moved back inside B.
+# group-wise, 5..32 columns (up to 8 from 4 Mi weights on: fewer stay on the
+# GEMV), K % 128 == 0: B read in place at any row length (3..16 bytes) and
+# alignment.  One and two column fragments, full and ragged, one group, every
+# K-slice count (G = 1, 3, 16, 17, 30, 32, 44, 52, 88), one to three weight
+# fragments; the loads of the last rows are moved back inside B.
 @pytest.mark.parametrize("off", [0, 1])
-@pytest.mark.parametrize("M,N,K", [(33, 3, 128), (70, 4, 2176), (9000, 7, 2048), (300, 8, 6656), (20, 9, 11264),
+@pytest.mark.parametrize("M,N,K", [(33000, 5, 128), (1933, 6, 2176), (9000, 7, 2048), (650, 8, 6656), (20, 9, 11264),
                                    (11000, 13, 4096), (100, 16, 1024), (50, 17, 128), (8200, 18, 2176), (130, 25, 3840),
-                                   (70, 31, 5632), (40, 32, 5632)])
+                                   (8300, 23, 384), (70, 31, 5632), (40, 32, 5632)])
 def test_groupwise_raw_b_bit_exact(M, N, K, off):
     import torch
     A_q, sA, zA, B_q, sB, zB = make_case(M, N, K, "rawb", pow2=True, small=True)
@@ -205,15 +206,19 @@ def test_groupwise_raw_b_bit_exact(M, N, K, off):
 
 
 # up to 8 columns any zero point is exact: sums past 2^24 (|z| > 256) and
-# q - z past fp16's integers (|z| > 2048) are computed again in integers
+# q - z past fp16's integers (|z| > 2048) are computed again in integers.  From 4
+# Mi weights on, below which the GEMV takes them: a far zero point of A in two
+# rows' workgroups (the others unaffected), or one of B, in every workgroup
 @pytest.mark.parametrize("z", [256.0, 257.0, -300.0, 2051.0, -7000.0])
-@pytest.mark.parametrize("N,col", [(3, 1), (8, 7)])
-def test_groupwise_raw_b_far_zero_points(N, col, z):
-    M, K = 37, 512
+@pytest.mark.parametrize("far_b", [False, True])
+@pytest.mark.parametrize("N,col", [(5, 1), (8, 7)])
+def test_groupwise_raw_b_far_zero_points(N, col, far_b, z):
+    M, K = 8203, 512
     A_q, sA, zA, B_q, sB, zB = make_case(M, N, K, "far")
     zA[5, 2] = z
-    zB[3, col] = -z
     zA[M - 1, 0] = z
+    if far_b:
+        zB[3, col] = -z
     # every scale one power of two: the fold's products are exact, so each
     # result is one rounding per group of an exact integer sum
     sA[:] = np.float16(2.0 ** -8)
@@ -222,12 +227,23 @@ def test_groupwise_raw_b_far_zero_points(N, col, z):
         sA[:] = np.float16(2.0 ** -12)
         sB[:] = np.float16(2.0 ** -12)
     C = run_int4(A_q, sA, zA, B_q, sB, zB, M, N, K)
-    P = partials_int64(A_q, zA, B_q, zB, np.arange(M), N, K)  # [M, N, G]
-    acc = np.zeros((M, N), np.float32)
+    rows = np.unique(np.concatenate([np.arange(128), np.arange(4000, 4096), np.arange(M - 128, M)]))
+    P = partials_int64(A_q, zA, B_q, zB, rows, N, K)  # [rows, N, G]
+    acc = np.zeros((len(rows), N), np.float32)
     s = np.float32(sA[0, 0]) * np.float32(sB[0, 0])
     for g in range(K // 128):
         acc = (np.float64(s) * np.float32(P[:, :, g]).astype(np.float64) + acc).astype(np.float32)
-    assert np.array_equal(f16bits(C), f16bits(acc.astype(np.float16)))
+    assert np.array_equal(f16bits(C[rows]), f16bits(acc.astype(np.float16)))
+
+
+# few columns over a long K on few weight rows: 64 x 32 tiles in several K splits
+@pytest.mark.parametrize("M,N,K", [(300, 20, 6144), (1600, 16, 12416), (65, 32, 5760)])
+def test_groupwise_few_tiles_long_k_bit_exact(M, N, K):
+    A_q, sA, zA, B_q, sB, zB = make_case(M, N, K, "fewlong", pow2=True, small=True)
+    C = run_int4(A_q, sA, zA, B_q, sB, zB, M, N, K)
+    rows = np.arange(M) if M <= 512 else np.unique(np.concatenate([np.arange(64), np.arange(M - 64, M)]))
+    _, ref, _ = oracle.gemm_int4_groupwise(A_q[rows], sA[rows], zA[rows], B_q, sB, zB, len(rows), N, K)
+    assert np.array_equal(f16bits(C[rows]), f16bits(ref.astype(np.float16)))
 
 
 # group-wise with N >= 64 and K % 256 == 0: the int8-MFMA kernel (i4i4_gemm)

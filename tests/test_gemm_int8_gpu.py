@@ -284,3 +284,18 @@ def test_mid_tiles_bit_exact(M, N, K, za, zb):
     Cref, _ = oracle.gemm_int8_rowcol(A[rows], B, sa[rows], sb, za, zb)
     assert np.array_equal(run_acc32(A, B, za, zb)[rows], accref)
     assert np.array_equal(f16bits(to_host(C)[rows]), f16bits(Cref))
+
+
+# tiles of the rules by size that no case above takes: 64x128 up to 64 rows over a
+# longer K, at 129..192 rows that pad another 64 and at short K up to 256, 128x64 at
+# 65..128 rows past one round of 32x128 tiles, 64x64 and 32x128 unsplit
+@pytest.mark.parametrize("M,N,K,za,zb", [(40, 8192, 4736, 0, 0), (141, 11200, 256, 0, 0), (200, 8992, 384, -9, 0),
+                                         (100, 9008, 512, 0, 3), (250, 1792, 1024, 0, 0), (28, 12160, 1024, 3, -5),
+                                         (339, 5440, 256, 0, 0), (33, 1040, 2048, 0, 0)])
+def test_tile_rules_bit_exact(M, N, K, za, zb):
+    g = rng("tile-rules8", M, N, K)
+    A = g.integers(-128, 128, (M, K)).astype(np.int8)
+    B = g.integers(-128, 128, (K, N)).astype(np.int8)
+    rows = np.unique(np.concatenate([[0, M // 2, M - 1], g.integers(0, M, 12)]))
+    _, accref = oracle.gemm_int8(A[rows], B, np.float32(0.01), za, np.float32(0.02), zb)
+    assert np.array_equal(run_acc32(A, B, za, zb)[rows], accref)

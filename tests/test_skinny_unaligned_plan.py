@@ -34,7 +34,7 @@ def fast(buf, off):
 
 # (int8, BM, BN, P): the tiles of skinny_gemm.hip and their K tiles in registers
 TILES = [(False, 32, 128, 4), (False, 128, 64, 3), (False, 128, 128, 2), (False, 64, 64, 4), (False, 32, 32, 6),
-         (False, 32, 64, 4), (True, 32, 128, 4), (True, 128, 64, 3), (True, 128, 128, 2), (True, 64, 64, 4),
+         (False, 64, 128, 3), (False, 32, 64, 4), (True, 32, 128, 4), (True, 128, 64, 3), (True, 128, 128, 2), (True, 64, 64, 4),
          (True, 64, 128, 3)]
 
 

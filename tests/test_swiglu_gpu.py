@@ -126,8 +126,9 @@ def check_rows(X, Wq, s, z, H, rows):
     assert ok, rep
 
 
-# T <= 4: GEMV; T > 4 with K % 128 == 0: the MFMA GEMM (64x32 tiles up to 32
-# tokens, 128x64 / 256x128 above, with and without split K; from 512 tokens
+# T <= 4: GEMV (three or four tokens below 12 Mi weights); T > 4 with K % 128 ==
+# 0: the MFMA GEMM (128x32 tiles up to 32 tokens and while they are few, 128x64 /
+# 256x128 above, with and without split K; from 512 tokens
 # 256x64, or 256x128 with eight waves where those tiles cover 3/4 of the CUs:
 # the Llama-1B MLP at T = 512 and the ragged 1000 x 3000); the Llama-1B MLP
 # (I = 8192, K = 2048) at decode and prefill
@@ -140,6 +141,16 @@ def test_w4a16_swiglu_shapes(T, I, K):
     H = run_w4a16_swiglu(X, Wq, s, z, I)
     rows = np.unique(np.concatenate([[0, T - 1], g.integers(0, T, min(T, 8))]))
     check_rows(X, Wq, s, z, H, rows)
+    assert np.all(np.isfinite(H.astype(np.float32)))
+
+
+# three or four tokens from 12 Mi weights on: the MFMA GEMM, with and without
+# split K, whole and ragged O
+@pytest.mark.parametrize("T,I,K", [(3, 1640, 4096), (4, 3333, 2048), (3, 8192, 1024), (4, 13000, 512)])
+def test_w4a16_swiglu_few_tokens_large_weight(T, I, K):
+    X, Wq, s, z, g = make_gate_up(T, I, K, "few-large")
+    H = run_w4a16_swiglu(X, Wq, s, z, I)
+    check_rows(X, Wq, s, z, H, np.arange(T))
     assert np.all(np.isfinite(H.astype(np.float32)))
 
 
@@ -268,6 +279,16 @@ def test_swiglu_fused_equals_gemms_small_tiles(T, H, I):
 # stay on it
 @pytest.mark.parametrize("T,H,I", [(2, 4104, 11008), (3, 1000, 8192), (3, 4104, 4096), (4, 2056, 4096)])
 def test_swiglu_fused_equals_gemms_ragged_hidden(T, H, I):
+    test_swiglu_fused_equals_gemms_then_swiglu(T, H, I)
+
+
+# where the GEMMs take 64x128 tiles the fused call takes 64x64 (333 x 5000 x 1152)
+# or 128x128 (360 x 8192 x 512, 199 x 12000 x 512) unsplit; 32x64 tiles past a
+# quarter of the CUs, with and without a K split; 64x64 under two splits and in
+# one pass; 128x64 past 32 K tiles
+@pytest.mark.parametrize("T,H,I", [(333, 1152, 5000), (360, 512, 8192), (199, 512, 12000), (20, 1600, 8000), (7, 1024, 12000),
+                                   (12, 2560, 4096), (101, 576, 960), (100, 1024, 4096), (70, 2304, 5120)])
+def test_swiglu_fused_equals_gemms_other_tiles(T, H, I):
     test_swiglu_fused_equals_gemms_then_swiglu(T, H, I)
 
 

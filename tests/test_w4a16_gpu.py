@@ -136,3 +136,14 @@ def test_stream_path_pow2_bit_exact(T, O, K):
     Y = run(X, W, s, z, None, O)
     _, ref = oracle.w4a16(X, W, s, z)
     assert np.array_equal(f16bits(Y), f16bits(ref.astype(np.float16)))
+
+
+# two K slices of eleven groups (17..22 groups from 8 tokens on, one or two
+# column fragments) and 64 x 32 tiles over a long K on few rows, exact in any order
+@pytest.mark.parametrize("T,O,K", [(8, 40, 2176), (12, 300, 2432), (20, 200, 2816), (17, 300, 5120), (26, 1536, 10368)])
+def test_slice_and_tile_rules_pow2_bit_exact(T, O, K):
+    X, W, s, z, g = make(T, O, K, "rules", pow2=True)
+    X = np.clip(X, -1, 1)
+    Y = run(X, W, s, z, None, O)
+    _, ref = oracle.w4a16(X, W, s, z, None, 1.0, 0.0)
+    assert np.array_equal(f16bits(Y), f16bits(ref.astype(np.float16)))
