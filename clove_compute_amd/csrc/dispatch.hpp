@@ -132,8 +132,9 @@ clove_status_t launch_i4i4_partials(const Int4Args& args, int32_t* P, int num_cu
 bool try_i4w_w4a16_swiglu(const W4A16Args& args, int num_cus, hipStream_t stream, clove_status_t* status);
 
 // H [T, O] = swiglu(X @ gate^T, X @ up^T) on a fused gate/up W4A16 weight
-// (w4a16.hip): GEMV for T <= 4, the INT4-weight MFMA GEMM above, or, for shapes
-// neither covers, the two linear layers and the elementwise SwiGLU
+// (w4a16.hip): GEMV for T <= 2, and for T = 3, 4 below 12 Mi weights, the
+// INT4-weight MFMA GEMM above, or, for shapes neither covers, the two linear
+// layers and the elementwise SwiGLU
 clove_status_t launch_w4a16_swiglu(const W4A16Args& args, hipStream_t stream);
 // out[i] = swiglu(gate[i], up[i]), n elements (swiglu.hip)
 clove_status_t launch_swiglu(const uint16_t* gate, const uint16_t* up, uint16_t* out, int64_t n,
@@ -151,7 +152,7 @@ constexpr int kBufSwiglu = 1;  // gate / up intermediates of the unfused SwiGLU 
 // FP16 with up to four rows of A: the skinny MFMA kernel rather than the GEMV.
 // Large weights first (cold, us per call: 11008 x 4096 at M = 2 / 3 / 4 21.1 /
 // 21.3 / 21.0 against 26.5 / 32.2 / 31.8 on the GEMV).  Below that line its small
-// tiles: three or four rows always (3 x 2424 x 816 9.1 -> 5.9, 4 x 8192 x 576 9.8
+// tiles (three operand sets in turn, which the Infinity Cache holds): three or four rows always (3 x 2424 x 816 9.1 -> 5.9, 4 x 8192 x 576 9.8
 // -> 5.0, 4 x 1024 x 4096 10.1 -> 10.3, 64 heads of 4 x 320 x 64 both ways 17.1 ->
 // 7.2), one or two up to K = 640 (1 x 8192 x 576 6.7 -> 5.4, 2 x 2048 x 512 6.1 ->
 // 4.2, 64 heads of 1 x 320 x 64 11.0 -> 8.1; 1 x 2424 x 816 stays, 5.2 against 5.8).

@@ -548,8 +548,8 @@ template <int NV, int MODE>
 clove_status_t run_gemv(const GemvParams& p, bool aligned, int cus, hipStream_t stream) {
     const GemvShape g = gemv_shape(p.M, p.nch, cus, NV <= 2 ? 2 : 1);
     // Unaligned rows take the same shapes, with 16-byte loads at byte alignment
-    // (cold, us per call, against byte loads of one chunk a lane: 4096 x 11006 N =
-    // 1 / 4 28.3 -> 9.2 / 31.5 -> 15.3, 1418 x 6712 N = 2 12.3 -> 4.9), but one row
+    // (us per call, three operand sets in turn, which the Infinity Cache holds,
+    // against byte loads of one chunk a lane: 4096 x 11006 N = 1 / 4 28.3 -> 9.2 / 31.5 -> 15.3, 1418 x 6712 N = 2 12.3 -> 4.9), but one row
     // a wave with eight columns, whose registers would spill
     return aligned ? run_gemv_by_shape<NV, MODE, true>(p, g, stream) : run_gemv_by_shape<NV, MODE, false>(p, g, stream);
 }
@@ -641,7 +641,8 @@ clove_status_t launch_gemm_int4(const Int4Args& a, hipStream_t stream) {
     }
     // five to eight columns: B read in place by the INT4-weight streaming kernel,
     // whose MFMAs cost the same for 3 or 16 columns, where the GEMV's VALU work
-    // grows with them.  Cold, us per call, GEMV against stream: 11008 x 4096 N = 3
+    // grows with them.  us per call, three operand sets in turn, which the Infinity
+    // Cache holds, GEMV against stream: 11008 x 4096 N = 3
     // / 4 / 5 / 8 9.7 / 9.9 / 19.4 / 15.1 against 10.1 / 10.2 / 11.0 / 10.0,
     // 4096 x 11008 N = 4 / 5 / 8 12.2 / 29.9 / 20.8 against 12.6 / 12.1 / 10.7;
     // small weights stay (1280 x 1664 N = 8 5.2 against 6.2; 2048 x 5504 10.7

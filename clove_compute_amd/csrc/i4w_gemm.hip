@@ -19,8 +19,9 @@ using CfgBig = Cfg<4, 1, 2, 4, 3>;  // 256 x 128, 4 waves of 64 x 128
 // 125.6 -> 122.9 us, fused 114.9 -> 111.1 us against three stages)
 using CfgC64 = Cfg<4, 1, 1, 2, 2>;
 // the same with two stages ahead (75 KB), where the grid leaves a CU one
-// workgroup: nothing else then covers a stage's round trip (W4A16, cold, T =
-// 140 on 3328 x 7424 25.3 -> 23.0 us, 187 on 1920 x 11008 27.2 -> 23.4)
+// workgroup: nothing else then covers a stage's round trip (W4A16, three
+// operand sets in turn, T = 140 on 3328 x 7424 25.3 -> 23.0 us, 187 on 1920 x 11008
+// 27.2 -> 23.4)
 using CfgC64S3 = Cfg<4, 1, 1, 2, 3>;
 // 128 x 32, three stages ahead (70 KB LDS: two workgroups per CU): few X rows
 // or few tiles, where a workgroup's chain of stages is the time
@@ -175,7 +176,7 @@ clove_status_t launch_stream(const Args& a, hipStream_t stream) {
 }
 
 // K slices: 4 or 8 waves of at most 11 groups.  Short slices: a wave's chain
-// of groups is most of a small product's time (cold, us per call, against the
+// of groups is most of a small product's time (us per call, against the
 // fewest waves that hold K: W4A16 T = 13 on 8128 x 1280 6.9 -> 5.2, INT4 N =
 // 12 on 10496 x 1152 7.5 -> 5.8, N = 19 on 1984 x 1920 7.2 -> 5.4, N = 9 on
 // 3840 x 5760 9.0 -> 7.6; three operand sets).  For 17..32 groups INT4 takes 8
@@ -235,8 +236,8 @@ clove_status_t run_stream(const Args& a, int cus, hipStream_t stream) {
 // Every workgroup of the streaming kernel reads all of X (C rows x K fp16),
 // so its cost grows with C x K per CU, while the split-K MFMA kernel reads
 // each X tile once per 128 weight rows and is flat in C.  Measured (W4A16, 90
-// shapes, T = 2..32, O 1024..11008, K 1024..11008; cold, us per call, stream
-// against 128 x 32 tiles): up to 16 rows the stream is ahead below ~200 KB of
+// shapes, T = 2..32, O 1024..11008, K 1024..11008; us per call, three operand sets
+// in turn, which the Infinity Cache holds, stream against 128 x 32 tiles): up to 16 rows the stream is ahead below ~200 KB of
 // X per CU, counting one copy per round of workgroups on a CU (T = 13 on 2048
 // x 7424, 188 KB, 10.5 against 11.1; 2176 x 8704, 221 KB, 13.6 against 11.9);
 // with two X fragments below ~128 KB and in one round (T = 24 on 2944 x 1664
@@ -253,8 +254,8 @@ bool stream_ahead(const Args& a, int cus) {
 }  // namespace
 
 bool try_i4w_w4a16(const W4A16Args& w, int cus, hipStream_t stream, clove_status_t* status) {
-    // three or four tokens: the streaming kernel rather than the GEMV (cold,
-    // T = 4: 4096x11008 12.1 against 22.0 us, 2176x2176 4.3 against 6.7, 1024 x
+    // three or four tokens: the streaming kernel rather than the GEMV (three operand
+    // sets in turn, T = 4: 4096x11008 12.1 against 22.0 us, 2176x2176 4.3 against 6.7, 1024 x
     // 1664 3.7 against 4.0; at T = 2 neither is ahead throughout)
     if (w.T <= 2 || w.K <= 0 || w.K % 128 != 0 || !aligned16(w.X) || !aligned16(w.W)) return false;
     if (!fits31((int64_t)w.T * w.K * 2) || !fits31((int64_t)w.O * (w.K / 2))) return false;

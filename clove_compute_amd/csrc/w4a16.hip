@@ -561,8 +561,8 @@ clove_status_t launch_w4a16_swiglu(const W4A16Args& a, hipStream_t stream) {
     const int nch = cdiv(a.K, 32);
     const int tv = a.T <= 1 ? 1 : (a.T <= 2 ? 2 : 4);
     clove_status_t st2;
-    // three or four tokens on larger weights: the MFMA kernel (cold, us per
-    // call, GEMV against MFMA: 2 x 6784 x 1152 T = 3 10.5 -> 7.6, 2 x 10880 x
+    // three or four tokens on larger weights: the MFMA kernel (us per call,
+    // three operand sets in turn, GEMV against MFMA: 2 x 6784 x 1152 T = 3 10.5 -> 7.6, 2 x 10880 x
     // 2560 T = 3 23.4 -> 14.0, 2 x 6528 x 2560 T = 4 16.3 -> 11.1; 2 x 2944 x
     // 1536, 8.6 Mi weights, stays: 6.2 against 7.9)
     if (a.T >= 3 && a.T <= 4 && (int64_t)2 * a.O * a.K >= ((int64_t)12 << 20) &&
