@@ -73,6 +73,7 @@
 
 #include "common.hpp"
 #include "f16_dma_gemm.hpp"
+#include "skinny_plan.hpp"
 
 namespace clove {
 namespace sk {
@@ -100,50 +101,6 @@ struct Args {
     float* part;
     unsigned* counters;
 };
-
-// KW > 1: KW waves share each wave tile and take disjoint slices of every K
-// tile's four k-steps, summed through LDS after the K loop (slice order, so
-// deterministic): KW times the workgroups of the same wave tiles for small
-// products (split K only with KW = 2)
-template <bool I8_, int BM_, int BN_, int WM_, int WN_, int S_, int NB_ = 1, int KW_ = 1>
-struct Cfg {
-    static constexpr bool I8 = I8_;
-    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, S = S_, NB = NB_, KW = KW_;
-    static constexpr int ES = I8 ? 1 : 2;  // bytes per element
-    static constexpr int NW = WM * WN * KW, NT = 64 * NW;
-    static constexpr int NKS = 4 / KW;     // k-steps per K tile per wave
-    static constexpr int BK = 128 / ES;    // K per stage: 128 bytes of every A row
-    static constexpr int BNB = BN * ES;    // bytes of one B k-row in the tile
-    static constexpr int FM = BM / (32 * WM), FN = BN / (32 * WN);
-    static constexpr int A_BYTES = BM * 128, B_BYTES = BK * BNB;
-    static constexpr int SB = A_BYTES + NB * B_BYTES;
-    static constexpr int DA = A_BYTES / 1024 / NW, DB = B_BYTES / 1024 / NW;  // DB per B operand
-    static constexpr int D = DA + NB * DB;  // DMA instructions per thread per stage
-    static_assert(NW == 4, "four waves");
-    static_assert(NB == 1 || (NB == 2 && !I8), "two B operands: FP16 only");
-    static_assert(FM >= 1 && FN >= 1 && BM == 32 * FM * WM && BN == 32 * FN * WN, "wave tiles");
-    static_assert(BNB == 64 || BNB == 128 || BNB == 256 || BNB == 512, "B row bytes");
-    static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0, "DMA split");
-    static_assert(S >= 2 && S <= 9 && (S - 2) * D <= 63, "stages");
-    static_assert(KW == 1 || ((KW == 2 || KW == 4) && !I8), "k slices");
-    // the k-slice sums: every wave's NB FN FM 32x32 blocks, 4 KB each
-    static constexpr int RED = KW > 1 ? NW * NB * FN * FM * 4096 : 0;
-    static constexpr int LDS = S * SB + RED;
-    static_assert(LDS <= 160 * 1024, "LDS");
-    // UA: K tiles held in registers (16 D bytes per thread each), two LDS stages
-    static constexpr int P = D <= 2 ? 6 : D <= 5 ? 4 : D <= 6 ? 3 : 2;
-    static constexpr int LDS_UA = 2 * SB + RED;
-};
-
-// chunk swizzle of B k-row r (see the header comment): the rows one
-// transposing read touches (4 rows x 2 chunks for fp16, 8 rows x 1 chunk for
-// int8) land in 8 different bank groups
-// (rows of 128 or 256 bytes start on bank 0, rows of 64 bytes alternate halves)
-template <int BNB, bool I8>
-__device__ __forceinline__ int swz_b(int r) {
-    if constexpr (BNB >= 128) return I8 ? (r & 7) : 2 * (r & 3);
-    else return I8 ? ((r >> 1) & 3) : 2 * ((r >> 1) & 1);
-}
 
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 typedef int i32x2v __attribute__((vector_size(8)));
@@ -433,19 +390,11 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
         const unsigned a_end = (unsigned)M * K * ES, b_end = (unsigned)K * N * ES;  // bytes of A, of B
         unsigned ua[CF::DA], ub[CF::DB];  // this lane's chunks of K tile 0
 #pragma unroll
-        for (int i = 0; i < CF::DA; ++i) {
-            const int row = m0 + 8 * (wave * CF::DA + i) + (lane >> 3);
-            ua[i] = (unsigned)(row < M ? row : 0) * K * ES + 16 * ((lane & 7) ^ (lane >> 3));
-        }
+        for (int i = 0; i < CF::DA; ++i) ua[i] = ua_chunk_a<CF>(m0, wave * CF::DA + i, lane, M, K);
 #pragma unroll
-        for (int i = 0; i < CF::DB; ++i) {
-            const int row = RPI * (wave * CF::DB + i) + lane / CPR;
-            const int nb = n0 * ES + 16 * ((lane % CPR) ^ swz_b<BNB, I8>(row));
-            ub[i] = (unsigned)row * N * ES + (nb < N * ES ? nb : 0);
-        }
+        for (int i = 0; i < CF::DB; ++i) ub[i] = ua_chunk_b<CF>(n0, wave * CF::DB + i, lane, N);
         u32x4 rg[P][D];
-        // a K tile that is not the operands' last: every chunk lies inside (a B
-        // chunk that passes its row's end reads into the next row)
+        // a K tile whose every chunk lies inside (ua_whole_tiles)
         auto load_fast = [&](u32x4 (&r)[D], int t) {
             const int k0 = kbeg + t * BK;
             const unsigned char* at = Ab + (int64_t)k0 * ES;
@@ -459,13 +408,12 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
             const int k0 = kbeg + t * BK;
 #pragma unroll
             for (int i = 0; i < CF::DA; ++i) {
-                const unsigned off = ua[i] + (unsigned)k0 * ES, at = min(off, a_end - 16);
-                r[i] = keep_bytes(shift_bytes(load_any16(Ab + at), off - at),
-                                  (K - k0) * ES - 16 * ((lane & 7) ^ (lane >> 3)));
+                const unsigned off = ua[i] + (unsigned)k0 * ES, at = ua_inside(off, a_end);
+                r[i] = keep_bytes(shift_bytes(load_any16(Ab + at), off - at), ua_keep_a<CF>(k0, lane, K));
             }
 #pragma unroll
             for (int i = 0; i < CF::DB; ++i) {
-                const unsigned off = ub[i] + (unsigned)k0 * N * ES, at = min(off, b_end - 16);
+                const unsigned off = ub[i] + (unsigned)k0 * N * ES, at = ua_inside(off, b_end);
                 r[CF::DA + i] = shift_bytes(load_any16(Bb + at), off - at);  // (zero from the end on)
             }
         };
@@ -482,13 +430,13 @@ __global__ void __launch_bounds__(CF::NT) skinny_gemm(Args p) {
         // barrier t + 1, and every wave reached that one with its reads of tile t
         // complete.  The steady loop's loads are unconditional, so that the wait
         // before a tile's LDS writes leaves the P - 1 later tiles in flight.
-        const int whole = kbeg + nkt * BK < K ? nkt : nkt - 1;  // K tiles for load_fast
+        const int whole = ua_whole_tiles<CF>(kbeg, nkt, K);
 #pragma unroll
         for (int u = 0; u < P; ++u)
             if (u < nkt) load_careful(rg[u], u);
         int t = 0;
 #pragma unroll 1
-        for (; t + 2 * P <= whole; t += P) {
+        for (; ua_steady<CF>(t, whole); t += P) {
 #pragma unroll
             for (int u = 0; u < P; ++u) {
                 put(rg[u], t + u);
